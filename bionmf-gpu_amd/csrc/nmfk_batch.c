@@ -23,10 +23,11 @@
 #include <string.h>
 
 /* Partial tables per half and body class: VALU half-steps without and with lane groups
- * (a factor with few rows), matrix-core half-steps of kt 16 and of kt 32 in 1 x 4 waves, and
- * the same in 2 x 2 waves (a lone job's plan over a short contraction range), each launched
- * on its own so that it runs at its own occupancy.  Empty classes launch nothing. */
-#define NCLS 6
+ * (a factor with few rows), matrix-core half-steps of kt 16 and of kt 32 in 1 x 4 waves, the
+ * same in 2 x 2 waves (a lone job's plan over a short contraction range), and these four on
+ * split products, each launched on its own so that it runs at its own occupancy.  Empty
+ * classes launch nothing. */
+#define NCLS 10
 enum { TAB_PART_H0, TAB_PART_W0 = TAB_PART_H0 + NCLS, TAB_FIN_H = TAB_PART_W0 + NCLS, TAB_FIN_W, TAB_TEST, NTAB };
 
 static int half_cls(const nmfk_job *j, int half)
@@ -34,7 +35,7 @@ static int half_cls(const nmfk_job *j, int half)
 	const nmfk_hplan *p = half ? &j->planW : &j->planH;
 	if (j->kt <= 8)
 		return p->lb > 1 ? 1 : 0;
-	return (j->kt == 16 ? 2 : 3) + (p->ap == 2 ? 2 : 0);
+	return (j->kt == 16 ? 2 : 3) + (p->ap == 2 ? 2 : 0) + (j->split ? 4 : 0);
 }
 
 struct nmfk_batch {
@@ -194,6 +195,7 @@ static void fill_desc(nmfk_bjob *d, const nmfk_job *j)
 	d->ncolW = j->ncolW, d->ncolH = j->ncolH;
 	d->planH = j->planH, d->planW = j->planW;
 	d->live = 1;
+	d->split = (uint32_t)j->split;
 }
 
 int nmfk_batch_add(nmfk_batch *b, nmfk_job *j, const nmfk_options *opt)
@@ -224,7 +226,7 @@ int nmfk_batch_add(nmfk_batch *b, nmfk_job *j, const nmfk_options *opt)
 		return -1;
 	int e = nmfk_launch_state_reset(j->st, opt->stop_threshold, opt->nIters / b->T, j->last, j->m, b->stream);
 	if (!e)
-		e = nmfk_launch_colsum_parts(j->W, j->n, j->kt, j->colW, b->stream);
+		e = nmfk_launch_colsum_parts(j->W, j->n, j->kt, j->split, j->colW, b->stream);
 	if (e) {
 		hipck(e, "nmfk_batch_add");
 		return -1;
@@ -638,7 +640,7 @@ int nmfk_batch_autotune(nmfk_batch *b, uint32_t iters, nmfk_batch_tuning *best_o
 			e2 = hipMemcpyAsync(j->H, save + o, 4 * (size_t)j->m * j->kt, hipMemcpyDeviceToDevice, b->stream);
 		o += (size_t)j->m * j->kt;
 		if (!e2)
-			e2 = nmfk_launch_colsum_parts(j->W, j->n, j->kt, j->colW, b->stream);
+			e2 = nmfk_launch_colsum_parts(j->W, j->n, j->kt, j->split, j->colW, b->stream);
 		if (!e && e2)
 			e = e2;
 	}

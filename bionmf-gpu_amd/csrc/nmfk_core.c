@@ -328,6 +328,14 @@ nmfk_job *nmfk_job_create_shared(nmfk_job *src, uint32_t k)
 	return job_create(src->n, src->m, k, src, NULL, NULL);
 }
 
+/* Jobs planned on their own (no workgroup target) may run on split products; a job replanned
+ * to a target, as the sweep and the serving loop do, keeps the FP32 instructions. */
+static void set_split(nmfk_job *j, uint32_t target_wgs)
+{
+	j->split = target_wgs == 0 && j->planH.path == NMFK_PATH_MFMA32 && j->planW.path == NMFK_PATH_MFMA32 &&
+		   nmfk_split_rule(j->n, j->m, j->kt, j->k);
+}
+
 static nmfk_job *job_create(uint32_t n, uint32_t m, uint32_t k, nmfk_job *src, nmfk_arena *arena,
 			    hipStream_t stream)
 {
@@ -352,6 +360,7 @@ static nmfk_job *job_create(uint32_t n, uint32_t m, uint32_t k, nmfk_job *src, n
 	j->ldv = L.ldv, j->ldvt = L.ldvt;
 	j->planH = L.planH, j->planW = L.planW;
 	j->part_cap = L.n_part;
+	set_split(j, 0);
 	j->ncolW = (n + NMFK_FIN_ROWS - 1) / NMFK_FIN_ROWS;
 	j->ncolH = (m + NMFK_FIN_ROWS - 1) / NMFK_FIN_ROWS;
 	j->ndot = nmfk_dot_kl_blocks(n, m);
@@ -468,6 +477,7 @@ int nmfk_job_set_kernel_path(nmfk_job *j, int path)
 	}
 	j->planH = h;
 	j->planW = w;
+	set_split(j, 0);
 	if (j->chunk_exec) {
 		hipGraphExecDestroy(j->chunk_exec);
 		j->chunk_exec = NULL;
@@ -490,6 +500,7 @@ int nmfk_job_replan(nmfk_job *j, uint32_t target_wgs)
 	}
 	j->planH = h;
 	j->planW = w;
+	set_split(j, target_wgs);
 	if (j->chunk_exec) {
 		hipGraphExecDestroy(j->chunk_exec);
 		j->chunk_exec = NULL;
@@ -726,6 +737,9 @@ int nmfk_job_get_H(nmfk_job *j, float *H, size_t ldh)
 
 static int partial_H(nmfk_job *j, const nmfk_state *st)
 {
+	if (j->split)
+		return nmfk_launch_partial_split(j->V, j->ldv, j->H, j->W, j->m, j->n, j->kt, &j->planH, j->part,
+						 j->colW, j->ncolW, j->denW, st, j->stream);
 	if (j->planH.path == NMFK_PATH_MFMA_BF16)
 		return nmfk_launch_partial_bf16(j->V, j->ldv, j->H, j->Wb, j->m, j->n, j->kt, &j->planH, j->part,
 						j->colW, j->ncolW, j->denW, st, j->stream);
@@ -735,6 +749,9 @@ static int partial_H(nmfk_job *j, const nmfk_state *st)
 
 static int partial_W(nmfk_job *j, const nmfk_state *st)
 {
+	if (j->split)
+		return nmfk_launch_partial_split(j->Vt, j->ldvt, j->W, j->H, j->n, j->m, j->kt, &j->planW, j->part,
+						 j->colH, j->ncolH, j->denH, st, j->stream);
 	if (j->planW.path == NMFK_PATH_MFMA_BF16)
 		return nmfk_launch_partial_bf16(j->Vt, j->ldvt, j->W, j->Hb, j->n, j->m, j->kt,
 						&j->planW, j->part, j->colH, j->ncolH, j->denH, st, j->stream);
@@ -746,24 +763,34 @@ static int partial_W(nmfk_job *j, const nmfk_state *st)
  * finish kernel applies the update to H and leaves colsum(H) partials for the W half (and
  * the BF16 copy of H when the W half runs in BF16).  On the BF16 path W is read from its
  * BF16 copy, which the W half's finish (or nmfk_job_shadow_for_H) keeps current. */
+static int finish_H(nmfk_job *j, const nmfk_state *st)
+{
+	if (j->split)
+		return nmfk_launch_finish_split(j->part, j->planH.S, j->H, j->m, j->k, j->kt, j->denW, j->colH, 0, st,
+						j->stream);
+	return nmfk_launch_finish_shadow(j->part, j->planH.S, j->H, j->m, j->k, j->kt, j->denW, j->colH, 0, st,
+					 j->planW.path == NMFK_PATH_MFMA_BF16 ? j->Hb : NULL, j->stream);
+}
+
+static int finish_W(nmfk_job *j, const nmfk_state *st, int clamp)
+{
+	if (j->split)
+		return nmfk_launch_finish_split(j->part, j->planW.S, j->W, j->n, j->k, j->kt, j->denH, j->colW, clamp, st,
+						j->stream);
+	return nmfk_launch_finish_shadow(j->part, j->planW.S, j->W, j->n, j->k, j->kt, j->denH, j->colW, clamp, st,
+					 j->planH.path == NMFK_PATH_MFMA_BF16 ? j->Wb : NULL, j->stream);
+}
+
 int nmfk_enqueue_half_H(nmfk_job *j, const nmfk_state *st)
 {
-	int e = partial_H(j, st);
-	const int sh = j->planW.path == NMFK_PATH_MFMA_BF16;
-	if (!e)
-		e = nmfk_launch_finish_shadow(j->part, j->planH.S, j->H, j->m, j->k, j->kt, j->denW, j->colH, 0, st,
-					      sh ? j->Hb : NULL, j->stream);
-	return e;
+	const int e = partial_H(j, st);
+	return e ? e : finish_H(j, st);
 }
 
 int nmfk_enqueue_half_W(nmfk_job *j, const nmfk_state *st, int clamp)
 {
-	int e = partial_W(j, st);
-	const int sh = j->planH.path == NMFK_PATH_MFMA_BF16;
-	if (!e)
-		e = nmfk_launch_finish_shadow(j->part, j->planW.S, j->W, j->n, j->k, j->kt, j->denH, j->colW, clamp, st,
-					      sh ? j->Wb : NULL, j->stream);
-	return e;
+	const int e = partial_W(j, st);
+	return e ? e : finish_W(j, st, clamp);
 }
 
 int nmfk_job_shadow_for_H(nmfk_job *j)
@@ -785,7 +812,7 @@ int nmfk_job_update_H(nmfk_job *j)
 {
 	if (j->streamed)
 		return nmfk_stream_update_H(j);
-	int e = nmfk_launch_colsum_parts(j->W, j->n, j->kt, j->colW, j->stream);
+	int e = nmfk_launch_colsum_parts(j->W, j->n, j->kt, j->split, j->colW, j->stream);
 	if (!e)
 		e = nmfk_job_shadow_for_H(j);
 	if (!e)
@@ -800,7 +827,7 @@ int nmfk_job_update_W(nmfk_job *j)
 		return nmfk_stream_update_W(j);
 	if (nmfk_job_refresh_Vt(j))
 		return NMFK_EHIP;
-	int e = nmfk_launch_colsum_parts(j->H, j->m, j->kt, j->colH, j->stream);
+	int e = nmfk_launch_colsum_parts(j->H, j->m, j->kt, j->split, j->colH, j->stream);
 	if (!e)
 		e = nmfk_job_shadow_for_W(j);
 	if (!e)
@@ -905,7 +932,7 @@ int nmfk_job_run(nmfk_job *j, const nmfk_options *opt, nmfk_result *res)
 			e = one_pass(j, 0, 0, j->st);
 	} else {
 		if (!e)
-			e = nmfk_launch_colsum_parts(j->W, j->n, j->kt, j->colW, j->stream);
+			e = nmfk_launch_colsum_parts(j->W, j->n, j->kt, j->split, j->colW, j->stream);
 		if (!e)
 			e = nmfk_job_shadow_for_H(j);
 	}
@@ -1049,15 +1076,13 @@ static int time_loop(nmfk_job *j, uint32_t iters, int kind, double *ms)
 			e = partial_H(j, NULL);
 			break;
 		case 2:
-			e = nmfk_launch_finish(j->part, j->planH.S, j->H, j->m, j->k, j->kt, j->denW, j->colH, 0,
-					       NULL, j->stream);
+			e = finish_H(j, NULL);
 			break;
 		case 3:
 			e = partial_W(j, NULL);
 			break;
 		case 4:
-			e = nmfk_launch_finish(j->part, j->planW.S, j->W, j->n, j->k, j->kt, j->denH, j->colW, 0,
-					       NULL, j->stream);
+			e = finish_W(j, NULL, 0);
 			break;
 		}
 	}
@@ -1181,7 +1206,7 @@ int nmfk_job_time_iterations(nmfk_job *j, uint32_t iters, nmfk_timing *t)
 {
 	if (needs_device_V(j, "nmfk_job_time_iterations"))
 		return NMFK_EINVAL;
-	int e = nmfk_launch_colsum_parts(j->W, j->n, j->kt, j->colW, j->stream);
+	int e = nmfk_launch_colsum_parts(j->W, j->n, j->kt, j->split, j->colW, j->stream);
 	if (!e)
 		e = nmfk_job_shadow_for_H(j);
 	if (!e)

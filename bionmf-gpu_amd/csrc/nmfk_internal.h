@@ -42,6 +42,7 @@ struct nmfk_job {
 	nmfk_state *st;                /* device stop-rule state */
 	nmfk_state *h_st;              /* pinned, 2 slots */
 	nmfk_hplan planH, planW;
+	int split;                     /* FP32 matrix-core half-steps run on split products (nmfk_split_rule) */
 	hipStream_t stream;
 	hipEvent_t ev[2];
 	hipGraphExec_t chunk_exec;

@@ -93,6 +93,14 @@ int nmfk_launch_partial(const float *U, size_t ldu, const float *A, const float 
 			float *part, const float *colB, uint32_t ncolB, float *den,
 			const nmfk_state *st, hipStream_t stream);
 
+/* The same sums from products of three-part BF16 operands (FP32 accuracy; kt 16, 32, 64 on
+ * plan path NMFK_PATH_MFMA32; sums every column of kt). */
+int nmfk_launch_partial_split(const float *U, size_t ldu, const float *A, const float *B, uint32_t p, uint32_t q,
+			      uint32_t kt, const nmfk_hplan *pl, float *part, const float *colB, uint32_t ncolB,
+			      float *den, const nmfk_state *st, hipStream_t stream);
+/* Whether a resident FP32 matrix-core job planned on its own runs on split products. */
+int nmfk_split_rule(uint32_t n, uint32_t m, uint32_t kt, uint32_t k);
+
 /*
  * Half-step, second kernel:
  *   A[a][c] = (A[a][c] * sum_s part[s][a][c]) / den[c]     for c < k
@@ -115,7 +123,10 @@ int nmfk_launch_finish(const float *part, uint32_t S, float *A, uint32_t p, uint
 		       const float *den, float *colA, int clamp, const nmfk_state *st,
 		       hipStream_t stream);
 
-/* The same, also writing the BF16 copy of the new A: Ab (p x kt, row-major); kt % 32 == 0
+/* The same for a job on split products: sums as trees instead of in ascending order. */
+int nmfk_launch_finish_split(const float *part, uint32_t S, float *A, uint32_t p, uint32_t k, uint32_t kt,
+			     const float *den, float *colA, int clamp, const nmfk_state *st, hipStream_t stream);
+/* The finish in ascending order, also writing the BF16 copy of the new A: Ab (p x kt, row-major); kt % 32 == 0
  * when Ab is given. */
 int nmfk_launch_finish_shadow(const float *part, uint32_t S, float *A, uint32_t p, uint32_t k, uint32_t kt,
 			      const float *den, float *colA, int clamp, const nmfk_state *st, uint16_t *Ab,
@@ -128,8 +139,9 @@ int nmfk_launch_partial_bf16(const float *U, size_t ldu, const float *A, const u
 			     uint32_t kt, const nmfk_hplan *pl, float *part, const float *colB, uint32_t ncolB,
 			     float *den, const nmfk_state *st, hipStream_t stream);
 
-/* colA[blk][c] = sum of A[a][c] over the rows of block blk (same order as k_finish). */
-int nmfk_launch_colsum_parts(const float *A, uint32_t p, uint32_t kt, float *colA, hipStream_t stream);
+/* colA[blk][c] = sum of A[a][c] over the rows of block blk (same order as the finish of a job
+ * with or without split products). */
+int nmfk_launch_colsum_parts(const float *A, uint32_t p, uint32_t kt, int split, float *colA, hipStream_t stream);
 
 /* den[c] = sum_g parts[g][c] in the fixed order the partial kernel uses. */
 int nmfk_launch_den(const float *parts, uint32_t nparts, uint32_t kt, float *den, hipStream_t stream);
@@ -165,7 +177,7 @@ typedef struct nmfk_bjob {
 	uint32_t ncolW, ncolH;
 	nmfk_hplan planH, planW;
 	uint32_t live;        /* 0: empty slot, every tile of it returns without reading the job */
-	uint32_t pad_;
+	uint32_t split;       /* the job runs on split products (its finishes add as trees) */
 } nmfk_bjob;
 
 typedef struct nmfk_tile {
@@ -178,7 +190,8 @@ typedef struct nmfk_tile {
 /* half: 0 = H half (U = V, A = H, B = W), 1 = W half (U = Vt, A = W, B = H).  cls: the body
  * class of every tile's half-step: 0 = vector ALUs (kt 4/8) without lane groups, 1 = vector
  * ALUs with lane groups (plan lb > 1), 2 and 3 = matrix cores at kt 16 and 32 in 1 x 4 waves,
- * 4 and 5 = the same in 2 x 2 waves (plan ap 2); tiles of other classes are skipped. */
+ * 4 and 5 = the same in 2 x 2 waves (plan ap 2), 6-9 = classes 2-5 on split products; tiles of
+ * other classes are skipped. */
 int nmfk_launch_batch_partial(const nmfk_bjob *jobs, const nmfk_tile *tiles, uint32_t ntiles, int half,
 			      int cls, uint32_t grid, hipStream_t stream);
 int nmfk_launch_batch_finish(const nmfk_bjob *jobs, const nmfk_tile *tiles, uint32_t ntiles, int half,

@@ -113,9 +113,21 @@ __device__ __forceinline__ double wave_sum_d(double v)
 // Workgroup size of every half-step kernel (single-job and batched launches alike).
 #define NMFK_WG 256
 
+// Eight values as a tree: 3 roundings deep instead of 8.  The sums over splits, rows and
+// column-sum partials of a job on split products are formed this way, which takes their
+// rounding errors well below those of the products (H half at 20000 x 1000, k = 16: 1.5e-7 rms
+// from 64 bits in order, 0.5e-7 without these errors).  Every other job keeps its ascending
+// order, and with it its bits.
+__device__ __forceinline__ float pair8(const float (&v)[8])
+{
+	return ((v[0] + v[1]) + (v[2] + v[3])) + ((v[4] + v[5]) + (v[6] + v[7]));
+}
+
 // den[c] = sum_g parts[g][c]: four interleaved running sums per column, added in a fixed
 // order at the end.  s4 is 4*KT floats of LDS; needs 4*KT <= NMFK_WG threads.
-template <int KT>
+// PAIR: 8 loaded values are added as a tree before they join the running sum (jobs on split
+// products; see pair8).
+template <int KT, bool PAIR = false>
 __device__ __forceinline__ void den_reduce(const float *__restrict__ parts, int nparts, float *__restrict__ den,
 					   float *__restrict__ s4)
 {
@@ -131,9 +143,13 @@ __device__ __forceinline__ void den_reduce(const float *__restrict__ parts, int 
 #pragma unroll
 			for (int u = 0; u < 8; u++)
 				v[u] = parts[(size_t)(g + 4 * u) * KT + c];
+			if constexpr (PAIR) {
+				s += pair8(v);
+			} else {
 #pragma unroll
-			for (int u = 0; u < 8; u++)
-				s += v[u];
+				for (int u = 0; u < 8; u++)
+					s += v[u];
+			}
 		}
 		for (; g < nparts; g += 4)
 			s += parts[(size_t)g * KT + c];
@@ -141,7 +157,8 @@ __device__ __forceinline__ void den_reduce(const float *__restrict__ parts, int 
 	}
 	__syncthreads();
 	if (t < KT)
-		den[t] = ((s4[4 * t] + s4[4 * t + 1]) + s4[4 * t + 2]) + s4[4 * t + 3];
+		den[t] = PAIR ? (s4[4 * t] + s4[4 * t + 1]) + (s4[4 * t + 2] + s4[4 * t + 3])
+			      : ((s4[4 * t] + s4[4 * t + 1]) + s4[4 * t + 2]) + s4[4 * t + 3];
 }
 
 // One finish block = NMFK_FIN_ROWS (64) rows of A with 4 threads per row, each thread
@@ -158,8 +175,9 @@ __host__ __device__ constexpr int fin_q(int kt)
 }
 static_assert(NMFK_FIN_ROWS * 4 == NMFK_WG, "finish block shape");
 
-// tile: NMFK_FIN_ROWS x (KT + 1) floats of LDS.
-template <int KT>
+// tile: NMFK_FIN_ROWS x (KT + 1) floats of LDS.  PAIR: NMFK_WG / KT groups of threads add
+// consecutive rows each, then one thread per column adds the groups.
+template <int KT, bool PAIR = false>
 __device__ __forceinline__ void block_colsum_store(const float (&x)[fin_q(KT)], float *__restrict__ out,
 						   float *__restrict__ tile)
 {
@@ -169,6 +187,25 @@ __device__ __forceinline__ void block_colsum_store(const float (&x)[fin_q(KT)], 
 	for (int i = 0; i < Q; i++)
 		tile[row * (KT + 1) + q * Q + i] = x[i];
 	__syncthreads();
+	if constexpr (PAIR) {
+		constexpr int G = NMFK_WG / KT, RG = NMFK_FIN_ROWS / G;
+		const int c = threadIdx.x % KT, gr = threadIdx.x / KT;
+		float s = 0.0f;
+#pragma unroll
+		for (int r = 0; r < RG; r++)
+			s += tile[(gr * RG + r) * (KT + 1) + c];
+		__syncthreads();
+		tile[gr * (KT + 1) + c] = s;
+		__syncthreads();
+		if (threadIdx.x < KT) {
+			float z[4] = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+			for (int i = 0; i < G; i++)
+				z[i % 4] += tile[i * (KT + 1) + threadIdx.x];
+			out[threadIdx.x] = (z[0] + z[1]) + (z[2] + z[3]);
+		}
+		return;
+	}
 	if (threadIdx.x < KT) {
 		float s = 0.0f;
 		for (int r = 0; r < NMFK_FIN_ROWS; r++)
@@ -472,6 +509,55 @@ __device__ __forceinline__ float4 loadq(const float *p)
 		return make_float4(v.x, v.y, 0.f, 0.f);
 	} else
 		return make_float4(p[0], 0.f, 0.f, 0.f);
+}
+
+// Sums of a wave's 64 rows a (acc[t][h][r] = partial for a = a0 + 4*(4g + r) + t, c = 16h + j):
+// the NB wave groups' are added through LDS in a fixed order and written to split by of part.
+template <int KT, int NA, int NB>
+__device__ __forceinline__ void mfma_store(floatx4 (&acc)[4][KT / 16], const half_args &ha, int by, int a0, bool idle,
+					   float *__restrict__ smem)
+{
+	constexpr int H = KT / 16;
+	const int lane = threadIdx.x & 63, j = lane & 15, g = lane >> 4;
+	const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+	const int wa = wave % NA, wb = wave / NA, p = ha.p;
+	if constexpr (NB > 1) {
+		float (*red)[NA][4][H][4][64] = reinterpret_cast<float (*)[NA][4][H][4][64]>(smem);
+		if (wb > 0) {
+#pragma unroll
+			for (int t = 0; t < 4; t++)
+#pragma unroll
+				for (int h = 0; h < H; h++)
+#pragma unroll
+					for (int r = 0; r < 4; r++)
+						red[wb - 1][wa][t][h][r][lane] = acc[t][h][r];
+		}
+		__syncthreads();
+		if (wb > 0 || idle)
+			return;
+#pragma unroll
+		for (int w = 0; w < NB - 1; w++)
+#pragma unroll
+			for (int t = 0; t < 4; t++)
+#pragma unroll
+				for (int h = 0; h < H; h++)
+#pragma unroll
+					for (int r = 0; r < 4; r++)
+						acc[t][h][r] += red[w][wa][t][h][r][lane];
+	}
+	if (idle)
+		return;
+	float *dst = ha.part + (size_t)by * p * KT;
+#pragma unroll
+	for (int t = 0; t < 4; t++)
+#pragma unroll
+		for (int r = 0; r < 4; r++) {
+			const int a = a0 + 4 * (4 * g + r) + t;
+			if (a < p)
+#pragma unroll
+				for (int h = 0; h < H; h++)
+					dst[(size_t)a * KT + 16 * h + j] = acc[t][h][r];
+		}
 }
 
 // Workgroup = NA x NB waves: NA waves side by side in a (lockstep over the same rows of U),
@@ -782,44 +868,7 @@ __device__ __forceinline__ void partial_mfma_body(int bx, int by, const half_arg
 		}
 		return;
 	}
-	// acc[t][h][r] = partial for a = a0 + 4*(4g + r) + t, c = 16h + j.
-	if constexpr (NB > 1) {
-		float (*red)[NA][4][H][4][64] = reinterpret_cast<float (*)[NA][4][H][4][64]>(smem);
-		if (wb > 0) {
-#pragma unroll
-			for (int t = 0; t < 4; t++)
-#pragma unroll
-				for (int h = 0; h < H; h++)
-#pragma unroll
-					for (int r = 0; r < 4; r++)
-						red[wb - 1][wa][t][h][r][lane] = acc[t][h][r];
-		}
-		__syncthreads();
-		if (wb > 0 || idle)
-			return;
-#pragma unroll
-		for (int w = 0; w < NB - 1; w++)
-#pragma unroll
-			for (int t = 0; t < 4; t++)
-#pragma unroll
-				for (int h = 0; h < H; h++)
-#pragma unroll
-					for (int r = 0; r < 4; r++)
-						acc[t][h][r] += red[w][wa][t][h][r][lane];
-	}
-	if (idle)
-		return;
-	float *dst = ha.part + (size_t)by * p * KT;
-#pragma unroll
-	for (int t = 0; t < 4; t++)
-#pragma unroll
-		for (int r = 0; r < 4; r++) {
-			const int a = a0 + 4 * (4 * g + r) + t;
-			if (a < p)
-#pragma unroll
-				for (int h = 0; h < H; h++)
-					dst[(size_t)a * KT + 16 * h + j] = acc[t][h][r];
-		}
+	mfma_store<KT, NA, NB>(acc, ha, by, a0, idle, smem);
 }
 
 template <int KT, int NA, int NB, int KE = KT>
@@ -1067,44 +1116,9 @@ __device__ __forceinline__ void partial_bf16_body(int bx, int by, const half_arg
 		gemm2(rt);
 	}
 
-	if constexpr (NB > 1) {
+	if constexpr (NB > 1)
 		__syncthreads();   // every wave is done with its B slot, which the sums below reuse
-		float (*red)[NA][4][H][4][64] = reinterpret_cast<float (*)[NA][4][H][4][64]>(smem);
-		if (wb > 0) {
-#pragma unroll
-			for (int t = 0; t < 4; t++)
-#pragma unroll
-				for (int h = 0; h < H; h++)
-#pragma unroll
-					for (int r = 0; r < 4; r++)
-						red[wb - 1][wa][t][h][r][lane] = acc[t][h][r];
-		}
-		__syncthreads();
-		if (wb > 0 || idle)
-			return;
-#pragma unroll
-		for (int w = 0; w < NB - 1; w++)
-#pragma unroll
-			for (int t = 0; t < 4; t++)
-#pragma unroll
-				for (int h = 0; h < H; h++)
-#pragma unroll
-					for (int r = 0; r < 4; r++)
-						acc[t][h][r] += red[w][wa][t][h][r][lane];
-	}
-	if (idle)
-		return;
-	float *dst = ha.part + (size_t)by * p * KT;
-#pragma unroll
-	for (int t = 0; t < 4; t++)
-#pragma unroll
-		for (int r = 0; r < 4; r++) {
-			const int a = a0 + 4 * (4 * g + r) + t;
-			if (a < p)
-#pragma unroll
-				for (int h = 0; h < H; h++)
-					dst[(size_t)a * KT + 16 * h + j] = acc[t][h][r];
-		}
+	mfma_store<KT, NA, NB>(acc, ha, by, a0, idle, smem);
 }
 
 template <int KT, int NA, int NB>
@@ -1118,6 +1132,377 @@ __global__ __launch_bounds__(64 * NA * NB) void k_partial_bf16(half_args h, bf16
 	if (!xcd_tile(h.nab + 1, (h.nab + 1) * S, bx, by))
 		return;
 	partial_bf16_body<KT, NA, NB>(bx, by, h, b, smem);
+}
+
+// --------------------------------------------------------------------------------------
+// The half-step in FP32 accuracy on the BF16 matrix cores (KT 16, 32, 64; nmfk_split_rule says
+// which jobs).
+// Every FP32 operand is the exact sum of three BF16 numbers, x = x1 + x2 + x3: 3 x 8
+// significand bits, each part the rounding of what the parts before it leave.  A product is
+// formed from the six partial products of relative size 2^-16 and more (x1 y1, x1 y2, x2 y1,
+// x2 y2, x1 y3, x3 y1), accumulated in FP32 by v_mfma_f32_16x16x32_bf16; the three left out
+// are below 2^-24.  Sums of 32, 64 and 256 products came out 3.4e-8, 7.4e-8 and 1.9e-7 rms
+// from the 64-bit sums, against 8.8e-8, 1.2e-7 and 2.4e-7 on the FP32 instructions.  Exact for
+// operands of 7.7e-34 and more (bits below 2^-133 are lost); infinities see partial_split_body.
+//
+// What bounds the FP32 instructions is their rate: 16x16x4 takes 32 cycles, 1024 per 16-row
+// block and 64 rows a at KT 16, 2048 at KT 32, 4096 at KT 64.  The split products take 384,
+// 768 and 1536, and 120-180 vector instructions for the ratios and the splitting.  Ownership
+// of rows, blocks and wave groups is that of the body above; per 16-row block a wave
+//   stages B (fetched as FP32, one block ahead) in its own LDS slot in three parts, row-major,
+//   from where both operand layouts are read: GEMM1's as 16-byte row segments, GEMM2's with
+//   ds_read_b64_tr_b16 (4 rows of one column per lane);
+//   GEMM1  K = 32 columns of one product; at KT 16 the 32 slots hold the 16 columns of two
+//          products: [b1 b1][a2 a1], [b2 b2][a2 a1], [b3 b1][a1 a3] over lane groups 0-1, 2-3;
+//   ratio  FP32, then split: lane (g, j) holds rows 4g + r, r = 0..3;
+//   GEMM2  K = the 16 rows of two products: lane group g's 8 elements are rows 4g..4g+3 in one
+//          part, then in another: [r1 r3][b3 b1], [r2 r1][b2 b2], [r2 r1][b1 b1].
+// Measured, partials of the two halves (FP32 instructions -> split): 20000 x 1000, k = 32
+// 30.9 + 31.3 -> 23.0 + 23.2 us; 50000 x 2000, k = 64 213 + 239 -> 138 + 155; 20000 x 1000,
+// k = 16 19.0 + 18.8 -> 17.8 + 18.0; 7013 x 333, k = 24 9.0 + 8.3 -> 7.7 + 7.3.  GEMM1 of the next block issued beside GEMM2 of this one, with and without a
+// fixed interleave of matrix and vector instructions, and 3-6 blocks of U in flight were all
+// even or slower: two or three waves per SIMD overlap the two pipes as well.
+// --------------------------------------------------------------------------------------
+
+typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+typedef float floatx2 __attribute__((ext_vector_type(2)));
+typedef short shortx4 __attribute__((ext_vector_type(4)));
+
+// The three parts of x0 and x1, packed in pairs.  x - part is one v_dot2_f32_bf16 (the pair
+// times (-1, 0) or (0, -1), plus x), which is exact.  The two constants go through scalar
+// registers: as an inline constant -1.0 would mean the low half only.
+__device__ __forceinline__ void split3(float x0, float x1, bf16x2 &p1, bf16x2 &p2, bf16x2 &p3)
+{
+	uint32_t c0, c1;
+	asm("s_mov_b32 %0, 0x0000bf80" : "=s"(c0));
+	asm("s_mov_b32 %0, 0xbf800000" : "=s"(c1));
+	bf16x2 m0, m1;
+	__builtin_memcpy(&m0, &c0, 4);
+	__builtin_memcpy(&m1, &c1, 4);
+	p1 = __builtin_convertvector((floatx2{x0, x1}), bf16x2);
+	const float r0 = __builtin_amdgcn_fdot2_f32_bf16(p1, m0, x0, false);
+	const float r1 = __builtin_amdgcn_fdot2_f32_bf16(p1, m1, x1, false);
+	p2 = __builtin_convertvector((floatx2{r0, r1}), bf16x2);
+	const float q0 = __builtin_amdgcn_fdot2_f32_bf16(p2, m0, r0, false);
+	const float q1 = __builtin_amdgcn_fdot2_f32_bf16(p2, m1, r1, false);
+	p3 = __builtin_convertvector((floatx2{q0, q1}), bf16x2);
+}
+
+// Part i of four floats: p[i], i = 0..2.
+__device__ __forceinline__ void split3x4(float a, float b, float c, float d, bf16x4 (&p)[3])
+{
+	bf16x2 lo[3], hi[3];
+	split3(a, b, lo[0], lo[1], lo[2]);
+	split3(c, d, hi[0], hi[1], hi[2]);
+#pragma unroll
+	for (int i = 0; i < 3; i++)
+		p[i] = __builtin_shufflevector(lo[i], hi[i], 0, 1, 2, 3);
+}
+
+__device__ __forceinline__ bf16x8 cat8(bf16x4 lo, bf16x4 hi)
+{
+	return __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
+}
+
+// One wave's sums of a split on the FP32 instructions (16x16x4), for operands that the three
+// parts cannot hold: rows a = aj + t, 16-row blocks wb, wb + NB, ... of rows b_begin .. b_end.
+template <int KT, int NB>
+__device__ __forceinline__ void sum32(const half_args &ha, int aj, int wb, int b_begin, int b_end, floatx4 (&acc)[4][KT / 16])
+{
+	constexpr int H = KT / 16;
+	const int lane = threadIdx.x & 63, j = lane & 15, g = lane >> 4;
+	const int avail = ha.p - aj, ucol = avail > 0 ? aj : 0;
+#pragma unroll
+	for (int t = 0; t < 4; t++)
+#pragma unroll
+		for (int h = 0; h < H; h++)
+			acc[t][h] = floatx4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll 1
+	for (int bb = b_begin + 16 * wb; bb < b_end; bb += 16 * NB) {
+		floatx4 s[4];
+#pragma unroll
+		for (int t = 0; t < 4; t++)
+			s[t] = floatx4{0.f, 0.f, 0.f, 0.f};
+		const bool jok = bb + j < b_end;
+		const float *Bj = ha.B + (size_t)(jok ? bb + j : b_begin) * KT + 4 * g;
+#pragma unroll 1
+		for (int c = 0; c < KT; c += 16)
+#pragma unroll
+			for (int qq = 0; qq < 4; qq++) {
+				const float bv = jok ? Bj[c + qq] : 0.0f;
+#pragma unroll
+				for (int t = 0; t < 4; t++) {
+					const float av = t < avail ? ha.A[(size_t)(aj + t) * KT + c + 4 * g + qq] : 0.0f;
+					s[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(bv, av, s[t], 0, 0, 0);
+				}
+			}
+#pragma unroll
+		for (int r = 0; r < 4; r++) {
+			const bool rok = bb + 4 * g + r < b_end;
+			const size_t row = rok ? bb + 4 * g + r : b_begin;
+			const float4 u = *reinterpret_cast<const float4 *>(ha.U + row * ha.ldu + ucol);
+			const float uv[4] = {u.x, u.y, u.z, u.w};
+#pragma unroll
+			for (int t = 0; t < 4; t++) {
+				const float v = uv[t] * __builtin_amdgcn_rcpf(s[t][r]);
+				const float rt = rok ? v : 0.0f;
+#pragma unroll
+				for (int h = 0; h < H; h++)
+					acc[t][h] = __builtin_amdgcn_mfma_f32_16x16x4f32(rt, ha.B[row * KT + 16 * h + j], acc[t][h], 0, 0, 0);
+			}
+		}
+	}
+}
+
+// LDS of the split body: each wave's 16-row block of B in three parts (rows of KT + 8 BF16),
+// and after it the wave groups' sums.
+__host__ __device__ constexpr int smem_split(int kt, int na, int nb)
+{
+	return smem_mfma(kt, na, nb) > na * nb * 3 * 8 * (kt + 8) ? smem_mfma(kt, na, nb) : na * nb * 3 * 8 * (kt + 8);
+}
+
+template <int KT, int NA, int NB>
+__device__ __forceinline__ void partial_split_body(int bx, int by, const half_args &ha, float *__restrict__ smem)
+{
+	static_assert(KT == 16 || KT % 32 == 0, "split body: KT 16, or whole 32-column chunks");
+	constexpr int H = KT / 16;
+	constexpr int CH = KT >= 32 ? KT / 32 : 1;   // 32-column chunks of GEMM1
+	constexpr int NQ = KT >= 32 ? 3 : 2;         // GEMM1 operands of A per tile and chunk
+	const float *__restrict__ U = ha.U;
+	const size_t ldu = ha.ldu;
+	const float *__restrict__ A = ha.A;
+	const float *__restrict__ B = ha.B;
+	const int p = ha.p, q = ha.q, bchunk = ha.bchunk;
+	if (bx == ha.nab) {
+		if (by == 0)
+			den_reduce<KT, true>(ha.colB, ha.ncolB, ha.den, smem);
+		return;
+	}
+	const int lane = threadIdx.x & 63;
+	const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+	const int wa = wave % NA, wb = wave / NA;
+	const int j = lane & 15, g = lane >> 4;
+	const int a0 = (bx * NA + wa) * 64;
+	const bool idle = a0 >= p;
+	const int aj = a0 + 4 * j;
+	const int avail = p - aj;
+	const int b_begin = by * bchunk;
+	const int b_end = min(q, b_begin + bchunk);
+	const int ucol = avail > 0 ? aj : 0;
+
+	const int nfull = (b_end - b_begin) / 16;
+	const int mine = idle ? 0 : (nfull > wb ? (nfull - wb + NB - 1) / NB : 0);
+	auto blk_row = [&](int i) { return b_begin + 16 * (wb + NB * min(i, mine - 1)); };
+
+	int uoff[4];
+#pragma unroll
+	for (int r = 0; r < 4; r++)
+		uoff[r] = ((4 * g + r) * (int)ldu + ucol) * 4;
+	auto load_u = [&](int bb, float4 (&u)[4]) {
+		const __amdgpu_buffer_rsrc_t rU = make_rsrc(U + (size_t)bb * ldu, (size_t)16 * ldu * 4);
+#pragma unroll
+		for (int r = 0; r < 4; r++)
+			u[r] = bload4(rU, uoff[r], 0);
+	};
+	constexpr int DU = KT <= 32 ? 2 : 1, DB = 1;   // blocks of U and of B in flight
+	float4 ur[DU][4], br[DB][H];
+	auto fetch_b = [&](int bb, float4 (&b)[H]) {
+		const __amdgpu_buffer_rsrc_t rB = make_rsrc(B + (size_t)bb * KT, (size_t)16 * KT * 4);
+#pragma unroll
+		for (int h = 0; h < H; h++)
+			b[h] = bload4(rB, (h * 64 + lane) * 16, 0);
+	};
+	if (mine > 0) {
+#pragma unroll
+		for (int d = 0; d < DU; d++) {
+			load_u(blk_row(d), ur[d]);
+			if (d < DB)
+				fetch_b(blk_row(d), br[d]);
+		}
+	}
+
+	// GEMM1's A operands.
+	bf16x8 aq[4][CH][NQ];
+#pragma unroll
+	for (int t = 0; t < 4; t++) {
+		const bool ok = t < avail;
+		const float *Ar = A + (size_t)(ok ? aj + t : 0) * KT;
+#pragma unroll
+		for (int ch = 0; ch < CH; ch++) {
+			const float *Ac = Ar + (KT >= 32 ? 32 * ch + 8 * g : 8 * (g & 1));
+			float4 lo = *reinterpret_cast<const float4 *>(Ac);
+			float4 hi = *reinterpret_cast<const float4 *>(Ac + 4);
+			if (!ok)
+				lo = hi = make_float4(0.f, 0.f, 0.f, 0.f);
+			bf16x4 pl[3], ph[3];
+			split3x4(lo.x, lo.y, lo.z, lo.w, pl);
+			split3x4(hi.x, hi.y, hi.z, hi.w, ph);
+			const bf16x8 a1 = cat8(pl[0], ph[0]), a2 = cat8(pl[1], ph[1]), a3 = cat8(pl[2], ph[2]);
+			if constexpr (KT >= 32) {
+				aq[t][ch][0] = a1, aq[t][ch][1] = a2, aq[t][ch][2] = a3;
+			} else {
+				aq[t][ch][0] = g < 2 ? a2 : a1;
+				aq[t][ch][1] = g < 2 ? a1 : a3;
+			}
+		}
+	}
+	floatx4 acc[4][H];
+#pragma unroll
+	for (int t = 0; t < 4; t++)
+#pragma unroll
+		for (int h = 0; h < H; h++)
+			acc[t][h] = floatx4{0.f, 0.f, 0.f, 0.f};
+
+	constexpr int BS = KT + 8;
+	__bf16 *slot = reinterpret_cast<__bf16 *>(smem) + (size_t)wave * 3 * 16 * BS;
+	auto stage_b = [&](const float4 (&b)[H]) {
+#pragma unroll
+		for (int h = 0; h < H; h++) {
+			const int e = (h * 64 + lane) * 4, row = e / KT, col = e % KT;
+			bf16x4 pt[3];
+			split3x4(b[h].x, b[h].y, b[h].z, b[h].w, pt);
+#pragma unroll
+			for (int i = 0; i < 3; i++)
+				*reinterpret_cast<bf16x4 *>(slot + (i * 16 + row) * BS + col) = pt[i];
+		}
+	};
+	auto mfma = [](bf16x8 a, bf16x8 b, floatx4 c) { return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0); };
+	auto gemm1 = [&](floatx4 (&s)[4]) {
+#pragma unroll
+		for (int t = 0; t < 4; t++)
+			s[t] = floatx4{0.f, 0.f, 0.f, 0.f};
+		if constexpr (KT >= 32) {
+			constexpr int ib[6] = {2, 0, 1, 1, 0, 0}, ia[6] = {0, 2, 1, 0, 1, 0};
+#pragma unroll
+			for (int ch = 0; ch < CH; ch++) {
+				bf16x8 bq[3];
+#pragma unroll
+				for (int i = 0; i < 3; i++)
+					bq[i] = *reinterpret_cast<const bf16x8 *>(slot + (i * 16 + j) * BS + 32 * ch + 8 * g);
+#pragma unroll
+				for (int x = 0; x < 6; x++)
+#pragma unroll
+					for (int t = 0; t < 4; t++)
+						s[t] = mfma(bq[ib[x]], aq[t][ch][ia[x]], s[t]);
+			}
+		} else {
+			bf16x8 bq[3];
+#pragma unroll
+			for (int i = 0; i < 3; i++) {
+				const int part = i < 2 ? i : (g < 2 ? 2 : 0);
+				bq[i] = *reinterpret_cast<const bf16x8 *>(slot + (part * 16 + j) * BS + 8 * (g & 1));
+			}
+#pragma unroll
+			for (int x = 2; x >= 0; x--)
+#pragma unroll
+				for (int t = 0; t < 4; t++)
+					s[t] = mfma(bq[x], aq[t][0][x == 2 ? 1 : 0], s[t]);
+		}
+	};
+	bf16x4 pr[4][3];
+	auto ratio = [&](const float4 (&u)[4], const floatx4 (&s)[4], int bb, auto mask_tag) {
+		constexpr bool MASK = decltype(mask_tag)::value;
+#pragma unroll
+		for (int t = 0; t < 4; t++) {
+			float rt[4];
+#pragma unroll
+			for (int r = 0; r < 4; r++) {
+				const float uv = t == 0 ? u[r].x : t == 1 ? u[r].y : t == 2 ? u[r].z : u[r].w;
+				const float v = uv * __builtin_amdgcn_rcpf(s[t][r]);
+				rt[r] = !MASK || bb + 4 * g + r < b_end ? v : 0.0f;
+			}
+			split3x4(rt[0], rt[1], rt[2], rt[3], pr[t]);
+		}
+	};
+	auto gemm2 = [&]() {
+#pragma unroll
+		for (int h = 0; h < H; h++) {
+			bf16x4 b2[3];
+#pragma unroll
+			for (int i = 0; i < 3; i++) {
+				typedef __attribute__((address_space(3))) shortx4 *lds4;
+				const shortx4 v = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+					(lds4)(slot + (i * 16 + 4 * g + (j >> 2)) * BS + 16 * h + 4 * (j & 3)));
+				__builtin_memcpy(&b2[i], &v, 8);
+			}
+#pragma unroll
+			for (int t = 0; t < 4; t++)
+				acc[t][h] = mfma(cat8(pr[t][0], pr[t][2]), cat8(b2[2], b2[0]), acc[t][h]);
+#pragma unroll
+			for (int t = 0; t < 4; t++)
+				acc[t][h] = mfma(cat8(pr[t][1], pr[t][0]), cat8(b2[1], b2[1]), acc[t][h]);
+#pragma unroll
+			for (int t = 0; t < 4; t++)
+				acc[t][h] = mfma(cat8(pr[t][1], pr[t][0]), cat8(b2[0], b2[0]), acc[t][h]);
+		}
+	};
+	if (mine > 0) {
+		for (int i = 0; i < mine; i += DU) {
+#pragma unroll
+			for (int d = 0; d < DU; d++) {
+				if (i + d < mine) {
+					floatx4 s[4];
+					stage_b(br[d % DB]);
+					fetch_b(blk_row(i + d + DB), br[d % DB]);
+					gemm1(s);
+					ratio(ur[d], s, 0, std::false_type{});
+					load_u(blk_row(i + d + DU), ur[d]);
+					gemm2();
+				}
+			}
+		}
+	}
+	if (!idle && (b_end - b_begin) % 16 != 0 && wb == nfull % NB) {
+		// Partial last block of the matrix: rows at or past b_end read row b_begin instead.
+		const int bb = b_begin + 16 * nfull;
+		float4 u[4];
+#pragma unroll
+		for (int r = 0; r < 4; r++) {
+			const int b = bb + 4 * g + r;
+			u[r] = *reinterpret_cast<const float4 *>(U + (size_t)(b < b_end ? b : b_begin) * ldu + ucol);
+		}
+#pragma unroll
+		for (int h = 0; h < H; h++) {
+			const int e = (h * 64 + lane) * 4, b = bb + e / KT;
+			br[0][h] = *reinterpret_cast<const float4 *>(B + (size_t)(b < b_end ? b : b_begin) * KT + e % KT);
+		}
+		floatx4 s[4];
+		stage_b(br[0]);
+		gemm1(s);
+		ratio(u, s, bb, std::true_type{});
+		gemm2();
+	}
+	// Splitting an infinity leaves NaN: where a sum is not finite, the wave's whole share is
+	// summed again on the FP32 instructions, so infinities and NaN come out as those give them.
+	// (Rows a past p divide by zero and are never stored: not looked at.)
+	float z = 0.0f;
+#pragma unroll
+	for (int t = 0; t < 4; t++)
+#pragma unroll
+		for (int r = 0; r < 4; r++) {
+			float y = 0.0f;
+#pragma unroll
+			for (int h = 0; h < H; h++)
+				y = fmaf(acc[t][h][r], 0.0f, y);
+			z += a0 + 4 * (4 * g + r) + t < p ? y : 0.0f;
+		}
+	if (__builtin_expect(!idle && __any(z != 0.0f), 0))
+		sum32<KT, NB>(ha, aj, wb, b_begin, b_end, acc);
+	if constexpr (NB > 1)
+		__syncthreads();   // every wave is done with its slot, which the sums below reuse
+	mfma_store<KT, NA, NB>(acc, ha, by, a0, idle, smem);
+}
+
+template <int KT, int NA, int NB>
+__global__ __launch_bounds__(64 * NA * NB, (KT <= 32 ? 3 : 2)) void k_partial_split(half_args h, const nmfk_state *__restrict__ st, int S)
+{
+	__shared__ __align__(16) float smem[smem_split(KT, NA, NB)];
+	if (st != nullptr && st->converged)
+		return;
+	int bx, by;
+	if (!xcd_tile(h.nab + 1, (h.nab + 1) * S, bx, by))
+		return;
+	partial_split_body<KT, NA, NB>(bx, by, h, smem);
 }
 
 // A[a][c] = (A[a][c] * sum_s part[s][a][c]) / den[c], optional clamp, then the column sums
@@ -1200,7 +1585,7 @@ __global__ __launch_bounds__(NMFK_WG) void k_shadow(const float *__restrict__ A,
 	store_shadow<KT>(a, c0, x, Ab);
 }
 
-template <int KT>
+template <int KT, bool PAIR = false>
 __device__ __forceinline__ void finish_body(int bx, const float *__restrict__ part, int S, float *__restrict__ A,
 					    int p, int k, const float *__restrict__ den, float *__restrict__ colA,
 					    int clamp, float *__restrict__ smem, const shadow_args &sh = shadow_args{})
@@ -1221,6 +1606,14 @@ __device__ __forceinline__ void finish_body(int bx, const float *__restrict__ pa
 #pragma unroll
 			for (int u = 0; u < 8; u++)
 				ldq<Q>(pa + (sp + u) * pst, v[u]);
+			if constexpr (PAIR) {
+#pragma unroll
+				for (int i = 0; i < Q; i++) {
+					const float w[8] = {v[0][i], v[1][i], v[2][i], v[3][i], v[4][i], v[5][i], v[6][i], v[7][i]};
+					s[i] += pair8(w);
+				}
+				continue;
+			}
 #pragma unroll
 			for (int u = 0; u < 8; u++)
 #pragma unroll
@@ -1278,10 +1671,10 @@ __device__ __forceinline__ void finish_body(int bx, const float *__restrict__ pa
 		for (int i = 0; i < Q; i++)
 			x[i] = 0.0f;
 	}
-	block_colsum_store<KT>(x, colA + (size_t)bx * KT, smem);
+	block_colsum_store<KT, PAIR>(x, colA + (size_t)bx * KT, smem);
 }
 
-template <int KT>
+template <int KT, bool PAIR>
 __global__ __launch_bounds__(NMFK_WG) void k_finish(const float *__restrict__ part, int S, float *__restrict__ A,
 						    int p, int k, const float *__restrict__ den,
 						    float *__restrict__ colA, int clamp,
@@ -1290,10 +1683,10 @@ __global__ __launch_bounds__(NMFK_WG) void k_finish(const float *__restrict__ pa
 	__shared__ float smem[smem_fin(KT)];
 	if (st != nullptr && st->converged)
 		return;
-	finish_body<KT>(blockIdx.x, part, S, A, p, k, den, colA, clamp, smem, sh);
+	finish_body<KT, PAIR>(blockIdx.x, part, S, A, p, k, den, colA, clamp, smem, sh);
 }
 
-template <int KT>
+template <int KT, bool PAIR>
 __global__ __launch_bounds__(NMFK_WG) void k_colsum_parts(const float *__restrict__ A, int p,
 							  float *__restrict__ colA)
 {
@@ -1305,7 +1698,7 @@ __global__ __launch_bounds__(NMFK_WG) void k_colsum_parts(const float *__restric
 #pragma unroll
 	for (int i = 0; i < Q; i++)
 		x[i] = (a < p) ? A[(size_t)a * KT + c0 + i] : 0.0f;
-	block_colsum_store<KT>(x, colA + (size_t)blockIdx.x * KT, smem);
+	block_colsum_store<KT, PAIR>(x, colA + (size_t)blockIdx.x * KT, smem);
 }
 
 template <int KT>
@@ -2007,7 +2400,8 @@ __global__ __launch_bounds__(NMFK_WG) void k_test_final(int m, const uint32_t *_
 // job.  Workgroups walk a tile table; a tile is one workgroup (bx, by) of the job's own
 // single-job grid, run by the same body, so the job's arithmetic does not depend on what
 // else is in the batch.  Bodies: VALU <KT, 4, 4> for KT 4/8, MFMA <KT, 1, 4> for KT 16/32
-// (the single-job planner's defaults; the host checks every job's plan before batching).
+// (the single-job planner's defaults; the host checks every job's plan before batching),
+// and the same MFMA shapes on split products.
 // --------------------------------------------------------------------------------------
 
 __device__ __forceinline__ half_args batch_half(const nmfk_bjob &J, int half)
@@ -2048,32 +2442,34 @@ __device__ __forceinline__ void batch_valu_body(int bx, int by, const half_args 
 	}
 }
 
-// Six batched partial kernels, one per body class, so each runs at its own occupancy: the
+// Ten batched partial kernels, one per body class, so each runs at its own occupancy: the
 // VALU bodies (KT 4/8) of half-steps without lane groups, those with lane groups (few rows
 // of the updated factor: their variants need more registers), the matrix-core bodies of KT 16
-// and of KT 32 in 1 x 4 waves, and the same in 2 x 2 waves (the plan of a lone job over a
-// short contraction range); a batch launches each over its own tile table.
+// and of KT 32 in 1 x 4 waves, the same in 2 x 2 waves (the plan of a lone job over a short
+// contraction range), and these four on split products (classes 6-9); a batch launches each
+// over its own tile table.
 __host__ __device__ constexpr int batch_cls_kt(int cls)
 {
-	return (cls == 2 || cls == 4) ? 16 : 32;
+	return cls % 2 == 0 ? 16 : 32;
 }
 __host__ __device__ constexpr int batch_cls_na(int cls)
 {
-	return cls >= 4 ? 2 : 1;
+	return (cls - 2) % 4 >= 2 ? 2 : 1;
 }
 
 template <int CLS>
 constexpr int smem_batch_partial()
 {
-	return CLS <= 1 ? smem_valu(8, 4, 4)
-			: smem_mfma(batch_cls_kt(CLS), batch_cls_na(CLS), 4 / batch_cls_na(CLS));
+	return CLS <= 1   ? smem_valu(8, 4, 4)
+	       : CLS >= 6 ? smem_split(batch_cls_kt(CLS), batch_cls_na(CLS), 4 / batch_cls_na(CLS))
+			  : smem_mfma(batch_cls_kt(CLS), batch_cls_na(CLS), 4 / batch_cls_na(CLS));
 }
 
 template <int CLS>
-__global__ __launch_bounds__(NMFK_WG, (CLS == 0 || CLS == 2 || CLS == 4 ? 4 : 1)) void k_batch_partial(const nmfk_bjob *__restrict__ jobs,
+__global__ __launch_bounds__(NMFK_WG, (CLS == 0 || CLS == 2 || CLS == 4 ? 4 : CLS >= 6 ? 3 : 1)) void k_batch_partial(const nmfk_bjob *__restrict__ jobs,
 							   const nmfk_tile *__restrict__ tiles, int ntiles, int half)
 {
-	__shared__ float smem[smem_batch_partial<CLS>()];
+	__shared__ __align__(16) float smem[smem_batch_partial<CLS>()];
 	for (int t = blockIdx.x; t < ntiles; t += gridDim.x) {
 		const nmfk_tile tl = tiles[t];
 		const nmfk_bjob &J = jobs[tl.job];
@@ -2083,7 +2479,7 @@ __global__ __launch_bounds__(NMFK_WG, (CLS == 0 || CLS == 2 || CLS == 4 ? 4 : 1)
 		bool fits;
 		if constexpr (CLS <= 1)
 			fits = J.kt <= 8 && ((half == 0 ? J.planH.lb : J.planW.lb) > 1) == (CLS == 1);
-		else if constexpr (CLS <= 3)
+		else if constexpr (batch_cls_na(CLS) == 1)
 			fits = J.kt == (uint32_t)batch_cls_kt(CLS);
 		else
 			fits = J.kt == (uint32_t)batch_cls_kt(CLS) && (half == 0 ? J.planH.ap : J.planW.ap) == 2u;
@@ -2102,7 +2498,9 @@ __global__ __launch_bounds__(NMFK_WG, (CLS == 0 || CLS == 2 || CLS == 4 ? 4 : 1)
 				batch_valu_body<8>(tl.bx, tl.by, h, smem);
 		} else {
 			constexpr int KT = batch_cls_kt(CLS), NA = batch_cls_na(CLS), NB = 4 / NA;
-			if constexpr (KT == 16) {
+			if constexpr (CLS >= 6) {
+				partial_split_body<KT, NA, NB>(tl.bx, tl.by, h, smem);
+			} else if constexpr (KT == 16) {
 				// a rank up to 4 or 8 sums only its columns in GEMM1 (nmfk_plan_set_rank)
 				const uint32_t ke = half == 0 ? J.planH.ke : J.planW.ke;
 				if (ke == 4)
@@ -2145,10 +2543,16 @@ __global__ __launch_bounds__(NMFK_WG) void k_batch_finish(const nmfk_bjob *__res
 			finish_body<8>(tl.bx, part, S, A, p, J.k, den, colA, cl, smem);
 			break;
 		case 16:
-			finish_body<16>(tl.bx, part, S, A, p, J.k, den, colA, cl, smem);
+			if (J.split)
+				finish_body<16, true>(tl.bx, part, S, A, p, J.k, den, colA, cl, smem);
+			else
+				finish_body<16>(tl.bx, part, S, A, p, J.k, den, colA, cl, smem);
 			break;
 		case 32:
-			finish_body<32>(tl.bx, part, S, A, p, J.k, den, colA, cl, smem);
+			if (J.split)
+				finish_body<32, true>(tl.bx, part, S, A, p, J.k, den, colA, cl, smem);
+			else
+				finish_body<32>(tl.bx, part, S, A, p, J.k, den, colA, cl, smem);
 			break;
 		}
 		__syncthreads();
@@ -2615,6 +3019,24 @@ extern "C" void nmfk_plan_set_rank(nmfk_hplan *pl, uint32_t kt, uint32_t k)
 		pl->ke = k <= 4u ? 4u : 8u;
 }
 
+// Resident jobs on the FP32 matrix-core path, planned on their own, that run on split products
+// (partial_split_body).  Per iteration, FP32 instructions against split products: k = 16 (12),
+// 5000 x 500 21.3 / 21.4 us, 10000 x 500 27.3 / 27.6, 8000 x 1000 30.3 / 28.8, 20000 x 500 36.0 /
+// 34.1, 20000 x 1000 45.9 / 43.7: at kt 16 the line lies between 5 and 8 million values, below
+// which a block's longer chain costs what the shorter products save.  At kt 32 and 64 they are
+// faster at every size (k = 24 or 32: 3000 x 300 26.4 / 24.5, 1000 x 1000 27.5 / 24.8, 20000 x
+// 1000 74.7 / 58.8; k = 48: 10000 x 1000 95.3 / 71.1), and the line is one of accuracy.  The BF16
+// instructions truncate small terms against large ones, 0.1-0.2 ulp toward zero in sums of
+// heavy-tailed terms, and on smaller lognormal matrices, over 100 iterations, that can show: W and
+// H then came out more than 1.5 times as far from 64 bits as on the FP32 instructions, and over
+// 1e-6, in 7 of 78 shapes of 1 to 6 million values, and in none of 82 larger ones, nor of 80
+// planted ones of all sizes.  In the mean, with the tree sums of pair8, their errors are 0.82
+// times those of the FP32 instructions.
+extern "C" int nmfk_split_rule(uint32_t n, uint32_t m, uint32_t kt, uint32_t k)
+{
+	return kt % 16u == 0 && k > 8u && (size_t)n * m >= (6u << 20);
+}
+
 extern "C" void nmfk_plan_half(uint32_t p, uint32_t q, uint32_t kt, nmfk_hplan *pl)
 {
 	nmfk_plan_half_path(p, q, kt, NMFK_PATH_AUTO, pl);
@@ -2730,6 +3152,61 @@ extern "C" int nmfk_launch_partial(const float *U, size_t ldu, const float *A, c
 	}
 }
 
+template <int KT>
+static int launch_partial_split_t(const half_args &h, const nmfk_hplan *pl, const nmfk_state *st, hipStream_t stream)
+{
+	const dim3 grid = xcd_grid(pl);
+	const int na = (int)pl->ap, nb = pl->ap ? (int)(pl->nw / pl->ap) : 0;
+#define NMFK_SPLIT_SHAPE(NA_, NB_)                                                                       \
+	if (na == NA_ && nb == NB_) {                                                                  \
+		hipLaunchKernelGGL((k_partial_split<KT, NA_, NB_>), grid, dim3(64 * NA_ * NB_), 0, stream, h, st, (int)pl->S); \
+		return (int)hipGetLastError();                                                         \
+	}
+	NMFK_SPLIT_SHAPE(1, 4)
+	NMFK_SPLIT_SHAPE(2, 2)
+	NMFK_SPLIT_SHAPE(4, 1)
+	NMFK_SPLIT_SHAPE(2, 4)
+	NMFK_SPLIT_SHAPE(4, 2)
+#undef NMFK_SPLIT_SHAPE
+	return (int)hipErrorInvalidValue;
+}
+
+extern "C" int nmfk_launch_partial_split(const float *U, size_t ldu, const float *A, const float *B, uint32_t p,
+					 uint32_t q, uint32_t kt, const nmfk_hplan *pl, float *part, const float *colB,
+					 uint32_t ncolB, float *den, const nmfk_state *st, hipStream_t stream)
+{
+	// byte offsets within one 16-row block of U are 32-bit
+	if (ldu % 4 != 0 || pl->path != NMFK_PATH_MFMA32 || pl->bchunk % 16 != 0 || (size_t)16 * ldu * 4 > 0x7fffffffull)
+		return (int)hipErrorInvalidValue;
+	const half_args h = {U, ldu, A, B, (int)p, (int)q, (int)pl->bchunk, (int)pl->nab, part, colB, (int)ncolB, den};
+	switch (kt) {
+#define X(K)                                                                                          \
+	case K:                                                                                       \
+		return launch_partial_split_t<K>(h, pl, st, stream);
+		NMFK_KT_MFMA_LIST(X)
+#undef X
+	default:
+		return (int)hipErrorInvalidValue;
+	}
+}
+
+extern "C" int nmfk_launch_finish_split(const float *part, uint32_t S, float *A, uint32_t p, uint32_t k, uint32_t kt,
+					const float *den, float *colA, int clamp, const nmfk_state *st, hipStream_t stream)
+{
+	const unsigned g = (p + NMFK_FIN_ROWS - 1) / NMFK_FIN_ROWS;
+	switch (kt) {
+#define X(K)                                                                                           \
+	case K:                                                                                        \
+		hipLaunchKernelGGL((k_finish<K, true>), dim3(g), dim3(NMFK_WG), 0, stream, part, (int)S, A, (int)p, \
+				   (int)k, den, colA, clamp, st, shadow_args{});                        \
+		return (int)hipGetLastError();
+		NMFK_KT_MFMA_LIST(X)
+#undef X
+	default:
+		return (int)hipErrorInvalidValue;
+	}
+}
+
 extern "C" int nmfk_launch_finish_shadow(const float *part, uint32_t S, float *A, uint32_t p, uint32_t k,
 					 uint32_t kt, const float *den, float *colA, int clamp, const nmfk_state *st,
 					 uint16_t *Ab, hipStream_t stream)
@@ -2741,7 +3218,7 @@ extern "C" int nmfk_launch_finish_shadow(const float *part, uint32_t S, float *A
 	switch (kt) {
 #define X(K)                                                                                           \
 	case K:                                                                                        \
-		hipLaunchKernelGGL((k_finish<K>), dim3(g), dim3(NMFK_WG), 0, stream, part, (int)S, A, (int)p, \
+		hipLaunchKernelGGL((k_finish<K, false>), dim3(g), dim3(NMFK_WG), 0, stream, part, (int)S, A, (int)p, \
 				   (int)k, den, colA, clamp, st, sh);                                   \
 		return (int)hipGetLastError();
 		NMFK_KT_LIST(X)
@@ -2863,13 +3340,25 @@ extern "C" int nmfk_launch_partial_bf16(const float *U, size_t ldu, const float 
 	}
 }
 
-extern "C" int nmfk_launch_colsum_parts(const float *A, uint32_t p, uint32_t kt, float *colA, hipStream_t stream)
+extern "C" int nmfk_launch_colsum_parts(const float *A, uint32_t p, uint32_t kt, int split, float *colA, hipStream_t stream)
 {
 	const unsigned g = (p + NMFK_FIN_ROWS - 1) / NMFK_FIN_ROWS;
+	if (split) {
+		switch (kt) {
+#define X(K)                                                                                      \
+	case K:                                                                                   \
+		hipLaunchKernelGGL((k_colsum_parts<K, true>), dim3(g), dim3(NMFK_WG), 0, stream, A, (int)p, colA); \
+		return (int)hipGetLastError();
+			NMFK_KT_MFMA_LIST(X)
+#undef X
+		default:
+			return (int)hipErrorInvalidValue;
+		}
+	}
 	switch (kt) {
 #define X(K)                                                                                      \
 	case K:                                                                                   \
-		hipLaunchKernelGGL((k_colsum_parts<K>), dim3(g), dim3(NMFK_WG), 0, stream, A, (int)p, colA); \
+		hipLaunchKernelGGL((k_colsum_parts<K, false>), dim3(g), dim3(NMFK_WG), 0, stream, A, (int)p, colA); \
 		return (int)hipGetLastError();
 		NMFK_KT_LIST(X)
 #undef X
@@ -2935,6 +3424,18 @@ extern "C" int nmfk_launch_batch_partial(const nmfk_bjob *jobs, const nmfk_tile 
 		break;
 	case 5:
 		hipLaunchKernelGGL((k_batch_partial<5>), g, dim3(NMFK_WG), 0, stream, jobs, tiles, (int)ntiles, half);
+		break;
+	case 6:
+		hipLaunchKernelGGL((k_batch_partial<6>), g, dim3(NMFK_WG), 0, stream, jobs, tiles, (int)ntiles, half);
+		break;
+	case 7:
+		hipLaunchKernelGGL((k_batch_partial<7>), g, dim3(NMFK_WG), 0, stream, jobs, tiles, (int)ntiles, half);
+		break;
+	case 8:
+		hipLaunchKernelGGL((k_batch_partial<8>), g, dim3(NMFK_WG), 0, stream, jobs, tiles, (int)ntiles, half);
+		break;
+	case 9:
+		hipLaunchKernelGGL((k_batch_partial<9>), g, dim3(NMFK_WG), 0, stream, jobs, tiles, (int)ntiles, half);
 		break;
 	default:
 		return (int)hipErrorInvalidValue;

@@ -396,7 +396,7 @@ int nmfk_stream_run(nmfk_job *j, const nmfk_options *opt, nmfk_result *res)
 	j->stream_bytes = 0.0;
 	int e = nmfk_launch_state_reset(j->st, opt->stop_threshold, UINT32_MAX, j->last, j->m, j->stream);
 	if (!e)
-		e = nmfk_launch_colsum_parts(j->W, j->n, j->kt, j->colW, j->stream);
+		e = nmfk_launch_colsum_parts(j->W, j->n, j->kt, j->split, j->colW, j->stream);
 	if (!e)
 		e = nmfk_launch_den(j->colW, j->ncolW, j->kt, j->denW, j->stream);
 	if (!e)
@@ -493,7 +493,7 @@ int nmfk_stream_dot_kl(nmfk_job *j, double *dot_V, double *dot_VWH, double *kl)
  * over V adding the H partial sums, then the H finish.  Not gated by the stop state. */
 int nmfk_stream_update_H(nmfk_job *j)
 {
-	int e = nmfk_launch_colsum_parts(j->W, j->n, j->kt, j->colW, j->stream);
+	int e = nmfk_launch_colsum_parts(j->W, j->n, j->kt, j->split, j->colW, j->stream);
 	if (!e)
 		e = nmfk_launch_den(j->colW, j->ncolW, j->kt, j->denW, j->stream);
 	if (e)
@@ -510,7 +510,7 @@ int nmfk_stream_update_H(nmfk_job *j)
  * block by block. */
 int nmfk_stream_update_W(nmfk_job *j)
 {
-	int e = nmfk_launch_colsum_parts(j->H, j->m, j->kt, j->colH, j->stream);
+	int e = nmfk_launch_colsum_parts(j->H, j->m, j->kt, j->split, j->colH, j->stream);
 	if (e)
 		return nmfk_hip_fail(e, "update_W");
 	return pass(j, PASS_W, NULL, 0, NULL, NULL);

@@ -115,6 +115,62 @@ def test_small_rank_shapes_match_oracle(nmfk, orc, k, na, nb):
         nmfk.tune_set(nmfk.TUNE_MFMA_NB, old[1])
 
 
+@pytest.mark.parametrize("n,m,k", [(98311, 64, 17), (98400, 65, 32), (6465, 1000, 33), (1041, 6151, 64),
+                                   (191000, 33, 24), (25601, 257, 48), (6465, 1000, 9), (6401, 1087, 16),
+                                   (1087, 6401, 12)])
+def test_split_products_match_oracle(nmfk, orc, n, m, k):
+    # Jobs that run on products of three-part BF16 operands (nmfk_split_rule), at sizes around
+    # the 16-row blocks, the 64-row tiles and the wave groups' shares: each half-step within the
+    # FP32 bar of the oracle, and the FP32 instructions (the same job replanned to a workgroup
+    # target) within the same bar.
+    job, V = make_job(nmfk, orc, n, m, k, seed_v=n + m, seed_init=k)
+    with job:
+        job.set_kernel_path(2)
+        W, H = orc.init_WH(n, m, k, k)
+        H1 = orc.update_H(V, W, H)
+        W1 = orc.update_W(V, W, H1)
+        for target in (0, 1024):
+            job.replan(target)
+            job.set_WH(W, H)
+            job.update_H()
+            assert rel_err(job.get_H(), H1) < 1e-5
+            job.update_W()
+            assert rel_err(job.get_W(), W1) < 1e-5
+
+
+@pytest.mark.parametrize("n,m,k", [(90001, 70, 12), (90001, 70, 24), (90001, 70, 48)])
+def test_split_products_keep_infinities(nmfk, orc, n, m, k):
+    # An infinite value of V makes its column's H row infinite, as on the FP32 instructions; the
+    # other rows of H stay finite and right.
+    V = orc.gen_lognormal(n, m, 3, 0.0, 1.0)
+    W, H = orc.init_WH(n, m, k, 5)
+    want = orc.update_H(V, W, H)
+    V[100, 37] = np.inf
+    with nmfk.Job(n, m, k) as job:
+        job.set_V(V)
+        job.init_random(5)
+        job.set_kernel_path(2)
+        job.update_H()
+        got = job.get_H()
+    assert np.all(np.isposinf(got[37]))
+    keep = np.arange(m) != 37
+    assert rel_err(got[keep], want[keep]) < 1e-5
+
+
+@pytest.mark.parametrize("n,m,k", [(6401, 1087, 13), (98400, 65, 30)])
+def test_split_products_same_bits_in_a_batch(nmfk, n, m, k):
+    with nmfk.Job(n, m, k) as a, nmfk.Job(n, m, k) as b:
+        batch = nmfk.Batch(5, 4)
+        for j in (a, b):
+            j.gen_V_lognormal(9, 0.0, 1.0)
+            j.init_random(4)
+        a.run(20, 5, 1000)
+        batch.add(b, 20, 1000)
+        batch.run()
+        batch.close()
+        assert np.array_equal(a.get_W(), b.get_W()) and np.array_equal(a.get_H(), b.get_H())
+
+
 def test_golden_tiny_runs(nmfk, orc):
     g = np.load(GOLDEN / "tiny.npz")
     for ci in range(int(g["ncases"])):
