@@ -2704,40 +2704,153 @@ __global__ __launch_bounds__(256) void k_transpose(const float *__restrict__ V, 
 
 // --------------------------------------------------------------------------------------
 // FP64 Frobenius and KL sums (dot_product_VWH, src/NMF_routines.c:1758-2794, plus the
-// generalized KL objective).  Lane = column j; the block's row range is strided over.
+// generalized KL objective).  Block (bx, by) covers columns 256 bx.. and the by-th of 64 row
+// ranges and writes one triple of sums.
+//
+// What bounds it is FP64 arithmetic on every element, the KL term's quotient and logarithm
+// above all (the 80 MB of V at 20000 x 1000 take 13 us).  So the products W . H run on the FP64
+// matrix cores (16x16x4, no conversions per element), and log(v / wh) takes one reciprocal
+// altogether: with v = mv 2^ev and wh = mw 2^ew, mantissas in [1/2, 1),
+//   log(v / wh) = (ev - ew) ln 2 + 2 atanh(s),  s = (mv - mw) / (mv + mw),  |s| < 1/3,
+// atanh(s) / s a polynomial of degree 10 in s^2 (interpolated at the Chebyshev points of
+// [0, 1/9]; relative error 2e-18).  The difference mv - mw is exact near v = wh, where the
+// logarithm is small.
+// A wave takes 64 columns in the 4 tiles of the partial kernels (column j0 + 4 l + t, so V
+// comes in whole float4s) and 16-row blocks; up to four waves side by side cover the columns,
+// the others share the rows, so a narrow V fills the workgroup too.  8 waves, 4 at KT 64 where
+// H takes 128 registers (8 waves spill: 740 against 397 us); 16 waves at KT 16 were even.
+// Measured, a lane per column and the library's division and logarithm -> this kernel:
+// 20000 x 1000, k = 16 197 -> 52 us; 50000 x 2000, k = 64 1469 -> 397; 60000 x 20, k = 4
+// 378 -> 29; 1000 x 20000, k = 20 207 -> 93.  About 57 vector instructions per element bound it.
 // --------------------------------------------------------------------------------------
 
 #define DOT_ROWSPLIT 64
 
-template <int KT>
-__global__ __launch_bounds__(256) void k_dot_kl(const float *__restrict__ V, size_t ldv,
-						const float *__restrict__ W, const float *__restrict__ H,
-						int n, int m, double *__restrict__ parts)
+typedef double doublex4 __attribute__((ext_vector_type(4)));
+
+// Q consecutive floats from any float's address (the buffers may be a caller's own).
+template <int Q>
+__device__ __forceinline__ void ldq_any(const float *__restrict__ p, float (&v)[Q])
 {
-	const int j = blockIdx.x * 256 + threadIdx.x;
-	const int rows_per = (n + gridDim.y - 1) / gridDim.y;
+	__builtin_memcpy(v, p, 4 * Q);
+}
+
+__host__ __device__ constexpr int dot_waves(int kt)
+{
+	return kt <= 32 ? 8 : 4;
+}
+
+// Coefficients of (atanh(s) / s - 1) / s^2, highest first.  Read from constant memory into
+// scalar registers: as literals each would first be copied into the vector register that the
+// multiply-add overwrites.
+__constant__ double c_atanh[10] = {0.08522081781390699, 0.0416225325593041,  0.06055084364034609, 0.06650187016337313,
+				   0.07693307021152004, 0.09090870416252403, 0.11111112040373837, 0.14285714272727057,
+				   0.20000000000092874, 0.33333333333333076};
+
+// log(v / wh) for v > 0 (see above), without branches; +inf for wh = 0, NaN for a negative wh
+// or NaN.
+__device__ __forceinline__ double log_ratio(float v, double wh)
+{
+	const double mv = (double)__builtin_amdgcn_frexp_mantf(v), mw = __builtin_amdgcn_frexp_mant(wh);
+	const int e = __builtin_amdgcn_frexp_expf(v) - __builtin_amdgcn_frexp_exp(wh);
+	const double num = mv - mw, den = mv + mw;
+	double r = __builtin_amdgcn_rcp(den);   // 2^-23; 2^-46 after the step
+	r = fma(r, fma(-den, r, 1.0), r);
+	double s = num * r;
+	s = fma(r, fma(-den, s, num), s);
+	const double z = s * s;
+	double p = c_atanh[0];
+#pragma unroll
+	for (int i = 1; i < 10; i++)
+		p = fma(p, z, c_atanh[i]);
+	// 2 s (1 + z p) + e ln 2, ln 2 in two parts whose first has 11 trailing zero bits
+	const double a = fma(s * z, p + p, s + s);
+	const double odd = wh == 0.0 ? __builtin_inf() : __builtin_nan(""), ei = (double)e;
+	const double ed = wh > 0.0 ? ei : odd;
+	return fma(ed, 0x1.62e42fefa3800p-1, fma(ed, 0x1.ef35793c76730p-45, a));
+}
+
+template <int KT>
+__global__ __launch_bounds__(64 * dot_waves(KT)) void k_dot_kl(const float *__restrict__ V, size_t ldv,
+							       const float *__restrict__ W, const float *__restrict__ H,
+							       int n, int m, double *__restrict__ parts)
+{
+	constexpr int NW = dot_waves(KT), KQ = KT / 4;
+	const int lane = threadIdx.x & 63, l16 = lane & 15, g = lane >> 4;
+	const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+	const int ncw = min(4, (m - (int)blockIdx.x * 256 + 63) / 64);   // waves side by side
+	const int cw = wave % ncw, rg = wave / ncw, nrg = NW / ncw;
+	// Row ranges in use: all 64, or for a wide V as many as give 512 workgroups (their set-up,
+	// H converted to FP64, is worth several row blocks).
+	const int nsp = min((int)gridDim.y, (511 + (int)gridDim.x) / (int)gridDim.x);
+	const int rows_per = ((n + nsp - 1) / nsp + 15) & ~15;
 	const int i0 = blockIdx.y * rows_per, i1 = min(n, i0 + rows_per);
-	double hj[KT];
-#pragma unroll
-	for (int c = 0; c < KT; c++)
-		hj[c] = (j < m) ? (double)H[(size_t)j * KT + c] : 0.0;
+	const int j0 = blockIdx.x * 256 + cw * 64, jl = j0 + 4 * l16;   // this lane's 4 columns: jl + t
 	double sv = 0.0, sd = 0.0, sk = 0.0;
-	if (j < m) {
-		for (int i = i0; i < i1; i++) {
-			const float *Wi = W + (size_t)i * KT;
-			double wh = 0.0;
+	if (rg < nrg && i0 < i1) {
+		// GEMM operand of H: lane (g, l16) supplies H[jl + t][KQ g + q] for K step q.
+		double hop[4][KQ];
 #pragma unroll
-			for (int c = 0; c < KT; c++)
-				wh += (double)Wi[c] * hj[c];
-			const double v = (double)V[(size_t)i * ldv + j];
-			const double d = v - wh;
-			sv += v * v;
-			sd += d * d;
-			sk += (v > 0.0 ? v * log(v / wh) : 0.0) - v + wh;
+		for (int t = 0; t < 4; t++) {
+			float x[KQ];
+			ldq_any<KQ>(H + (size_t)(jl + t < m ? jl + t : 0) * KT + KQ * g, x);
+#pragma unroll
+			for (int q = 0; q < KQ; q++)
+				hop[t][q] = jl + t < m ? (double)x[q] : 0.0;
+		}
+		// V rows come through a descriptor that ends with the matrix (rows past it read zero);
+		// columns past m are masked.
+		const int voff = jl * 4;
+		struct blk {
+			float4 v[4];
+			float w[KQ];
+		};
+		auto load = [&](int ib, blk &x) {
+			const int rows = min(16, i1 - ib);
+			const size_t row = (size_t)ib * ldv;
+			const __amdgpu_buffer_rsrc_t rv = make_rsrc(V + row, ((size_t)(rows - 1) * ldv + m) * 4);
+#pragma unroll
+			for (int r = 0; r < 4; r++)
+				x.v[r] = bload4(rv, (4 * r + g) * (int)(ldv * 4) + voff, 0);
+			ldq_any<KQ>(W + (size_t)min(ib + l16, n - 1) * KT + KQ * g, x.w);
+		};
+		blk x;
+		if (i0 + 16 * rg < i1)
+			load(i0 + 16 * rg, x);
+		for (int ib = i0 + 16 * rg; ib < i1; ib += 16 * nrg) {
+			double wop[KQ];
+#pragma unroll
+			for (int q = 0; q < KQ; q++)
+				wop[q] = ib + l16 < i1 ? (double)x.w[q] : 0.0;
+			float v[4][4];
+#pragma unroll
+			for (int r = 0; r < 4; r++) {
+				const float u[4] = {x.v[r].x, x.v[r].y, x.v[r].z, x.v[r].w};
+#pragma unroll
+				for (int t = 0; t < 4; t++)
+					v[r][t] = jl + t < m && ib + 4 * r + g < i1 ? u[t] : 0.0f;
+			}
+			if (ib + 16 * nrg < i1)
+				load(ib + 16 * nrg, x);
+#pragma unroll
+			for (int t = 0; t < 4; t++) {
+				// wh[r] = W[ib + 4r + g] . H[jl + t]
+				doublex4 wh = {0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+				for (int q = 0; q < KQ; q++)
+					wh = __builtin_amdgcn_mfma_f64_16x16x4f64(wop[q], hop[t][q], wh, 0, 0, 0);
+#pragma unroll
+				for (int r = 0; r < 4; r++) {
+					const double vd = (double)v[r][t], d = vd - wh[r];
+					sv = fma(vd, vd, sv);
+					sd = fma(d, d, sd);
+					const double kl = vd * log_ratio(v[r][t], wh[r]);   // for every v: a select, no branch
+					sk += (v[r][t] > 0.0f ? kl : 0.0) - d;
+				}
+			}
 		}
 	}
-	__shared__ double red[3][4];
-	const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+	__shared__ double red[3][NW];
 	sv = wave_sum_d(sv);
 	sd = wave_sum_d(sd);
 	sk = wave_sum_d(sk);
@@ -2749,8 +2862,10 @@ __global__ __launch_bounds__(256) void k_dot_kl(const float *__restrict__ V, siz
 	__syncthreads();
 	if (threadIdx.x < 3) {
 		const int q = threadIdx.x;
-		parts[((size_t)blockIdx.y * gridDim.x + blockIdx.x) * 3 + q] =
-			((red[q][0] + red[q][1]) + red[q][2]) + red[q][3];
+		double s = 0.0;
+		for (int w = 0; w < NW; w++)
+			s += red[q][w];
+		parts[((size_t)blockIdx.y * gridDim.x + blockIdx.x) * 3 + q] = s;
 	}
 }
 
@@ -3541,7 +3656,7 @@ extern "C" int nmfk_launch_dot_kl(const float *V, size_t ldv, const float *W, co
 	switch (kt) {
 #define X(K)                                                                                      \
 	case K:                                                                                   \
-		hipLaunchKernelGGL((k_dot_kl<K>), grid, dim3(256), 0, stream, V, ldv, W, H, (int)n, (int)m, \
+		hipLaunchKernelGGL((k_dot_kl<K>), grid, dim3(64 * dot_waves(K)), 0, stream, V, ldv, W, H, (int)n, (int)m, \
 				   parts);                                                        \
 		return (int)hipGetLastError();
 		NMFK_KT_LIST(X)

@@ -269,6 +269,36 @@ def test_dot_and_kl_match_oracle(nmfk, orc):
         assert abs(kl - okl) / okl < 1e-9
 
 
+@pytest.mark.parametrize("n,m,k", [(1, 1, 1), (16, 64, 4), (17, 65, 9), (333, 20, 8), (1023, 257, 16), (50, 5003, 20),
+                                   (2049, 70, 33)])
+def test_dot_kl_matches_float64(nmfk, orc, n, m, k):
+    # Sizes around the 16-row blocks, the 64-column waves and the 256-column workgroups, V with
+    # zeros, values of 60 orders of magnitude; a zero product under a positive value gives an
+    # infinite divergence.
+    rng = np.random.default_rng(n + m)
+    V = np.exp(rng.normal(0.0, 20.0, (n, m))).clip(0, 1e18).astype(np.float32)
+    V[rng.random((n, m)) < 0.1] = 0.0
+    W, H = orc.init_WH(n, m, k, 3)
+    with nmfk.Job(n, m, k) as job:
+        W0 = W.copy()
+        W0[0] = 0.0
+        V[0, 0] = 1.0
+        job.set_V(V)
+        job.set_WH(W0, H)
+        assert job.dot_kl()[2] == np.inf
+    V[0, 0] = 0.0
+    v, wh = V.astype(np.float64), W.astype(np.float64) @ H.T.astype(np.float64)
+    with nmfk.Job(n, m, k) as job:
+        job.set_V(V)
+        job.set_WH(W, H)
+        got = job.dot_kl()
+    kl = np.where(v > 0, v * np.log(np.where(v > 0, v, 1.0) / wh), 0.0) - v + wh
+    want = (np.sum(v * v), np.sum((v - wh) ** 2), np.sum(kl))
+    scale = (want[0], want[1], np.sum(np.abs(kl)))
+    for a, b, c in zip(got, want, scale):
+        assert abs(a - b) <= 1e-12 * c + 1e-300
+
+
 def test_stop_rule_on_device_matches_oracle_trace(nmfk, orc):
     # Per-test differences counted on the device (contingency table) reproduce the
     # oracle's pairwise count through the whole run, including the reset cases.
