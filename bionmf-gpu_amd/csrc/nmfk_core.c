@@ -735,62 +735,32 @@ int nmfk_job_get_H(nmfk_job *j, float *H, size_t ldh)
 
 /* ---------------------------------------------------------------- half-steps */
 
-static int partial_H(nmfk_job *j, const nmfk_state *st)
-{
-	if (j->split)
-		return nmfk_launch_partial_split(j->V, j->ldv, j->H, j->W, j->m, j->n, j->kt, &j->planH, j->part,
-						 j->colW, j->ncolW, j->denW, st, j->stream);
-	if (j->planH.path == NMFK_PATH_MFMA_BF16)
-		return nmfk_launch_partial_bf16(j->V, j->ldv, j->H, j->Wb, j->m, j->n, j->kt, &j->planH, j->part,
-						j->colW, j->ncolW, j->denW, st, j->stream);
-	return nmfk_launch_partial(j->V, j->ldv, j->H, j->W, j->m, j->n, j->kt, &j->planH, j->part, j->colW,
-				   j->ncolW, j->denW, st, j->stream);
-}
+/* Half-step <half>: 0 = H through V against W, 1 = W through Vt against H.  Finishing it updates
+ * the factor, its column-sum partials (the other half's denominators) and its BF16 copy where
+ * the other half reads that.  what: the whole half-step, or for timing its sums or its finish. */
+enum { HALF_WHOLE, HALF_SUMS, HALF_FINISH };
 
-static int partial_W(nmfk_job *j, const nmfk_state *st)
+static int half_step(nmfk_job *j, int half, int what, int clamp, const nmfk_state *st)
 {
-	if (j->split)
-		return nmfk_launch_partial_split(j->Vt, j->ldvt, j->W, j->H, j->n, j->m, j->kt, &j->planW, j->part,
-						 j->colH, j->ncolH, j->denH, st, j->stream);
-	if (j->planW.path == NMFK_PATH_MFMA_BF16)
-		return nmfk_launch_partial_bf16(j->Vt, j->ldvt, j->W, j->Hb, j->n, j->m, j->kt,
-						&j->planW, j->part, j->colH, j->ncolH, j->denH, st, j->stream);
-	return nmfk_launch_partial(j->Vt, j->ldvt, j->W, j->H, j->n, j->m, j->kt, &j->planW, j->part, j->colH,
-				   j->ncolH, j->denH, st, j->stream);
-}
-
-/* H half: the partial kernel streams V against W (and reduces colsum(W) into denW), the
- * finish kernel applies the update to H and leaves colsum(H) partials for the W half (and
- * the BF16 copy of H when the W half runs in BF16).  On the BF16 path W is read from its
- * BF16 copy, which the W half's finish (or nmfk_job_shadow_for_H) keeps current. */
-static int finish_H(nmfk_job *j, const nmfk_state *st)
-{
-	if (j->split)
-		return nmfk_launch_finish_split(j->part, j->planH.S, j->H, j->m, j->k, j->kt, j->denW, j->colH, 0, st,
-						j->stream);
-	return nmfk_launch_finish_shadow(j->part, j->planH.S, j->H, j->m, j->k, j->kt, j->denW, j->colH, 0, st,
-					 j->planW.path == NMFK_PATH_MFMA_BF16 ? j->Hb : NULL, j->stream);
-}
-
-static int finish_W(nmfk_job *j, const nmfk_state *st, int clamp)
-{
-	if (j->split)
-		return nmfk_launch_finish_split(j->part, j->planW.S, j->W, j->n, j->k, j->kt, j->denH, j->colW, clamp, st,
-						j->stream);
-	return nmfk_launch_finish_shadow(j->part, j->planW.S, j->W, j->n, j->k, j->kt, j->denH, j->colW, clamp, st,
-					 j->planH.path == NMFK_PATH_MFMA_BF16 ? j->Wb : NULL, j->stream);
+	const nmfk_hplan *pl = half ? &j->planW : &j->planH, *other = half ? &j->planH : &j->planW;
+	const nmfk_half g = {half ? j->Vt : j->V, half ? j->ldvt : j->ldv, half ? j->W : j->H, half ? j->H : j->W,
+			     half ? j->Hb : j->Wb, half ? j->n : j->m, half ? j->m : j->n, j->kt, j->split, j->part};
+	const nmfk_fin f = {half ? j->W : j->H, half ? j->colW : j->colH,
+			    other->path != NMFK_PATH_MFMA_BF16 ? NULL : half ? j->Wb : j->Hb, half ? j->colH : j->colW,
+			    half ? j->ncolH : j->ncolW, half ? j->denH : j->denW, j->k, clamp};
+	if (what == HALF_FINISH)
+		return nmfk_launch_finish(j->part, pl->S, g.p, j->kt, j->split, &f, st, j->stream);
+	return nmfk_launch_half(&g, pl, what == HALF_WHOLE ? &f : NULL, st, j->stream);
 }
 
 int nmfk_enqueue_half_H(nmfk_job *j, const nmfk_state *st)
 {
-	const int e = partial_H(j, st);
-	return e ? e : finish_H(j, st);
+	return half_step(j, 0, HALF_WHOLE, 0, st);
 }
 
 int nmfk_enqueue_half_W(nmfk_job *j, const nmfk_state *st, int clamp)
 {
-	const int e = partial_W(j, st);
-	return e ? e : finish_W(j, st, clamp);
+	return half_step(j, 1, HALF_WHOLE, clamp, st);
 }
 
 int nmfk_job_shadow_for_H(nmfk_job *j)
@@ -1064,7 +1034,13 @@ static int time_loop(nmfk_job *j, uint32_t iters, int kind, double *ms)
 		e = hipEventCreate(&b);
 	if (e)
 		return nmfk_hip_fail(e, "hipEventCreate");
-	e = hipEventRecord(a, j->stream);
+	/* the finishes alone divide by denominators a half-step leaves behind */
+	if (kind == 2)
+		e = nmfk_launch_den(j->colW, j->ncolW, j->kt, j->denW, j->stream);
+	else if (kind == 4)
+		e = nmfk_launch_den(j->colH, j->ncolH, j->kt, j->denH, j->stream);
+	if (!e)
+		e = hipEventRecord(a, j->stream);
 	for (uint32_t i = 0; i < iters && !e; i++) {
 		switch (kind) {
 		case 0:
@@ -1073,16 +1049,16 @@ static int time_loop(nmfk_job *j, uint32_t iters, int kind, double *ms)
 				e = nmfk_enqueue_half_W(j, NULL, 0);
 			break;
 		case 1:
-			e = partial_H(j, NULL);
+			e = half_step(j, 0, HALF_SUMS, 0, NULL);
 			break;
 		case 2:
-			e = finish_H(j, NULL);
+			e = half_step(j, 0, HALF_FINISH, 0, NULL);
 			break;
 		case 3:
-			e = partial_W(j, NULL);
+			e = half_step(j, 1, HALF_SUMS, 0, NULL);
 			break;
 		case 4:
-			e = finish_W(j, NULL, 0);
+			e = half_step(j, 1, HALF_FINISH, 0, NULL);
 			break;
 		}
 	}

@@ -74,7 +74,6 @@ struct nmfk_job {
 	float *partH;                  /* the H half's partial sums of all blocks, in block order */
 	uint32_t SH;                   /* slices in partH */
 	float *Hc;                     /* clamped copy of H that test passes contract against */
-	float *den_scratch;            /* where the block partials' denominator tile writes */
 	hipStream_t cstream;           /* host-to-device copies */
 	hipEvent_t up[2], done[2];     /* slot s: block uploaded / block's kernels finished */
 	double stream_bytes;           /* bytes of V copied to the device by the last run */

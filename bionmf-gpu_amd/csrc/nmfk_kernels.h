@@ -83,30 +83,40 @@ void nmfk_plan_half_path(uint32_t p, uint32_t q, uint32_t kt, int path, nmfk_hpl
 void nmfk_plan_half_target(uint32_t p, uint32_t q, uint32_t kt, int path, uint32_t target, nmfk_hplan *pl);
 
 /*
- * Half-step, first kernel: part[s][a][c] = sum over b in split s of
+ * A half-step: part[s][a][c] = sum over b in split s of
  *   B[b][c] * U[b][a] / (sum_c' A[a][c'] * B[b][c'])
  * H half: U = V (q = n, p = m), A = H, B = W.   W half: U = Vt (q = m, p = n), A = W, B = H.
- * Workgroup (0,0) also writes den[c] = sum_g colB[g][c] (the column sums of B).
+ * With a nmfk_fin it is finished, in the same launch where the plan has one split, else in a
+ * second one:
+ *   A[a][c] = (A[a][c] * sum_s part[s][a][c]) / sum_g colB[g][c]     for c < k
+ * then optionally the R_MIN clamp, then colA[blk][c] = column sums of the new A over each block
+ * of NMFK_FIN_ROWS rows (the next half-step's denominators).  Without one it leaves part.
  */
-int nmfk_launch_partial(const float *U, size_t ldu, const float *A, const float *B,
-			uint32_t p, uint32_t q, uint32_t kt, const nmfk_hplan *pl,
-			float *part, const float *colB, uint32_t ncolB, float *den,
-			const nmfk_state *st, hipStream_t stream);
+typedef struct nmfk_half {
+	const float *U;
+	size_t ldu;
+	const float *A, *B;
+	const uint16_t *Bb;   /* row-major BF16 copy of B (plan path NMFK_PATH_MFMA_BF16 reads it instead of B) */
+	uint32_t p, q, kt;
+	int split;            /* products of three-part BF16 operands (FP32 accuracy; kt 16, 32, 64 on plan path
+				 NMFK_PATH_MFMA32; sums every column of kt, and splits, rows and column sums as trees) */
+	float *part;
+} nmfk_half;
+typedef struct nmfk_fin {
+	float *A, *colA;
+	uint16_t *Ab;         /* BF16 copy of the new A to keep (kt % 32 == 0), or NULL */
+	const float *colB;
+	uint32_t ncolB;
+	float *den;           /* receives the column sums of B */
+	uint32_t k;
+	int clamp;
+} nmfk_fin;
+int nmfk_launch_half(const nmfk_half *g, const nmfk_hplan *pl, const nmfk_fin *fin, const nmfk_state *st,
+		     hipStream_t stream);
 
-/* The same sums from products of three-part BF16 operands (FP32 accuracy; kt 16, 32, 64 on
- * plan path NMFK_PATH_MFMA32; sums every column of kt). */
-int nmfk_launch_partial_split(const float *U, size_t ldu, const float *A, const float *B, uint32_t p, uint32_t q,
-			      uint32_t kt, const nmfk_hplan *pl, float *part, const float *colB, uint32_t ncolB,
-			      float *den, const nmfk_state *st, hipStream_t stream);
 /* Whether a resident FP32 matrix-core job planned on its own runs on split products. */
 int nmfk_split_rule(uint32_t n, uint32_t m, uint32_t kt, uint32_t k);
 
-/*
- * Half-step, second kernel:
- *   A[a][c] = (A[a][c] * sum_s part[s][a][c]) / den[c]     for c < k
- * then optionally the R_MIN clamp, then colA[blk][c] = column sums of the new A over
- * each block of NMFK_FIN_ROWS rows (the next half-step's denominators).
- */
 /* One pass over V per iteration (k_fused_mfma): eligible shapes and their launch plan.
  * Returns 0 and the workgroups G and waves per workgroup when the pass can run the job
  * (kt 16, m <= 1024), else nonzero. */
@@ -119,31 +129,16 @@ int nmfk_launch_fused(const float *V, size_t ldv, float *W, const float *H, uint
 /* H = H * (sum of the G slices) / (sum of the G colW rows), columns < k. */
 int nmfk_launch_fused_finish(const float *part, uint32_t G, const float *colW, float *H, uint32_t m, uint32_t k,
 			     uint32_t kt, const nmfk_state *st, hipStream_t stream);
-int nmfk_launch_finish(const float *part, uint32_t S, float *A, uint32_t p, uint32_t k, uint32_t kt,
-		       const float *den, float *colA, int clamp, const nmfk_state *st,
-		       hipStream_t stream);
-
-/* The same for a job on split products: sums as trees instead of in ascending order. */
-int nmfk_launch_finish_split(const float *part, uint32_t S, float *A, uint32_t p, uint32_t k, uint32_t kt,
-			     const float *den, float *colA, int clamp, const nmfk_state *st, hipStream_t stream);
-/* The finish in ascending order, also writing the BF16 copy of the new A: Ab (p x kt, row-major); kt % 32 == 0
- * when Ab is given. */
-int nmfk_launch_finish_shadow(const float *part, uint32_t S, float *A, uint32_t p, uint32_t k, uint32_t kt,
-			      const float *den, float *colA, int clamp, const nmfk_state *st, uint16_t *Ab,
-			      hipStream_t stream);
+/* The finish by itself: S slices of part, with fin->den given (colB is not read). */
+int nmfk_launch_finish(const float *part, uint32_t S, uint32_t p, uint32_t kt, int split, const nmfk_fin *fin,
+		       const nmfk_state *st, hipStream_t stream);
 /* The BF16 copy of A alone (initial factors). */
 int nmfk_launch_shadow(const float *A, uint32_t p, uint32_t kt, uint16_t *Ab, hipStream_t stream);
-/* Partial kernel with both contractions in BF16 (plan path NMFK_PATH_MFMA_BF16): B is read
- * from its row-major BF16 copy Bb (q x kt). */
-int nmfk_launch_partial_bf16(const float *U, size_t ldu, const float *A, const uint16_t *Bb, uint32_t p, uint32_t q,
-			     uint32_t kt, const nmfk_hplan *pl, float *part, const float *colB, uint32_t ncolB,
-			     float *den, const nmfk_state *st, hipStream_t stream);
-
 /* colA[blk][c] = sum of A[a][c] over the rows of block blk (same order as the finish of a job
  * with or without split products). */
 int nmfk_launch_colsum_parts(const float *A, uint32_t p, uint32_t kt, int split, float *colA, hipStream_t stream);
 
-/* den[c] = sum_g parts[g][c] in the fixed order the partial kernel uses. */
+/* den[c] = sum_g parts[g][c] in the fixed order a half-step uses. */
 int nmfk_launch_den(const float *parts, uint32_t nparts, uint32_t kt, float *den, hipStream_t stream);
 
 /*

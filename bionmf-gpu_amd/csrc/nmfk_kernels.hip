@@ -107,11 +107,10 @@ __device__ __forceinline__ double wave_sum_d(double v)
 	return v;
 }
 
-// Denominator of a half-step: den[c] = sum over the nparts column-sum partials of the
-// other factor.  Four interleaved ascending partial sums per column, combined in a fixed
-// order, so every kernel that forms it gets the same bits.  Needs 4*KT <= blockDim.x.
 // Workgroup size of every half-step kernel (single-job and batched launches alike).
 #define NMFK_WG 256
+
+typedef float floatx4 __attribute__((ext_vector_type(4)));
 
 // Eight values as a tree: 3 roundings deep instead of 8.  The sums over splits, rows and
 // column-sum partials of a job on split products are formed this way, which takes their
@@ -123,38 +122,49 @@ __device__ __forceinline__ float pair8(const float (&v)[8])
 	return ((v[0] + v[1]) + (v[2] + v[3])) + ((v[4] + v[5]) + (v[6] + v[7]));
 }
 
-// den[c] = sum_g parts[g][c]: four interleaved running sums per column, added in a fixed
-// order at the end.  s4 is 4*KT floats of LDS; needs 4*KT <= NMFK_WG threads.
-// PAIR: 8 loaded values are added as a tree before they join the running sum (jobs on split
-// products; see pair8).
+// den[c] = sum_g parts[g][c]: four interleaved ascending sums per column, added in a fixed order
+// at the end (PAIR, jobs on split products: 8 values at a time are added as a tree before they
+// join the running sum; see pair8).  s4 is 4 KT floats of LDS, and <room> more follow it, through
+// which all threads fetch the rows: read one by one from memory by the 4 KT threads that add
+// them, 938 rows at kt 4 (60000 rows of A) took 13 us, longer than the streaming they run beside.
 template <int KT, bool PAIR = false>
-__device__ __forceinline__ void den_reduce(const float *__restrict__ parts, int nparts, float *__restrict__ den,
-					   float *__restrict__ s4)
+__device__ __forceinline__ void den_reduce(const float *__restrict__ parts, int nparts, float *den, float *__restrict__ s4,
+					   int room)
 {
 	static_assert(4 * KT <= NMFK_WG, "den_reduce: one thread per (column, lane of 4)");
-	const int t = threadIdx.x;
-	if (t < 4 * KT) {
-		const int c = t >> 2, j = t & 3;
-		float s = 0.0f;
-		int g = j;
-		// 8 loads in flight per step; the additions keep ascending g order.
-		for (; g + 28 < nparts; g += 32) {
-			float v[8];
-#pragma unroll
-			for (int u = 0; u < 8; u++)
-				v[u] = parts[(size_t)(g + 4 * u) * KT + c];
-			if constexpr (PAIR) {
-				s += pair8(v);
-			} else {
+	const int t = threadIdx.x, c = t >> 2, j = t & 3;
+	float *buf = s4 + 4 * KT;
+	const int chunk = room / KT / 32 * 32;   // whole groups of 8 rows per lane
+	float s = 0.0f;
+	for (int g0 = 0; g0 < nparts; g0 += chunk) {
+		const int rows = min(chunk, nparts - g0);
+		const float4 *src = reinterpret_cast<const float4 *>(parts + (size_t)g0 * KT);
+		if (g0 > 0)
+			__syncthreads();
+		for (int e = t; e < rows * (KT / 4); e += blockDim.x)
+			reinterpret_cast<float4 *>(buf)[e] = src[e];
+		__syncthreads();
+		if (t < 4 * KT) {
+			int g = j;
+			for (; g + 28 < rows; g += 32) {
+				float v[8];
 #pragma unroll
 				for (int u = 0; u < 8; u++)
-					s += v[u];
+					v[u] = buf[(g + 4 * u) * KT + c];
+				if constexpr (PAIR) {
+					s += pair8(v);
+				} else {
+#pragma unroll
+					for (int u = 0; u < 8; u++)
+						s += v[u];
+				}
 			}
+			for (; g < rows; g += 4)
+				s += buf[g * KT + c];
 		}
-		for (; g < nparts; g += 4)
-			s += parts[(size_t)g * KT + c];
-		s4[t] = s;
 	}
+	if (t < 4 * KT)
+		s4[t] = s;
 	__syncthreads();
 	if (t < KT)
 		den[t] = PAIR ? (s4[4 * t] + s4[4 * t + 1]) + (s4[4 * t + 2] + s4[4 * t + 3])
@@ -175,21 +185,22 @@ __host__ __device__ constexpr int fin_q(int kt)
 }
 static_assert(NMFK_FIN_ROWS * 4 == NMFK_WG, "finish block shape");
 
-// tile: NMFK_FIN_ROWS x (KT + 1) floats of LDS.  PAIR: NMFK_WG / KT groups of threads add
+// tid: the thread's index among the block's NMFK_WG threads; out: null where the block has no
+// rows.  tile: NMFK_FIN_ROWS x (KT + 1) floats of LDS.  PAIR: NMFK_WG / KT groups of threads add
 // consecutive rows each, then one thread per column adds the groups.
 template <int KT, bool PAIR = false>
-__device__ __forceinline__ void block_colsum_store(const float (&x)[fin_q(KT)], float *__restrict__ out,
+__device__ __forceinline__ void block_colsum_store(int tid, const float (&x)[fin_q(KT)], float *__restrict__ out,
 						   float *__restrict__ tile)
 {
 	constexpr int TPR = fin_tpr(KT), Q = fin_q(KT);
-	const int row = threadIdx.x / TPR, q = threadIdx.x % TPR;
+	const int row = tid / TPR, q = tid % TPR;
 #pragma unroll
 	for (int i = 0; i < Q; i++)
 		tile[row * (KT + 1) + q * Q + i] = x[i];
 	__syncthreads();
 	if constexpr (PAIR) {
 		constexpr int G = NMFK_WG / KT, RG = NMFK_FIN_ROWS / G;
-		const int c = threadIdx.x % KT, gr = threadIdx.x / KT;
+		const int c = tid % KT, gr = tid / KT;
 		float s = 0.0f;
 #pragma unroll
 		for (int r = 0; r < RG; r++)
@@ -197,20 +208,20 @@ __device__ __forceinline__ void block_colsum_store(const float (&x)[fin_q(KT)], 
 		__syncthreads();
 		tile[gr * (KT + 1) + c] = s;
 		__syncthreads();
-		if (threadIdx.x < KT) {
+		if (tid < KT && out != nullptr) {
 			float z[4] = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
 			for (int i = 0; i < G; i++)
-				z[i % 4] += tile[i * (KT + 1) + threadIdx.x];
-			out[threadIdx.x] = (z[0] + z[1]) + (z[2] + z[3]);
+				z[i % 4] += tile[i * (KT + 1) + tid];
+			out[tid] = (z[0] + z[1]) + (z[2] + z[3]);
 		}
 		return;
 	}
-	if (threadIdx.x < KT) {
+	if (tid < KT && out != nullptr) {
 		float s = 0.0f;
 		for (int r = 0; r < NMFK_FIN_ROWS; r++)
-			s += tile[r * (KT + 1) + threadIdx.x];
-		out[threadIdx.x] = s;
+			s += tile[r * (KT + 1) + tid];
+		out[tid] = s;
 	}
 }
 
@@ -245,11 +256,19 @@ struct half_args {
 	size_t ldu;
 	const float *A, *B;
 	int p, q, bchunk, nab;
-	float *part;
-	const float *colB;
-	int ncolB;
-	float *den;
-	int lb;   // VALU lane groups (see partial_valu_body)
+	float *part;   // null: the one split's sums are left in LDS for finish_rows
+	int S;         // splits of the q rows
+	int lb;        // VALU lane groups (see partial_valu_body)
+};
+
+// What turns a half-step's partial sums into the new A (see finish_rows).
+struct fin_args {
+	float *A;             // p x KT
+	float *colA;          // column sums of the new A per NMFK_FIN_ROWS rows
+	__bf16 *Ab;           // BF16 copy of the new A, or null
+	const float *colB;    // column-sum partials of B, ncolB rows, whose sum divides
+	float *den;           // that sum
+	int ncolB, k, clamp;
 };
 
 // LDS floats the partial bodies need (VALU: NW/2 wave slots of AP*KT*64; MFMA: NB-1 wave
@@ -263,11 +282,278 @@ __host__ __device__ constexpr int smem_mfma(int kt, int na, int nb)
 	return (nb > 1 ? nb - 1 : 1) * na * 4 * (kt / 16) * 4 * 64;
 }
 
-// Workgroup (bx, by) of a half-step's partial grid, bx in [0, nab], by in [0, S):
+typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+typedef __bf16 bf16x4 __attribute__((ext_vector_type(4)));
+
+// Finishing a half-step: A[a][c] = (A[a][c] * sum_s part[s][a][c]) / den[c], optional clamp,
+// then the column sums of the new A per block of 64 rows (the next half-step's denominators).
+// Kernel_mul_div order: multiply first, then divide (src/GPU_kernels.cu:2029-2033).  A block is
+// 64 rows of A and NMFK_WG threads; smem_fin floats of LDS hold its rows.
+__host__ __device__ constexpr int smem_fin(int kt)
+{
+	return NMFK_FIN_ROWS * (kt + 1);
+}
+
+// Q consecutive floats at a Q-aligned float offset (Q = KT/4: 1, 2, or a multiple of 4).
+template <int Q>
+__device__ __forceinline__ void ldq(const float *__restrict__ p, float (&v)[Q])
+{
+	if constexpr (Q % 4 == 0) {
+#pragma unroll
+		for (int i = 0; i < Q; i += 4) {
+			const float4 t = *reinterpret_cast<const float4 *>(p + i);
+			v[i] = t.x, v[i + 1] = t.y, v[i + 2] = t.z, v[i + 3] = t.w;
+		}
+	} else if constexpr (Q == 2) {
+		const float2 t = *reinterpret_cast<const float2 *>(p);
+		v[0] = t.x, v[1] = t.y;
+	} else {
+#pragma unroll
+		for (int i = 0; i < Q; i++)
+			v[i] = p[i];
+	}
+}
+
+template <int Q>
+__device__ __forceinline__ void stq(float *__restrict__ p, const float (&v)[Q])
+{
+	if constexpr (Q % 4 == 0) {
+#pragma unroll
+		for (int i = 0; i < Q; i += 4)
+			*reinterpret_cast<float4 *>(p + i) = make_float4(v[i], v[i + 1], v[i + 2], v[i + 3]);
+	} else if constexpr (Q == 2) {
+		*reinterpret_cast<float2 *>(p) = make_float2(v[0], v[1]);
+	} else {
+#pragma unroll
+		for (int i = 0; i < Q; i++)
+			p[i] = v[i];
+	}
+}
+
+// BF16 copy of a factor A (p x KT), row-major like A: thread (row a, quarter c0) writes its
+// KT / 4 consecutive values, 16 bytes at a time.
+template <int KT>
+__device__ __forceinline__ void store_shadow(int a, int c0, const float (&x)[KT / 4], __bf16 *__restrict__ Ab)
+{
+	constexpr int Q = KT / 4;
+	static_assert(Q % 8 == 0, "BF16 copies: kt a multiple of 32");
+#pragma unroll
+	for (int i = 0; i < Q; i += 8) {
+		bf16x8 v;
+#pragma unroll
+		for (int e = 0; e < 8; e++)
+			v[e] = (__bf16)x[i + e];
+		*reinterpret_cast<bf16x8 *>(Ab + (size_t)a * KT + c0 + i) = v;
+	}
+}
+
+template <int KT>
+__global__ __launch_bounds__(NMFK_WG) void k_shadow(const float *__restrict__ A, int p, __bf16 *__restrict__ Ab)
+{
+	constexpr int Q = KT / 4;
+	const int a = blockIdx.x * NMFK_FIN_ROWS + threadIdx.x / 4;
+	const int c0 = (threadIdx.x % 4) * Q;
+	if (a >= p)
+		return;
+	float x[Q];
+	ldq<Q>(A + (size_t)a * KT + c0, x);
+	store_shadow<KT>(a, c0, x, Ab);
+}
+
+// Block blk by the NMFK_WG threads tid.  LDS: its rows' sums are in smem already, row by row
+// (stride KT + 1), instead of S slices of part.  DEEP: more loads in flight, for a launch of
+// few workgroups that waits on latency; a batch's finish has workgroups enough, and would lose
+// occupancy to the registers.
+template <int KT, bool PAIR, bool LDS, bool DEEP>
+__device__ __forceinline__ void finish_block(int blk, int tid, const float *__restrict__ part, int S, float *A, int p, int k,
+					     const float *den, float *colA, int clamp, __bf16 *Ab, float *smem)
+{
+	constexpr int TPR = fin_tpr(KT), Q = fin_q(KT);
+	const int a = blk * NMFK_FIN_ROWS + tid / TPR;
+	const int c0 = (tid % TPR) * Q;
+	float x[Q];
+	if (a < p) {
+		// DEEP: the operands of the update first, so that their latency passes under that of the sums
+		float ar[Q], dn[Q], s[Q];
+		auto operands = [&]() {
+			ldq<Q>(A + (size_t)a * KT + c0, ar);
+#pragma unroll
+			for (int i = 0; i < Q; i++)
+				dn[i] = den[c0 + i];
+		};
+		constexpr bool EARLY = DEEP && KT <= 32;
+		if constexpr (EARLY)
+			operands();
+		if constexpr (LDS) {
+#pragma unroll
+			for (int i = 0; i < Q; i++)
+				s[i] = smem[(tid / TPR) * (KT + 1) + c0 + i];
+		} else {
+			const size_t pst = (size_t)p * KT;
+			const float *pa = part + (size_t)a * KT + c0;
+			ldq<Q>(pa, s);
+			int sp = 1;
+			// 8 splits' loads in flight per step (DEEP: 16 where a thread's share of a split is 4
+			// columns or fewer); the additions keep ascending split order, or that of pair8.
+			auto add = [&](auto count) {
+				constexpr int N = decltype(count)::value;
+				float v[N][Q];
+#pragma unroll
+				for (int u = 0; u < N; u++)
+					ldq<Q>(pa + (sp + u) * pst, v[u]);
+#pragma unroll
+				for (int u0 = 0; u0 < N; u0 += 8)
+#pragma unroll
+					for (int i = 0; i < Q; i++) {
+						const float w[8] = {v[u0][i],	  v[u0 + 1][i], v[u0 + 2][i], v[u0 + 3][i],
+								    v[u0 + 4][i], v[u0 + 5][i], v[u0 + 6][i], v[u0 + 7][i]};
+						if constexpr (PAIR) {
+							s[i] += pair8(w);
+						} else {
+#pragma unroll
+							for (int u = 0; u < 8; u++)
+								s[i] += w[u];
+						}
+					}
+				sp += N;
+			};
+			if constexpr (DEEP && Q <= 4)
+				while (sp + 16 <= S)
+					add(std::integral_constant<int, 16>{});
+			while (sp + 8 <= S)
+				add(std::integral_constant<int, 8>{});
+			// The last S - sp < 8 splits.  Up to KT 32 all their loads go out at once before the
+			// same ascending additions (c1 H finish, 30 splits: 4.02 -> 3.76 us); at KT 64 the
+			// registers that takes halve the occupancy and the W finish at 50000 x 2000 slows from
+			// 11.4 to 12.7 us, so there they stay one at a time.
+			if constexpr (KT <= 32) {
+				if (sp < S) {
+					float v[7][Q];
+#pragma unroll
+					for (int u = 0; u < 7; u++)
+						if (sp + u < S)
+							ldq<Q>(pa + (sp + u) * pst, v[u]);
+#pragma unroll
+					for (int u = 0; u < 7; u++)
+						if (sp + u < S)
+#pragma unroll
+							for (int i = 0; i < Q; i++)
+								s[i] += v[u][i];
+				}
+			} else {
+				for (; sp < S; sp++) {
+					float v[Q];
+					ldq<Q>(pa + sp * pst, v);
+#pragma unroll
+					for (int i = 0; i < Q; i++)
+						s[i] += v[i];
+				}
+			}
+		}
+		if constexpr (!EARLY)
+			operands();
+#pragma unroll
+		for (int i = 0; i < Q; i++) {
+			float v = 0.0f;
+			if (c0 + i < k) {
+				v = ar[i] * s[i];
+				v = v / dn[i];
+				if (clamp)
+					v = clamp_rmin(v);
+			}
+			x[i] = v;
+		}
+		stq<Q>(A + (size_t)a * KT + c0, x);
+		if constexpr (KT % 32 == 0) {
+			if (Ab != nullptr)
+				store_shadow<KT>(a, c0, x, Ab);
+		}
+	} else {
+#pragma unroll
+		for (int i = 0; i < Q; i++)
+			x[i] = 0.0f;
+	}
+	block_colsum_store<KT, PAIR>(tid, x, blk * NMFK_FIN_ROWS < p ? colA + (size_t)blk * KT : nullptr, smem);
+}
+
+// Single-job partial grids are 1-D: gx x S tiles, rounded up to a multiple of
+// the 8 XCDs.  The dispatcher places workgroup L on XCD L % 8; tile T = (L % 8) * per + L / 8
+// gives every XCD a contiguous run of tiles in by-major order, so the workgroups that share
+// a split of B (same by) mostly share one L2 instead of fetching it on every XCD.  Returns
+// false for the padding workgroups.
+__device__ __forceinline__ bool xcd_tile(int gx, int total, int &bx, int &by)
+{
+	const int per = (total + 7) >> 3;
+	const int L = blockIdx.x;
+	const int T = (L & 7) * per + (L >> 3);
+	if (T >= total)
+		return false;
+	by = T / gx;
+	bx = T - by * gx;
+	return true;
+}
+
+// The end of a half-step that takes one split: the workgroup finishes its own rows from the sums
+// the body left in LDS, instead of passing them to a second launch through memory.  That launch
+// took 3-5 us (11.5 us for W at 50000 x 2000, k = 64).
+// With several splits the sums of a row group come from several XCDs, and the second launch is
+// the cheaper way: the last of them to arrive at an atomic counter finishing the rows, with
+// stores and loads past the XCDs' caches, took 4 us more per iteration at 20000 x 1000, k = 16
+// than the launch, and 2.5 us more at 7013 x 333.
+// NT threads; tile_rows x (KT + 1) floats of smem hold the sums, and den_reduce's come after them.
+__host__ __device__ constexpr int smem_den(int kt)
+{
+	return (4 + 32) * kt;
+}
+__host__ __device__ constexpr int max2(int a, int b)
+{
+	return a > b ? a : b;
+}
+__host__ __device__ constexpr int tile_rows(int rows)
+{
+	return rows > NMFK_FIN_ROWS ? rows : NMFK_FIN_ROWS;
+}
+__host__ __device__ constexpr int smem_finish(int kt, int rows)
+{
+	return (tile_rows(rows) * (kt + 1) + 3) / 4 * 4 + smem_den(kt) + kt;
+}
+
+template <int KT, bool PAIR, int NT>
+__device__ __forceinline__ void finish_rows(int bx, int rows, const half_args &h, const fin_args &f, float *smem)
+{
+	constexpr int PP = NT / NMFK_WG;   // blocks at a time
+	float *s4 = smem + (tile_rows(rows) * (KT + 1) + 3) / 4 * 4, *den = s4 + smem_den(KT);
+	den_reduce<KT, PAIR>(f.colB, f.ncolB, den, s4, 32 * KT);
+	__syncthreads();
+	if (bx == 0 && threadIdx.x < KT)
+		f.den[threadIdx.x] = den[threadIdx.x];
+	const int sub = threadIdx.x / NMFK_WG, tid = threadIdx.x % NMFK_WG;
+	const int b0 = bx * rows / NMFK_FIN_ROWS;
+	for (int b = sub; b < tile_rows(rows) / NMFK_FIN_ROWS; b += PP)
+		finish_block<KT, PAIR, true, true>(b0 + b, tid, nullptr, 1, f.A, h.p, f.k, den, f.colA, f.clamp, f.Ab,
+					     smem + b * NMFK_FIN_ROWS * (KT + 1));
+}
+
+// A half-step's grid has nab workgroups, which finish their rows themselves, where there is one
+// split.  Where there are more it has (nab + 1) x S, and the first workgroup of column nab reduces
+// the other factor's column-sum partials into the denominators the finish divides by, off the
+// critical path of the streaming ones; the rest of that column return at once.  True for a
+// workgroup with rows (bx, by) to stream.
+template <int KT, bool PAIR, int ROOM>
+__device__ __forceinline__ bool half_tile(const half_args &h, const fin_args &f, float *smem, int &bx, int &by)
+{
+	const int gx = h.part ? h.nab + 1 : h.nab;
+	if (!xcd_tile(gx, gx * h.S, bx, by))
+		return false;
+	if (bx < h.nab)
+		return true;
+	if (by == 0 && f.den != nullptr)
+		den_reduce<KT, PAIR>(f.colB, f.ncolB, f.den, smem, ROOM - 4 * KT);
+	return false;
+}
+
+// Workgroup (bx, by) of a half-step's grid, bx in [0, nab), by in [0, S):
 // part[by][a][c] = sum_{b in split by} B[b][c] * U[b][a] / (A[a] . B[b]).
-// Column bx == nab is the denominator column: its first workgroup reduces the other
-// factor's column-sum partials into the denominators the finish kernel divides by, off
-// the critical path of the streaming workgroups; the rest return at once.
 // A wave's 64 lanes are LB groups of 64 / LB: lane (la, lb) owns rows a of A
 // (AP per lane) and takes every LB-th of the wave's rows of U, so that a factor with few
 // rows (p <= 64 AP / LB) still keeps every lane busy.  The groups' sums are added by a
@@ -282,11 +568,6 @@ __device__ __forceinline__ void partial_valu_body(int bx, int by, const half_arg
 	const float *__restrict__ A = h.A;
 	const float *__restrict__ B = h.B;
 	const int p = h.p, q = h.q, bchunk = h.bchunk;
-	if (bx == h.nab) {
-		if (by == 0)
-			den_reduce<KT>(h.colB, h.ncolB, h.den, smem);
-		return;
-	}
 	const int lane = threadIdx.x & 63;
 	const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
 	const int la = lane % LA, lg = lane / LA;
@@ -395,46 +676,39 @@ __device__ __forceinline__ void partial_valu_body(int bx, int by, const half_arg
 		__syncthreads();
 	}
 	if (wave == 0 && lg == 0) {
-		float *dst = h.part + ((size_t)by * p + a0) * KT;
+		float *dst = h.part ? h.part + ((size_t)by * p + a0) * KT : nullptr;
 #pragma unroll
 		for (int r = 0; r < AP; r++)
 			if (r < avail) {
+				if (dst == nullptr) {
 #pragma unroll
-				for (int c = 0; c < KT; c += 4)
-					if constexpr (KT % 4 == 0)
+					for (int c = 0; c < KT; c++)
+						red[(la * AP + r) * (KT + 1) + c] = acc[r][c];
+				} else {
+#pragma unroll
+					for (int c = 0; c < KT; c += 4)
 						*reinterpret_cast<float4 *>(dst + r * KT + c) =
 							make_float4(acc[r][c], acc[r][c + 1], acc[r][c + 2], acc[r][c + 3]);
+				}
 			}
 	}
-}
-
-// Single-job partial grids are 1-D: the (nab + 1) x S tiles, rounded up to a multiple of
-// the 8 XCDs.  The dispatcher places workgroup L on XCD L % 8; tile T = (L % 8) * per + L / 8
-// gives every XCD a contiguous run of tiles in by-major order, so the workgroups that share
-// a split of B (same by) mostly share one L2 instead of fetching it on every XCD.  Returns
-// false for the padding workgroups.
-__device__ __forceinline__ bool xcd_tile(int gx, int total, int &bx, int &by)
-{
-	const int per = (total + 7) >> 3;
-	const int L = blockIdx.x;
-	const int T = (L & 7) * per + (L >> 3);
-	if (T >= total)
-		return false;
-	by = T / gx;
-	bx = T - by * gx;
-	return true;
+	if (h.part == nullptr)
+		__syncthreads();
 }
 
 template <int KT, int AP, int NW, int LB>
-__global__ __launch_bounds__(64 * NW) void k_partial(half_args h, const nmfk_state *__restrict__ st, int S)
+__global__ __launch_bounds__(64 * NW) void k_partial(half_args h, fin_args f, const nmfk_state *__restrict__ st)
 {
-	__shared__ float smem[smem_valu(KT, AP, NW)];
+	constexpr int LDS = max2(smem_valu(KT, AP, NW), smem_finish(KT, 64 / LB * AP));
+	__shared__ __align__(16) float smem[LDS];
 	if (st != nullptr && st->converged)
 		return;
 	int bx, by;
-	if (!xcd_tile(h.nab + 1, (h.nab + 1) * S, bx, by))
+	if (!half_tile<KT, false, LDS>(h, f, smem, bx, by))
 		return;
 	partial_valu_body<KT, AP, NW, LB>(bx, by, h, smem);
+	if (h.part == nullptr)
+		finish_rows<KT, false, 64 * NW>(bx, 64 / LB * AP, h, f, smem);
 }
 
 // --------------------------------------------------------------------------------------
@@ -458,7 +732,6 @@ __global__ __launch_bounds__(64 * NW) void k_partial(half_args h, const nmfk_sta
 // per-lane address arithmetic.
 // --------------------------------------------------------------------------------------
 
-typedef float floatx4 __attribute__((ext_vector_type(4)));
 typedef int intx4 __attribute__((ext_vector_type(4)));
 typedef int intx2 __attribute__((ext_vector_type(2)));
 
@@ -512,7 +785,8 @@ __device__ __forceinline__ float4 loadq(const float *p)
 }
 
 // Sums of a wave's 64 rows a (acc[t][h][r] = partial for a = a0 + 4*(4g + r) + t, c = 16h + j):
-// the NB wave groups' are added through LDS in a fixed order and written to split by of part.
+// the NB wave groups' are added through LDS in a fixed order and written to split by of part, or
+// left in LDS where part is null.
 template <int KT, int NA, int NB>
 __device__ __forceinline__ void mfma_store(floatx4 (&acc)[4][KT / 16], const half_args &ha, int by, int a0, bool idle,
 					   float *__restrict__ smem)
@@ -521,6 +795,7 @@ __device__ __forceinline__ void mfma_store(floatx4 (&acc)[4][KT / 16], const hal
 	const int lane = threadIdx.x & 63, j = lane & 15, g = lane >> 4;
 	const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
 	const int wa = wave % NA, wb = wave / NA, p = ha.p;
+	const bool owner = wb == 0 && !idle;
 	if constexpr (NB > 1) {
 		float (*red)[NA][4][H][4][64] = reinterpret_cast<float (*)[NA][4][H][4][64]>(smem);
 		if (wb > 0) {
@@ -533,19 +808,33 @@ __device__ __forceinline__ void mfma_store(floatx4 (&acc)[4][KT / 16], const hal
 						red[wb - 1][wa][t][h][r][lane] = acc[t][h][r];
 		}
 		__syncthreads();
-		if (wb > 0 || idle)
-			return;
+		if (owner) {
 #pragma unroll
-		for (int w = 0; w < NB - 1; w++)
+			for (int w = 0; w < NB - 1; w++)
+#pragma unroll
+				for (int t = 0; t < 4; t++)
+#pragma unroll
+					for (int h = 0; h < H; h++)
+#pragma unroll
+						for (int r = 0; r < 4; r++)
+							acc[t][h][r] += red[w][wa][t][h][r][lane];
+		}
+	}
+	if (ha.part == nullptr) {
+		__syncthreads();   // the wave groups' sums have been read
+		if (owner) {
 #pragma unroll
 			for (int t = 0; t < 4; t++)
 #pragma unroll
-				for (int h = 0; h < H; h++)
+				for (int r = 0; r < 4; r++)
 #pragma unroll
-					for (int r = 0; r < 4; r++)
-						acc[t][h][r] += red[w][wa][t][h][r][lane];
+					for (int h = 0; h < H; h++)
+						smem[(wa * 64 + 4 * (4 * g + r) + t) * (KT + 1) + 16 * h + j] = acc[t][h][r];
+		}
+		__syncthreads();
+		return;
 	}
-	if (idle)
+	if (!owner)
 		return;
 	float *dst = ha.part + (size_t)by * p * KT;
 #pragma unroll
@@ -593,12 +882,6 @@ __device__ __forceinline__ void partial_mfma_body(int bx, int by, const half_arg
 	const float *__restrict__ A = ha.A;
 	const float *__restrict__ B = ha.B;
 	const int p = ha.p, q = ha.q, bchunk = ha.bchunk;
-	// Denominator column (see partial_valu_body).
-	if (bx == ha.nab) {
-		if (by == 0)
-			den_reduce<KT>(ha.colB, ha.ncolB, ha.den, smem);
-		return;
-	}
 
 	const int lane = threadIdx.x & 63;
 	const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -845,22 +1128,35 @@ __device__ __forceinline__ void partial_mfma_body(int bx, int by, const half_arg
 						red[wb - 1][wa][t][cg][lane] = o[t][cg];
 			}
 			__syncthreads();
-			if (wb > 0 || idle)
-				return;
+			if (wb == 0 && !idle) {
 #pragma unroll
-			for (int w = 0; w < NB - 1; w++)
+				for (int w = 0; w < NB - 1; w++)
+#pragma unroll
+					for (int t = 0; t < 4; t++)
+#pragma unroll
+						for (int cg = 0; cg < CW; cg++)
+							o[t][cg] += red[w][wa][t][cg][lane];
+			}
+		}
+		const int al = 16 * (j >> 2) + 4 * g;   // row of o[0], from the wave's first
+		if (ha.part == nullptr) {
+			__syncthreads();
+			if (wb == 0 && !idle) {
 #pragma unroll
 				for (int t = 0; t < 4; t++)
 #pragma unroll
 					for (int cg = 0; cg < CW; cg++)
-						o[t][cg] += red[w][wa][t][cg][lane];
+						smem[(wa * 64 + al + t) * (KT + 1) + c2 + cg] = o[t][cg];
+			}
+			__syncthreads();
+			return;
 		}
-		if (idle)
+		if (wb > 0 || idle)
 			return;
 		float *dst = ha.part + (size_t)by * p * KT;
 #pragma unroll
 		for (int t = 0; t < 4; t++) {
-			const int a = a0 + 16 * (j >> 2) + 4 * g + t;
+			const int a = a0 + al + t;
 			if (a < p)
 #pragma unroll
 				for (int cg = 0; cg < CW; cg++)
@@ -872,16 +1168,19 @@ __device__ __forceinline__ void partial_mfma_body(int bx, int by, const half_arg
 }
 
 template <int KT, int NA, int NB, int KE = KT>
-__global__ __launch_bounds__(64 * NA * NB, (KT == 32 ? 3 : 1)) void k_partial_mfma(half_args h, const nmfk_state *__restrict__ st,
-										       int S)
+__global__ __launch_bounds__(64 * NA * NB, (KT == 32 ? 3 : 1)) void k_partial_mfma(half_args h, fin_args f,
+										       const nmfk_state *__restrict__ st)
 {
-	__shared__ float smem[smem_mfma(KT, NA, NB)];
+	constexpr int LDS = max2(smem_mfma(KT, NA, NB), smem_finish(KT, 64 * NA));
+	__shared__ __align__(16) float smem[LDS];
 	if (st != nullptr && st->converged)
 		return;
 	int bx, by;
-	if (!xcd_tile(h.nab + 1, (h.nab + 1) * S, bx, by))
+	if (!half_tile<KT, false, LDS>(h, f, smem, bx, by))
 		return;
 	partial_mfma_body<KT, NA, NB, KE>(bx, by, h, smem);
+	if (h.part == nullptr)
+		finish_rows<KT, false, 64 * NA * NB>(bx, 64 * NA, h, f, smem);
 }
 
 // --------------------------------------------------------------------------------------
@@ -900,8 +1199,6 @@ __global__ __launch_bounds__(64 * NA * NB, (KT == 32 ? 3 : 1)) void k_partial_mf
 // factor, staged per block through LDS (see the body).
 // --------------------------------------------------------------------------------------
 
-typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
-typedef __bf16 bf16x4 __attribute__((ext_vector_type(4)));
 
 // LDS floats of the BF16 body: the wave groups' sums (smem_mfma), and before them each
 // wave's 32-row B slot (32 x (kt + 4) BF16).
@@ -934,11 +1231,6 @@ __device__ __forceinline__ void partial_bf16_body(int bx, int by, const half_arg
 	const float *__restrict__ A = ha.A;
 	const __bf16 *__restrict__ Bb = bb16.Bb;
 	const int p = ha.p, q = ha.q, bchunk = ha.bchunk;
-	if (bx == ha.nab) {
-		if (by == 0)
-			den_reduce<KT>(ha.colB, ha.ncolB, ha.den, smem);
-		return;
-	}
 	const int lane = threadIdx.x & 63;
 	const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
 	const int wa = wave % NA, wb = wave / NA;
@@ -1122,16 +1414,19 @@ __device__ __forceinline__ void partial_bf16_body(int bx, int by, const half_arg
 }
 
 template <int KT, int NA, int NB>
-__global__ __launch_bounds__(64 * NA * NB) void k_partial_bf16(half_args h, bf16_args b, const nmfk_state *__restrict__ st,
-							     int S)
+__global__ __launch_bounds__(64 * NA * NB) void k_partial_bf16(half_args h, bf16_args b, fin_args f,
+							     const nmfk_state *__restrict__ st)
 {
-	__shared__ __align__(16) float smem[smem_bf16(KT, NA, NB)];
+	constexpr int LDS = max2(smem_bf16(KT, NA, NB), smem_finish(KT, 64 * NA));
+	__shared__ __align__(16) float smem[LDS];
 	if (st != nullptr && st->converged)
 		return;
 	int bx, by;
-	if (!xcd_tile(h.nab + 1, (h.nab + 1) * S, bx, by))
+	if (!half_tile<KT, false, LDS>(h, f, smem, bx, by))
 		return;
 	partial_bf16_body<KT, NA, NB>(bx, by, h, b, smem);
+	if (h.part == nullptr)
+		finish_rows<KT, false, 64 * NA * NB>(bx, 64 * NA, h, f, smem);
 }
 
 // --------------------------------------------------------------------------------------
@@ -1273,11 +1568,6 @@ __device__ __forceinline__ void partial_split_body(int bx, int by, const half_ar
 	const float *__restrict__ A = ha.A;
 	const float *__restrict__ B = ha.B;
 	const int p = ha.p, q = ha.q, bchunk = ha.bchunk;
-	if (bx == ha.nab) {
-		if (by == 0)
-			den_reduce<KT, true>(ha.colB, ha.ncolB, ha.den, smem);
-		return;
-	}
 	const int lane = threadIdx.x & 63;
 	const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
 	const int wa = wave % NA, wb = wave / NA;
@@ -1494,196 +1784,31 @@ __device__ __forceinline__ void partial_split_body(int bx, int by, const half_ar
 }
 
 template <int KT, int NA, int NB>
-__global__ __launch_bounds__(64 * NA * NB, (KT <= 32 ? 3 : 2)) void k_partial_split(half_args h, const nmfk_state *__restrict__ st, int S)
+__global__ __launch_bounds__(64 * NA * NB, (KT <= 32 ? 3 : 2)) void k_partial_split(half_args h, fin_args f, const nmfk_state *__restrict__ st)
 {
-	__shared__ __align__(16) float smem[smem_split(KT, NA, NB)];
+	constexpr int LDS = max2(smem_split(KT, NA, NB), smem_finish(KT, 64 * NA));
+	__shared__ __align__(16) float smem[LDS];
 	if (st != nullptr && st->converged)
 		return;
 	int bx, by;
-	if (!xcd_tile(h.nab + 1, (h.nab + 1) * S, bx, by))
+	if (!half_tile<KT, true, LDS>(h, f, smem, bx, by))
 		return;
 	partial_split_body<KT, NA, NB>(bx, by, h, smem);
+	if (h.part == nullptr)
+		finish_rows<KT, true, 64 * NA * NB>(bx, 64 * NA, h, f, smem);
 }
 
-// A[a][c] = (A[a][c] * sum_s part[s][a][c]) / den[c], optional clamp, then the column sums
-// of the new A per block of 64 rows (the next half-step's denominators).  Kernel_mul_div
-// order: multiply first, then divide (src/GPU_kernels.cu:2029-2033).  Block bx covers rows
-// [64 bx, 64 bx + 64); smem holds NMFK_FIN_ROWS x (KT + 1) floats.
-__host__ __device__ constexpr int smem_fin(int kt)
-{
-	return NMFK_FIN_ROWS * (kt + 1);
-}
-
-// Q consecutive floats at a Q-aligned float offset (Q = KT/4: 1, 2, or a multiple of 4).
-template <int Q>
-__device__ __forceinline__ void ldq(const float *__restrict__ p, float (&v)[Q])
-{
-	if constexpr (Q % 4 == 0) {
-#pragma unroll
-		for (int i = 0; i < Q; i += 4) {
-			const float4 t = *reinterpret_cast<const float4 *>(p + i);
-			v[i] = t.x, v[i + 1] = t.y, v[i + 2] = t.z, v[i + 3] = t.w;
-		}
-	} else if constexpr (Q == 2) {
-		const float2 t = *reinterpret_cast<const float2 *>(p);
-		v[0] = t.x, v[1] = t.y;
-	} else {
-#pragma unroll
-		for (int i = 0; i < Q; i++)
-			v[i] = p[i];
-	}
-}
-
-template <int Q>
-__device__ __forceinline__ void stq(float *__restrict__ p, const float (&v)[Q])
-{
-	if constexpr (Q % 4 == 0) {
-#pragma unroll
-		for (int i = 0; i < Q; i += 4)
-			*reinterpret_cast<float4 *>(p + i) = make_float4(v[i], v[i + 1], v[i + 2], v[i + 3]);
-	} else if constexpr (Q == 2) {
-		*reinterpret_cast<float2 *>(p) = make_float2(v[0], v[1]);
-	} else {
-#pragma unroll
-		for (int i = 0; i < Q; i++)
-			p[i] = v[i];
-	}
-}
-
-// The BF16 copy the finish kernel keeps of the factor it updates (null: none).
-struct shadow_args {
-	__bf16 *Ab;
-};
-
-// BF16 copy of a factor A (p x KT), row-major like A: thread (row a, quarter c0) writes its
-// KT / 4 consecutive values, 16 bytes at a time.
-template <int KT>
-__device__ __forceinline__ void store_shadow(int a, int c0, const float (&x)[KT / 4], __bf16 *__restrict__ Ab)
-{
-	constexpr int Q = KT / 4;
-	static_assert(Q % 8 == 0, "BF16 copies: kt a multiple of 32");
-#pragma unroll
-	for (int i = 0; i < Q; i += 8) {
-		bf16x8 v;
-#pragma unroll
-		for (int e = 0; e < 8; e++)
-			v[e] = (__bf16)x[i + e];
-		*reinterpret_cast<bf16x8 *>(Ab + (size_t)a * KT + c0 + i) = v;
-	}
-}
-
-template <int KT>
-__global__ __launch_bounds__(NMFK_WG) void k_shadow(const float *__restrict__ A, int p, __bf16 *__restrict__ Ab)
-{
-	constexpr int Q = KT / 4;
-	const int a = blockIdx.x * NMFK_FIN_ROWS + threadIdx.x / 4;
-	const int c0 = (threadIdx.x % 4) * Q;
-	if (a >= p)
-		return;
-	float x[Q];
-	ldq<Q>(A + (size_t)a * KT + c0, x);
-	store_shadow<KT>(a, c0, x, Ab);
-}
-
-template <int KT, bool PAIR = false>
-__device__ __forceinline__ void finish_body(int bx, const float *__restrict__ part, int S, float *__restrict__ A,
-					    int p, int k, const float *__restrict__ den, float *__restrict__ colA,
-					    int clamp, float *__restrict__ smem, const shadow_args &sh = shadow_args{})
-{
-	constexpr int TPR = fin_tpr(KT), Q = fin_q(KT);
-	const int a = bx * NMFK_FIN_ROWS + threadIdx.x / TPR;
-	const int c0 = (threadIdx.x % TPR) * Q;
-	float x[Q];
-	if (a < p) {
-		const size_t pst = (size_t)p * KT;
-		const float *pa = part + (size_t)a * KT + c0;
-		float s[Q];
-		ldq<Q>(pa, s);
-		int sp = 1;
-		// 8 splits' loads in flight per step; the additions keep ascending split order.
-		for (; sp + 8 <= S; sp += 8) {
-			float v[8][Q];
-#pragma unroll
-			for (int u = 0; u < 8; u++)
-				ldq<Q>(pa + (sp + u) * pst, v[u]);
-			if constexpr (PAIR) {
-#pragma unroll
-				for (int i = 0; i < Q; i++) {
-					const float w[8] = {v[0][i], v[1][i], v[2][i], v[3][i], v[4][i], v[5][i], v[6][i], v[7][i]};
-					s[i] += pair8(w);
-				}
-				continue;
-			}
-#pragma unroll
-			for (int u = 0; u < 8; u++)
-#pragma unroll
-				for (int i = 0; i < Q; i++)
-					s[i] += v[u][i];
-		}
-		// The last S - sp < 8 splits.  Up to KT 32 all their loads go out at once before the
-		// same ascending additions (c1 H finish, 30 splits: 4.02 -> 3.76 us); at KT 64 the
-		// registers that takes halve the occupancy and the W finish at 50000 x 2000 slows from
-		// 11.4 to 12.7 us, so there they stay one at a time.
-		if constexpr (KT <= 32) {
-			if (sp < S) {
-				float v[7][Q];
-#pragma unroll
-				for (int u = 0; u < 7; u++)
-					if (sp + u < S)
-						ldq<Q>(pa + (sp + u) * pst, v[u]);
-#pragma unroll
-				for (int u = 0; u < 7; u++)
-					if (sp + u < S)
-#pragma unroll
-						for (int i = 0; i < Q; i++)
-							s[i] += v[u][i];
-			}
-		} else {
-			for (; sp < S; sp++) {
-				float v[Q];
-				ldq<Q>(pa + sp * pst, v);
-#pragma unroll
-				for (int i = 0; i < Q; i++)
-					s[i] += v[i];
-			}
-		}
-		float *Ar = A + (size_t)a * KT + c0;
-		float ar[Q];
-		ldq<Q>(Ar, ar);
-#pragma unroll
-		for (int i = 0; i < Q; i++) {
-			float v = 0.0f;
-			if (c0 + i < k) {
-				v = ar[i] * s[i];
-				v = v / den[c0 + i];
-				if (clamp)
-					v = clamp_rmin(v);
-			}
-			x[i] = v;
-		}
-		stq<Q>(Ar, x);
-		if constexpr (KT % 32 == 0) {
-			if (sh.Ab != nullptr)
-				store_shadow<KT>(a, c0, x, sh.Ab);
-		}
-	} else {
-#pragma unroll
-		for (int i = 0; i < Q; i++)
-			x[i] = 0.0f;
-	}
-	block_colsum_store<KT, PAIR>(x, colA + (size_t)bx * KT, smem);
-}
-
+// A finish by itself, where the partial sums of several launches make up a half-step.
 template <int KT, bool PAIR>
 __global__ __launch_bounds__(NMFK_WG) void k_finish(const float *__restrict__ part, int S, float *__restrict__ A,
 						    int p, int k, const float *__restrict__ den,
 						    float *__restrict__ colA, int clamp,
-						    const nmfk_state *__restrict__ st, shadow_args sh)
+						    const nmfk_state *__restrict__ st, __bf16 *__restrict__ Ab)
 {
 	__shared__ float smem[smem_fin(KT)];
 	if (st != nullptr && st->converged)
 		return;
-	finish_body<KT, PAIR>(blockIdx.x, part, S, A, p, k, den, colA, clamp, smem, sh);
+	finish_block<KT, PAIR, false, true>(blockIdx.x, threadIdx.x, part, S, A, p, k, den, colA, clamp, Ab, smem);
 }
 
 template <int KT, bool PAIR>
@@ -1698,14 +1823,15 @@ __global__ __launch_bounds__(NMFK_WG) void k_colsum_parts(const float *__restric
 #pragma unroll
 	for (int i = 0; i < Q; i++)
 		x[i] = (a < p) ? A[(size_t)a * KT + c0 + i] : 0.0f;
-	block_colsum_store<KT, PAIR>(x, colA + (size_t)blockIdx.x * KT, smem);
+	block_colsum_store<KT, PAIR>(threadIdx.x, x, colA + (size_t)blockIdx.x * KT, smem);
 }
 
 template <int KT>
 __global__ __launch_bounds__(NMFK_WG) void k_den(const float *__restrict__ parts, int nparts, float *__restrict__ den)
 {
-	__shared__ float smem[4 * KT];
-	den_reduce<KT>(parts, nparts, den, smem);
+	constexpr int LDS = 4 * KT + 8192;
+	__shared__ __align__(16) float smem[LDS];
+	den_reduce<KT>(parts, nparts, den, smem, LDS - 4 * KT);
 }
 
 // --------------------------------------------------------------------------------------
@@ -2153,11 +2279,11 @@ __global__ __launch_bounds__(64 * NMFK_FFIN_WAVES) void k_fused_finish(const flo
 									 const nmfk_state *__restrict__ st)
 {
 	__shared__ float red[NMFK_FFIN_WAVES][64];
-	__shared__ float s4[4 * KT];
+	__shared__ __align__(16) float s4[4 * KT + 4096];
 	__shared__ float den[KT];
 	if (st != nullptr && st->converged)
 		return;
-	den_reduce<KT>(colW, G, den, s4);
+	den_reduce<KT>(colW, G, den, s4, 4096);
 	const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
 	const size_t tot = (size_t)m * KT;
 	const size_t e = (size_t)blockIdx.x * 64 + lane;
@@ -2418,11 +2544,24 @@ __device__ __forceinline__ half_args batch_half(const nmfk_bjob &J, int half)
 	h.bchunk = pl.bchunk;
 	h.nab = pl.nab;
 	h.part = J.part;
-	h.colB = hh ? J.colW : J.colH;
-	h.ncolB = hh ? J.ncolW : J.ncolH;
-	h.den = hh ? J.denW : J.denH;
+	h.S = pl.S;
 	h.lb = (int)pl.lb;
 	return h;
+}
+
+__device__ __forceinline__ fin_args batch_fin(const nmfk_bjob &J, int half, int clamp)
+{
+	fin_args f;
+	const bool hh = half == 0;
+	f.A = hh ? J.H : J.W;
+	f.colA = hh ? J.colH : J.colW;
+	f.Ab = nullptr;
+	f.colB = hh ? J.colW : J.colH;
+	f.ncolB = hh ? J.ncolW : J.ncolH;
+	f.den = hh ? J.denW : J.denH;
+	f.k = J.k;
+	f.clamp = hh ? 0 : clamp;
+	return f;
 }
 
 // VALU body of a batched half-step with lane groups (2, 4 or 8, from its plan).
@@ -2486,6 +2625,19 @@ __global__ __launch_bounds__(NMFK_WG, (CLS == 0 || CLS == 2 || CLS == 4 ? 4 : CL
 		if (!fits || !J.live || J.st->converged)
 			continue;
 		const half_args h = batch_half(J, half);
+		__builtin_assume(h.part != nullptr);   // batched half-steps are finished in k_batch_finish
+		if (tl.bx == (uint32_t)h.nab) {   // the denominators
+			const fin_args f = batch_fin(J, half, 0);
+			constexpr int LDS = smem_batch_partial<CLS>();
+			if constexpr (CLS > 1)
+				den_reduce<batch_cls_kt(CLS), (CLS >= 6)>(f.colB, f.ncolB, f.den, smem, LDS - 4 * batch_cls_kt(CLS));
+			else if (J.kt == 4)
+				den_reduce<4>(f.colB, f.ncolB, f.den, smem, LDS - 16);
+			else
+				den_reduce<8>(f.colB, f.ncolB, f.den, smem, LDS - 32);
+			__syncthreads();
+			continue;
+		}
 		if constexpr (CLS == 0) {
 			if (J.kt == 4)
 				partial_valu_body<4, 4, 4, 1>(tl.bx, tl.by, h, smem);
@@ -2527,33 +2679,12 @@ __global__ __launch_bounds__(NMFK_WG) void k_batch_finish(const nmfk_bjob *__res
 		const nmfk_bjob &J = jobs[tl.job];
 		if (!J.live || J.st->converged)
 			continue;
-		const bool hh = half == 0;
-		const float *part = J.part;
-		const int S = hh ? J.planH.S : J.planW.S;
-		float *A = hh ? J.H : J.W;
-		const int p = hh ? J.m : J.n;
-		const float *den = hh ? J.denW : J.denH;
-		float *colA = hh ? J.colH : J.colW;
-		const int cl = hh ? 0 : clamp;
-		switch (J.kt) {
-		case 4:
-			finish_body<4>(tl.bx, part, S, A, p, J.k, den, colA, cl, smem);
-			break;
-		case 8:
-			finish_body<8>(tl.bx, part, S, A, p, J.k, den, colA, cl, smem);
-			break;
-		case 16:
-			if (J.split)
-				finish_body<16, true>(tl.bx, part, S, A, p, J.k, den, colA, cl, smem);
-			else
-				finish_body<16>(tl.bx, part, S, A, p, J.k, den, colA, cl, smem);
-			break;
-		case 32:
-			if (J.split)
-				finish_body<32, true>(tl.bx, part, S, A, p, J.k, den, colA, cl, smem);
-			else
-				finish_body<32>(tl.bx, part, S, A, p, J.k, den, colA, cl, smem);
-			break;
+		const fin_args f = batch_fin(J, half, clamp);
+		const int S = half == 0 ? J.planH.S : J.planW.S, p = half == 0 ? J.m : J.n, tid = threadIdx.x;
+		switch (J.kt + J.split) {
+#define X(K, PAIR)                                                                                     	case K + PAIR:                                                                                 		finish_block<K, PAIR, false, false>(tl.bx, tid, J.part, S, f.A, p, f.k, f.den, f.colA, f.clamp, nullptr, smem); 		break;
+			X(4, false) X(8, false) X(16, false) X(16, true) X(32, false) X(32, true)
+#undef X
 		}
 		__syncthreads();
 	}
@@ -3157,62 +3288,76 @@ extern "C" void nmfk_plan_half(uint32_t p, uint32_t q, uint32_t kt, nmfk_hplan *
 	nmfk_plan_half_path(p, q, kt, NMFK_PATH_AUTO, pl);
 }
 
-// (nab + 1) x S tiles (+ the denominator column) as a 1-D grid padded to a multiple of 8
-// (see xcd_tile).
-static inline dim3 xcd_grid(const nmfk_hplan *pl)
+// Kernel arguments and grid (padded to a multiple of 8, see xcd_tile) of a half-step; fin may be
+// null (partial sums only).  Workgroups that finish <rows> rows themselves take whole blocks of
+// rows, or all of them.
+static bool kernel_args(const nmfk_half *g, const nmfk_hplan *pl, const nmfk_fin *fin, uint32_t rows, half_args *h, fin_args *f,
+			dim3 *grid)
 {
-	const unsigned total = (pl->nab + 1) * pl->S;
-	return dim3((total + 7u) & ~7u);
+	const bool own = fin && pl->S == 1;
+	*h = half_args{g->U, g->ldu, g->A, g->B, (int)g->p, (int)g->q, (int)pl->bchunk, (int)pl->nab, own ? nullptr : g->part,
+		       (int)pl->S, (int)pl->lb};
+	*f = fin_args{};
+	if (fin)
+		*f = fin_args{fin->A, fin->colA, (__bf16 *)fin->Ab, fin->colB, fin->den, (int)fin->ncolB, (int)fin->k, fin->clamp};
+	*grid = dim3(((own ? pl->nab : pl->nab + 1) * pl->S + 7u) & ~7u);
+	return g->part != nullptr && !(own && rows % NMFK_FIN_ROWS != 0 && pl->nab != 1);
 }
 
 template <int KT, int AP>
-static int launch_partial_t(const float *U, size_t ldu, const float *A, const float *B, uint32_t p,
-			    uint32_t q, const nmfk_hplan *pl, float *part, const float *colB, uint32_t ncolB,
-			    float *den, const nmfk_state *st, hipStream_t stream)
+static int launch_half_valu(const nmfk_half *g, const nmfk_hplan *pl, const nmfk_fin *fin, const nmfk_state *st,
+			    hipStream_t stream)
 {
-	const dim3 grid = xcd_grid(pl);
-	if (pl->nw != 4)
+	half_args h;
+	fin_args f;
+	dim3 grid;
+	if (pl->nw != 4 || pl->ap != AP || pl->lb < 1 || !kernel_args(g, pl, fin, 64u / pl->lb * AP, &h, &f, &grid))
 		return (int)hipErrorInvalidValue;
-	const half_args h = {U, ldu, A, B, (int)p, (int)q, (int)pl->bchunk, (int)pl->nab, part, colB, (int)ncolB, den,
-			     (int)pl->lb};
 	switch (pl->lb) {
-	case 1:
-		hipLaunchKernelGGL((k_partial<KT, AP, 4, 1>), grid, dim3(256), 0, stream, h, st, (int)pl->S);
+#define X(LB)                                                                                          \
+	case LB:                                                                                       \
+		hipLaunchKernelGGL((k_partial<KT, AP, 4, LB>), grid, dim3(256), 0, stream, h, f, st);       \
 		break;
-	case 2:
-		hipLaunchKernelGGL((k_partial<KT, AP, 4, 2>), grid, dim3(256), 0, stream, h, st, (int)pl->S);
-		break;
-	case 4:
-		hipLaunchKernelGGL((k_partial<KT, AP, 4, 4>), grid, dim3(256), 0, stream, h, st, (int)pl->S);
-		break;
-	case 8:
-		hipLaunchKernelGGL((k_partial<KT, AP, 4, 8>), grid, dim3(256), 0, stream, h, st, (int)pl->S);
-		break;
+		X(1) X(2) X(4) X(8)
+#undef X
 	default:
 		return (int)hipErrorInvalidValue;
 	}
 	return (int)hipGetLastError();
 }
 
+// The workgroup shapes NA x NB of the matrix-core kernels.
+#define NMFK_SHAPE_LIST(X) X(1, 4) X(2, 2) X(4, 1) X(2, 4) X(4, 2)
+
 template <int KT>
-static int launch_partial_mfma_t(const float *U, size_t ldu, const float *A, const float *B, uint32_t p,
-				 uint32_t q, const nmfk_hplan *pl, float *part, const float *colB, uint32_t ncolB,
-				 float *den, const nmfk_state *st, hipStream_t stream)
+static int launch_half_mfma(const nmfk_half *g, const nmfk_hplan *pl, const nmfk_fin *fin, const nmfk_state *st,
+			    hipStream_t stream)
 {
-	const dim3 grid = xcd_grid(pl);
 	const int na = (int)pl->ap, nb = pl->ap ? (int)(pl->nw / pl->ap) : 0;
+	half_args h;
+	fin_args f;
+	dim3 grid;
 	// byte offsets within one 16-row block of U are 32-bit
-	if (pl->bchunk % 16 != 0 || !mfma_shape_ok(na, nb) || (size_t)16 * ldu * 4 > 0x7fffffffull)
+	if (pl->bchunk % 16 != 0 || !mfma_shape_ok(na, nb) || (size_t)16 * g->ldu * 4 > 0x7fffffffull ||
+	    !kernel_args(g, pl, fin, 64u * na, &h, &f, &grid))
 		return (int)hipErrorInvalidValue;
-	const half_args h = {U, ldu, A, B, (int)p, (int)q, (int)pl->bchunk, (int)pl->nab, part, colB, (int)ncolB, den};
+	if (g->split) {
+#define X(NA_, NB_)                                                                                    \
+	if (na == NA_ && nb == NB_) {                                                                  \
+		hipLaunchKernelGGL((k_partial_split<KT, NA_, NB_>), grid, dim3(64 * NA_ * NB_), 0, stream, h, f, st); \
+		return (int)hipGetLastError();                                                         \
+	}
+		NMFK_SHAPE_LIST(X)
+#undef X
+		return (int)hipErrorInvalidValue;
+	}
 	// A rank up to 4 or 8 at KT 16 sums only its columns in GEMM1 (the default shapes have
 	// these bodies; any other shape sums all 16, which is as correct).
 	if constexpr (KT == 16) {
 		const int ke = (pl->ke == 4 || pl->ke == 8) ? (int)pl->ke : 16;
 #define NMFK_MFMA_KE(NA_, NB_, KE_)                                                                      \
 	if (na == NA_ && nb == NB_ && ke == KE_) {                                                     \
-		hipLaunchKernelGGL((k_partial_mfma<KT, NA_, NB_, KE_>), grid, dim3(64 * NA_ * NB_), 0, stream, h, st, \
-				   (int)pl->S);                                                              \
+		hipLaunchKernelGGL((k_partial_mfma<KT, NA_, NB_, KE_>), grid, dim3(64 * NA_ * NB_), 0, stream, h, f, st); \
 		return (int)hipGetLastError();                                                         \
 	}
 		NMFK_MFMA_KE(1, 4, 4)
@@ -3221,45 +3366,68 @@ static int launch_partial_mfma_t(const float *U, size_t ldu, const float *A, con
 		NMFK_MFMA_KE(2, 2, 8)
 #undef NMFK_MFMA_KE
 	}
-#define NMFK_MFMA_SHAPE(NA_, NB_)                                                                        \
+#define X(NA_, NB_)                                                                                    \
 	if (na == NA_ && nb == NB_) {                                                                  \
-		hipLaunchKernelGGL((k_partial_mfma<KT, NA_, NB_>), grid, dim3(64 * NA_ * NB_), 0, stream, h, st, (int)pl->S); \
+		hipLaunchKernelGGL((k_partial_mfma<KT, NA_, NB_>), grid, dim3(64 * NA_ * NB_), 0, stream, h, f, st); \
 		return (int)hipGetLastError();                                                         \
 	}
-	NMFK_MFMA_SHAPE(1, 4)
-	NMFK_MFMA_SHAPE(2, 2)
-	NMFK_MFMA_SHAPE(4, 1)
-	NMFK_MFMA_SHAPE(2, 4)
-	NMFK_MFMA_SHAPE(4, 2)
-#undef NMFK_MFMA_SHAPE
+	NMFK_SHAPE_LIST(X)
+#undef X
 	return (int)hipErrorInvalidValue;
 }
 
-extern "C" int nmfk_launch_partial(const float *U, size_t ldu, const float *A, const float *B, uint32_t p,
-				   uint32_t q, uint32_t kt, const nmfk_hplan *pl, float *part,
-				   const float *colB, uint32_t ncolB, float *den,
-				   const nmfk_state *st, hipStream_t stream)
+template <int KT>
+static int launch_half_bf16(const nmfk_half *g, const nmfk_hplan *pl, const nmfk_fin *fin, const nmfk_state *st,
+			    hipStream_t stream)
 {
-	if (ldu % 4 != 0 || pl->path == NMFK_PATH_MFMA_BF16)   // BF16: nmfk_launch_partial_bf16
+	const int na = (int)pl->ap, nb = pl->ap ? (int)(pl->nw / pl->ap) : 0;
+	half_args h;
+	fin_args f;
+	dim3 grid;
+	if (pl->bchunk % 32 != 0 || !mfma_shape_ok(na, nb) || g->Bb == nullptr || !kernel_args(g, pl, fin, 64u * na, &h, &f, &grid))
 		return (int)hipErrorInvalidValue;
-	if (pl->path == NMFK_PATH_MFMA32) {
-		switch (kt) {
+	const bf16_args b = {(const __bf16 *)g->Bb};
+#define X(NA_, NB_)                                                                                    \
+	if (na == NA_ && nb == NB_) {                                                                  \
+		hipLaunchKernelGGL((k_partial_bf16<KT, NA_, NB_>), grid, dim3(64 * NA_ * NB_), 0, stream, h, b, f, st); \
+		return (int)hipGetLastError();                                                         \
+	}
+	NMFK_SHAPE_LIST(X)
+#undef X
+	return (int)hipErrorInvalidValue;
+}
+
+static int launch_half_sums(const nmfk_half *g, const nmfk_hplan *pl, const nmfk_fin *fin, const nmfk_state *st,
+			    hipStream_t stream)
+{
+	if (g->ldu % 4 != 0 || (g->split && pl->path != NMFK_PATH_MFMA32))
+		return (int)hipErrorInvalidValue;
+	if (pl->path == NMFK_PATH_MFMA_BF16) {
+		switch (g->kt) {
 #define X(K)                                                                                          \
 	case K:                                                                                       \
-		return launch_partial_mfma_t<K>(U, ldu, A, B, p, q, pl, part, colB, ncolB, den, st, stream);
+		return launch_half_bf16<K>(g, pl, fin, st, stream);
+			NMFK_KT_BF16_LIST(X)
+#undef X
+		default:
+			return (int)hipErrorInvalidValue;
+		}
+	}
+	if (pl->path == NMFK_PATH_MFMA32) {
+		switch (g->kt) {
+#define X(K)                                                                                          \
+	case K:                                                                                       \
+		return launch_half_mfma<K>(g, pl, fin, st, stream);
 			NMFK_KT_MFMA_LIST(X)
 #undef X
 		default:
 			return (int)hipErrorInvalidValue;
 		}
 	}
-	if (pl->ap != default_ap(kt))
-		return (int)hipErrorInvalidValue;
-	switch (kt) {
+	switch (g->kt) {
 #define X(K)                                                                                          \
 	case K:                                                                                       \
-		return launch_partial_t<K, (K <= 8 ? 4 : (K <= 32 ? 2 : 1))>(U, ldu, A, B, p, q, pl, part, \
-									      colB, ncolB, den, st, stream);
+		return launch_half_valu<K, (K <= 8 ? 4 : (K <= 32 ? 2 : 1))>(g, pl, fin, st, stream);
 		NMFK_KT_LIST(X)
 #undef X
 	default:
@@ -3267,80 +3435,33 @@ extern "C" int nmfk_launch_partial(const float *U, size_t ldu, const float *A, c
 	}
 }
 
-template <int KT>
-static int launch_partial_split_t(const half_args &h, const nmfk_hplan *pl, const nmfk_state *st, hipStream_t stream)
+extern "C" int nmfk_launch_finish(const float *part, uint32_t S, uint32_t p, uint32_t kt, int split, const nmfk_fin *f,
+				  const nmfk_state *st, hipStream_t stream)
 {
-	const dim3 grid = xcd_grid(pl);
-	const int na = (int)pl->ap, nb = pl->ap ? (int)(pl->nw / pl->ap) : 0;
-#define NMFK_SPLIT_SHAPE(NA_, NB_)                                                                       \
-	if (na == NA_ && nb == NB_) {                                                                  \
-		hipLaunchKernelGGL((k_partial_split<KT, NA_, NB_>), grid, dim3(64 * NA_ * NB_), 0, stream, h, st, (int)pl->S); \
+	const unsigned g = (p + NMFK_FIN_ROWS - 1) / NMFK_FIN_ROWS;
+	if (f->Ab != nullptr && kt % 32 != 0)
+		return (int)hipErrorInvalidValue;
+#define X(K, PAIR)                                                                                     \
+	if (kt == K && (split != 0) == PAIR) {                                                         \
+		hipLaunchKernelGGL((k_finish<K, PAIR>), dim3(g), dim3(NMFK_WG), 0, stream, part, (int)S, f->A, (int)p, \
+				   (int)f->k, f->den, f->colA, f->clamp, st, (__bf16 *)f->Ab);          \
 		return (int)hipGetLastError();                                                         \
 	}
-	NMFK_SPLIT_SHAPE(1, 4)
-	NMFK_SPLIT_SHAPE(2, 2)
-	NMFK_SPLIT_SHAPE(4, 1)
-	NMFK_SPLIT_SHAPE(2, 4)
-	NMFK_SPLIT_SHAPE(4, 2)
-#undef NMFK_SPLIT_SHAPE
+	X(4, false) X(8, false) X(16, false) X(32, false) X(64, false)
+	X(16, true) X(32, true) X(64, true)
+#undef X
 	return (int)hipErrorInvalidValue;
 }
 
-extern "C" int nmfk_launch_partial_split(const float *U, size_t ldu, const float *A, const float *B, uint32_t p,
-					 uint32_t q, uint32_t kt, const nmfk_hplan *pl, float *part, const float *colB,
-					 uint32_t ncolB, float *den, const nmfk_state *st, hipStream_t stream)
+extern "C" int nmfk_launch_half(const nmfk_half *g, const nmfk_hplan *pl, const nmfk_fin *fin, const nmfk_state *st,
+				hipStream_t stream)
 {
-	// byte offsets within one 16-row block of U are 32-bit
-	if (ldu % 4 != 0 || pl->path != NMFK_PATH_MFMA32 || pl->bchunk % 16 != 0 || (size_t)16 * ldu * 4 > 0x7fffffffull)
+	if (fin && fin->Ab != nullptr && g->kt % 32 != 0)
 		return (int)hipErrorInvalidValue;
-	const half_args h = {U, ldu, A, B, (int)p, (int)q, (int)pl->bchunk, (int)pl->nab, part, colB, (int)ncolB, den};
-	switch (kt) {
-#define X(K)                                                                                          \
-	case K:                                                                                       \
-		return launch_partial_split_t<K>(h, pl, st, stream);
-		NMFK_KT_MFMA_LIST(X)
-#undef X
-	default:
-		return (int)hipErrorInvalidValue;
-	}
-}
-
-extern "C" int nmfk_launch_finish_split(const float *part, uint32_t S, float *A, uint32_t p, uint32_t k, uint32_t kt,
-					const float *den, float *colA, int clamp, const nmfk_state *st, hipStream_t stream)
-{
-	const unsigned g = (p + NMFK_FIN_ROWS - 1) / NMFK_FIN_ROWS;
-	switch (kt) {
-#define X(K)                                                                                           \
-	case K:                                                                                        \
-		hipLaunchKernelGGL((k_finish<K, true>), dim3(g), dim3(NMFK_WG), 0, stream, part, (int)S, A, (int)p, \
-				   (int)k, den, colA, clamp, st, shadow_args{});                        \
-		return (int)hipGetLastError();
-		NMFK_KT_MFMA_LIST(X)
-#undef X
-	default:
-		return (int)hipErrorInvalidValue;
-	}
-}
-
-extern "C" int nmfk_launch_finish_shadow(const float *part, uint32_t S, float *A, uint32_t p, uint32_t k,
-					 uint32_t kt, const float *den, float *colA, int clamp, const nmfk_state *st,
-					 uint16_t *Ab, hipStream_t stream)
-{
-	const unsigned g = (p + NMFK_FIN_ROWS - 1) / NMFK_FIN_ROWS;
-	if (Ab != nullptr && kt % 32 != 0)
-		return (int)hipErrorInvalidValue;
-	const shadow_args sh = {(__bf16 *)Ab};
-	switch (kt) {
-#define X(K)                                                                                           \
-	case K:                                                                                        \
-		hipLaunchKernelGGL((k_finish<K, false>), dim3(g), dim3(NMFK_WG), 0, stream, part, (int)S, A, (int)p, \
-				   (int)k, den, colA, clamp, st, sh);                                   \
-		return (int)hipGetLastError();
-		NMFK_KT_LIST(X)
-#undef X
-	default:
-		return (int)hipErrorInvalidValue;
-	}
+	const int e = launch_half_sums(g, pl, fin, st, stream);
+	if (e || !fin || pl->S == 1)
+		return e;
+	return nmfk_launch_finish(g->part, pl->S, g->p, g->kt, g->split, fin, st, stream);
 }
 
 extern "C" int nmfk_fused_plan(uint32_t n, uint32_t m, uint32_t kt, uint32_t *G, uint32_t *nwv)
@@ -3391,13 +3512,6 @@ extern "C" int nmfk_launch_fused_finish(const float *part, uint32_t G, const flo
 	return (int)hipGetLastError();
 }
 
-extern "C" int nmfk_launch_finish(const float *part, uint32_t S, float *A, uint32_t p, uint32_t k, uint32_t kt,
-				  const float *den, float *colA, int clamp, const nmfk_state *st,
-				  hipStream_t stream)
-{
-	return nmfk_launch_finish_shadow(part, S, A, p, k, kt, den, colA, clamp, st, nullptr, stream);
-}
-
 extern "C" int nmfk_launch_shadow(const float *A, uint32_t p, uint32_t kt, uint16_t *Ab, hipStream_t stream)
 {
 	const unsigned g = (p + NMFK_FIN_ROWS - 1) / NMFK_FIN_ROWS;
@@ -3406,48 +3520,6 @@ extern "C" int nmfk_launch_shadow(const float *A, uint32_t p, uint32_t kt, uint1
 	case K:                                                                                        \
 		hipLaunchKernelGGL((k_shadow<K>), dim3(g), dim3(NMFK_WG), 0, stream, A, (int)p, (__bf16 *)Ab); \
 		return (int)hipGetLastError();
-		NMFK_KT_BF16_LIST(X)
-#undef X
-	default:
-		return (int)hipErrorInvalidValue;
-	}
-}
-
-template <int KT>
-static int launch_partial_bf16_t(const float *U, size_t ldu, const float *A, const uint16_t *Bb, uint32_t p,
-				 uint32_t q, const nmfk_hplan *pl, float *part, const float *colB, uint32_t ncolB,
-				 float *den, const nmfk_state *st, hipStream_t stream)
-{
-	const dim3 grid = xcd_grid(pl);
-	const int na = (int)pl->ap, nb = pl->ap ? (int)(pl->nw / pl->ap) : 0;
-	if (pl->bchunk % 32 != 0 || !mfma_shape_ok(na, nb))
-		return (int)hipErrorInvalidValue;
-	const half_args h = {U, ldu, A, nullptr, (int)p, (int)q, (int)pl->bchunk, (int)pl->nab, part, colB, (int)ncolB, den};
-	const bf16_args b = {(const __bf16 *)Bb};
-#define NMFK_BF16_SHAPE(NA_, NB_)                                                                        \
-	if (na == NA_ && nb == NB_) {                                                                  \
-		hipLaunchKernelGGL((k_partial_bf16<KT, NA_, NB_>), grid, dim3(64 * NA_ * NB_), 0, stream, h, b, st, (int)pl->S); \
-		return (int)hipGetLastError();                                                         \
-	}
-	NMFK_BF16_SHAPE(1, 4)
-	NMFK_BF16_SHAPE(2, 2)
-	NMFK_BF16_SHAPE(4, 1)
-	NMFK_BF16_SHAPE(2, 4)
-	NMFK_BF16_SHAPE(4, 2)
-#undef NMFK_BF16_SHAPE
-	return (int)hipErrorInvalidValue;
-}
-
-extern "C" int nmfk_launch_partial_bf16(const float *U, size_t ldu, const float *A, const uint16_t *Bb, uint32_t p,
-					uint32_t q, uint32_t kt, const nmfk_hplan *pl, float *part, const float *colB,
-					uint32_t ncolB, float *den, const nmfk_state *st, hipStream_t stream)
-{
-	if (ldu % 4 != 0 || pl->path != NMFK_PATH_MFMA_BF16)
-		return (int)hipErrorInvalidValue;
-	switch (kt) {
-#define X(K)                                                                                          \
-	case K:                                                                                       \
-		return launch_partial_bf16_t<K>(U, ldu, A, Bb, p, q, pl, part, colB, ncolB, den, st, stream);
 		NMFK_KT_BF16_LIST(X)
 #undef X
 	default:

@@ -72,7 +72,6 @@ void nmfk_stream_free(nmfk_job *j)
 	}
 	hipFree(j->partH);
 	hipFree(j->Hc);
-	hipFree(j->den_scratch);
 	if (j->cstream)
 		hipStreamDestroy(j->cstream);
 }
@@ -125,7 +124,7 @@ static void stream_layout(uint32_t n, uint32_t m, uint32_t k, uint32_t block_row
 	L->ndot = nmfk_dot_kl_blocks(br, m);
 	const size_t kt = L->kt;
 	L->bytes = 4 * ((size_t)n * kt + 2 * (size_t)m * kt + L->part_cap + (size_t)L->SH * m * kt +
-			((size_t)L->ncolW + L->ncolH + 3) * kt + 2 * (size_t)m) +
+			((size_t)L->ncolW + L->ncolH + 2) * kt + 2 * (size_t)m) +
 		   8 * 3 * (size_t)L->ndot + sizeof(nmfk_state) +
 		   2 * 4 * ((size_t)br * L->ldv + (size_t)m * L->ldvtb) + 20 * 256;
 }
@@ -187,7 +186,6 @@ nmfk_job *nmfk_job_create_streamed(uint32_t n, uint32_t m, uint32_t k, const flo
 	if (!e) e |= salloc((void **)&j->colH, 4 * (size_t)j->ncolH * kt, "hipMalloc(colH)");
 	if (!e) e |= salloc((void **)&j->denW, 4 * 2 * kt, "hipMalloc(den)");
 	if (!e) j->denH = j->denW + kt;
-	if (!e) e |= salloc((void **)&j->den_scratch, 4 * kt, "hipMalloc(den scratch)");
 	if (!e) e |= salloc((void **)&j->dot, 8 * 3 * (size_t)j->ndot, "hipMalloc(dot)");
 	if (!e) e |= salloc((void **)&j->cls, 4 * (size_t)m, "hipMalloc(cls)");
 	if (!e) e |= salloc((void **)&j->last, 4 * (size_t)m, "hipMalloc(last)");
@@ -358,19 +356,17 @@ static int pass(nmfk_job *j, int kind, const float *Hp, int clamp, double acc[3]
 		float *Wb = j->W + (size_t)i0 * j->kt;
 		if (!e && (kind == PASS_WH || kind == PASS_W)) {
 			e = nmfk_launch_transpose(j->Vb[s], r, j->m, j->ldv, j->Vtb[s], j->ldvtb, j->stream);
+			const nmfk_half g = {j->Vtb[s], j->ldvtb, Wb, j->H, NULL, r, j->m, j->kt, 0, j->part};
+			const nmfk_fin f = {Wb, j->colW + (size_t)(i0 / NMFK_FIN_ROWS) * j->kt, NULL, j->colH, j->ncolH,
+					    j->denH, j->k, clamp};
 			if (!e)
-				e = nmfk_launch_partial(j->Vtb[s], j->ldvtb, Wb, j->H, r, j->m, j->kt, pw, j->part, j->colH,
-							j->ncolH, j->denH, st, j->stream);
-			if (!e)
-				e = nmfk_launch_finish(j->part, pw->S, Wb, r, j->k, j->kt, j->denH,
-						       j->colW + (size_t)(i0 / NMFK_FIN_ROWS) * j->kt, clamp, st, j->stream);
+				e = nmfk_launch_half(&g, pw, &f, st, j->stream);
 		}
 		if (!e && (kind == PASS_H0 || kind == PASS_WH)) {
-			/* the partial kernel's denominator tile reduces no parts into a scratch buffer:
-			 * colsum(W) is complete only after the pass */
-			e = nmfk_launch_partial(j->Vb[s], j->ldv, Hp, Wb, j->m, r, j->kt, ph,
-						j->partH + (size_t)hoff * j->m * j->kt, j->colW, 0, j->den_scratch, st,
-						j->stream);
+			/* sums only: the other blocks' and colsum(W) are complete after the pass */
+			const nmfk_half g = {j->Vb[s], j->ldv, Hp, Wb, NULL, j->m, r, j->kt, 0,
+					     j->partH + (size_t)hoff * j->m * j->kt};
+			e = nmfk_launch_half(&g, ph, NULL, st, j->stream);
 			hoff += ph->S;
 		}
 		if (!e && kind == PASS_DOT) {
@@ -388,6 +384,13 @@ static int pass(nmfk_job *j, int kind, const float *Hp, int clamp, double acc[3]
 	}
 	free(h);
 	return e ? nmfk_hip_fail(e, "streamed pass") : 0;
+}
+
+/* The H half-step from the sums of all blocks. */
+static int finish_H(nmfk_job *j, const nmfk_state *st)
+{
+	const nmfk_fin f = {j->H, j->colH, NULL, NULL, 0, j->denW, j->k, 0};
+	return nmfk_launch_finish(j->partH, j->SH, j->m, j->kt, 0, &f, st, j->stream);
 }
 
 int nmfk_stream_run(nmfk_job *j, const nmfk_options *opt, nmfk_result *res)
@@ -408,8 +411,7 @@ int nmfk_stream_run(nmfk_job *j, const nmfk_options *opt, nmfk_result *res)
 		/* iteration 0's H half-step */
 		e = pass(j, PASS_H0, j->H, 0, NULL, j->st);
 		if (!e)
-			e = nmfk_hip_fail(nmfk_launch_finish(j->partH, j->SH, j->H, j->m, j->k, j->kt, j->denW, j->colH, 0,
-							     j->st, j->stream),
+			e = nmfk_hip_fail(finish_H(j, j->st),
 					  "H finish");
 	}
 	/* Pass it completes iteration it - 1 (its W half-step) and adds iteration it's H partial sums. */
@@ -433,8 +435,7 @@ int nmfk_stream_run(nmfk_job *j, const nmfk_options *opt, nmfk_result *res)
 		if (!e && more) {
 			e = nmfk_launch_den(j->colW, j->ncolW, j->kt, j->denW, j->stream);
 			if (!e)
-				e = nmfk_launch_finish(j->partH, j->SH, j->H, j->m, j->k, j->kt, j->denW, j->colH, 0, j->st,
-						       j->stream);
+				e = finish_H(j, j->st);
 			e = nmfk_hip_fail(e, "H finish");
 		}
 		if (!e && test) {
@@ -500,8 +501,7 @@ int nmfk_stream_update_H(nmfk_job *j)
 		return nmfk_hip_fail(e, "update_H");
 	e = pass(j, PASS_H0, j->H, 0, NULL, NULL);
 	if (!e)
-		e = nmfk_hip_fail(nmfk_launch_finish(j->partH, j->SH, j->H, j->m, j->k, j->kt, j->denW, j->colH, 0, NULL,
-						     j->stream),
+		e = nmfk_hip_fail(finish_H(j, NULL),
 				  "update_H");
 	return e;
 }

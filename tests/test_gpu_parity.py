@@ -171,6 +171,35 @@ def test_split_products_same_bits_in_a_batch(nmfk, n, m, k):
         assert np.array_equal(a.get_W(), b.get_W()) and np.array_equal(a.get_H(), b.get_H())
 
 
+@pytest.mark.parametrize("n,m,k,path,na,nb", [
+    (1985, 33, 3, 2, 1, 4), (2049, 64, 7, 2, 2, 2), (2111, 65, 16, 2, 4, 1), (1985, 40, 12, 2, 2, 4), (2305, 39, 30, 2, 4, 2),
+    (2049, 65, 40, 2, 4, 2), (1985, 33, 20, 3, 2, 4), (2111, 63, 48, 3, 1, 4), (30, 5, 4, 1, 1, 4), (2047, 5, 5, 1, 1, 4),
+    (65, 9, 7, 1, 1, 4), (2049, 20, 13, 1, 1, 4), (2001, 30, 20, 1, 1, 4), (32801, 40, 34, 1, 1, 4)])
+def test_one_split_finishes_in_its_launch(nmfk, orc, n, m, k, path, na, nb):
+    # A half-step of one split updates its rows, their column sums and BF16 copies in the launch
+    # that sums them: two iterations, so that the second divides by those column sums, in every
+    # workgroup shape and with partly filled last blocks of rows, against the FP64 oracle.  The
+    # bar is four half-steps at the 1e-5 of one (BF16: that of the ragged shapes).
+    old = (nmfk.tune_get(nmfk.TUNE_MFMA_NA), nmfk.tune_get(nmfk.TUNE_MFMA_NB))
+    nmfk.tune_set(nmfk.TUNE_MFMA_NA, na)
+    nmfk.tune_set(nmfk.TUNE_MFMA_NB, nb)
+    try:
+        job, V = make_job(nmfk, orc, n, m, k, seed_v=n + k, seed_init=k)
+        with job:
+            job.set_kernel_path(path)
+            assert job.plan()["W"]["S"] == 1
+            W, H = orc.init_WH(n, m, k, k)
+            for _ in range(2):
+                H = orc.update_H(V, W, H)
+                W = orc.update_W(V, W, H)
+            job.run(2, 2, 1000)
+            tol = 2e-2 if path == 3 else 4e-5
+            assert rel_err(job.get_H(), H) < tol and rel_err(job.get_W(), W) < tol
+    finally:
+        nmfk.tune_set(nmfk.TUNE_MFMA_NA, old[0])
+        nmfk.tune_set(nmfk.TUNE_MFMA_NB, old[1])
+
+
 def test_golden_tiny_runs(nmfk, orc):
     g = np.load(GOLDEN / "tiny.npz")
     for ci in range(int(g["ncases"])):
