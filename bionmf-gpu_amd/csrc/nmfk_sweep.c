@@ -38,15 +38,34 @@ void nmfk_sweep_default_config(nmfk_sweep_config *c)
 	c->autotune_iters = 20;
 }
 
-static int sweep_fail(nmfk_job **jobs, uint32_t nj, nmfk_batch *b, int32_t *dC, int e)
+/* What one sweep holds; its jobs' buffers come from one arena and their work before and after
+ * the batch runs on one stream, so that 54 jobs make one hipMalloc and one stream instead of
+ * 600 and 54. */
+typedef struct sweep_state {
+	nmfk_job **jobs;
+	uint32_t nj;
+	nmfk_arena *arena;
+	hipStream_t stream;
+	nmfk_batch *b;
+} sweep_state;
+
+static int sweep_end(sweep_state *s, int e)
 {
-	if (b)
-		nmfk_batch_destroy(b);
-	for (uint32_t i = 0; i < nj; i++)
-		nmfk_job_destroy(jobs[i]);
-	free(jobs);
-	hipFree(dC);
-	return e ? e : NMFK_EINVAL;
+	nmfk_batch_destroy(s->b);
+	for (uint32_t i = 0; i < s->nj; i++)
+		nmfk_job_destroy(s->jobs[i]);
+	free(s->jobs);
+	if (s->stream) {
+		hipStreamSynchronize(s->stream);
+		hipStreamDestroy(s->stream);
+	}
+	nmfk_arena_destroy(s->arena);
+	return e;
+}
+
+static int sweep_fail(sweep_state *s, int e)
+{
+	return sweep_end(s, e ? e : NMFK_EINVAL);
 }
 
 int nmfk_sweep_run(nmfk_job *src, const nmfk_sweep_config *cfg, nmfk_sweep_out *out)
@@ -59,19 +78,34 @@ int nmfk_sweep_run(nmfk_job *src, const nmfk_sweep_config *cfg, nmfk_sweep_out *
 		nmfk_set_error("nmfk_sweep_run: batched mode needs nIters >= niter_test_conv");
 		return NMFK_EINVAL;
 	}
+	if (src->streamed) {
+		nmfk_set_error("nmfk_sweep_run: the source job's V is in host memory (streamed job)");
+		return NMFK_EINVAL;
+	}
 	const uint32_t R = cfg->restarts, nj = cfg->nk * R, m = src->m;
 	nmfk_job **jobs = (nmfk_job **)calloc(nj, sizeof(nmfk_job *));
 	if (!jobs) {
 		nmfk_set_error("out of host memory");
 		return NMFK_ENOMEM;
 	}
+	const size_t mm = (size_t)m * m, c_bytes = cfg->nk * mm * sizeof(int32_t);
 	int32_t *dC = NULL;
 	nmfk_batch *b = NULL;
-	int e = 0;
+	sweep_state sw = {jobs, nj, NULL, NULL, NULL};
+	size_t bytes = nmfk_arena_round(c_bytes);
+	for (uint32_t q = 0; q < cfg->nk; q++)
+		bytes += (cfg->ks[q] >= 1 && cfg->ks[q] <= NMFK_KMAX) ? R * nmfk_job_bytes_shared(src->n, m, cfg->ks[q]) : 0;
+	int e = nmfk_hip_fail(hipStreamCreateWithFlags(&sw.stream, hipStreamNonBlocking), "hipStreamCreate(sweep)");
+	if (!e && !(sw.arena = nmfk_arena_create(bytes, bytes)))
+		e = NMFK_ENOMEM;
+	if (!e && !(dC = (int32_t *)nmfk_arena_alloc(sw.arena, c_bytes))) {
+		nmfk_set_error("nmfk_sweep_run: cannot reserve %zu bytes of device memory", bytes);
+		e = NMFK_EHIP;
+	}
 	for (uint32_t q = 0; q < cfg->nk && !e; q++)
 		for (uint32_t r = 0; r < R && !e; r++) {
 			const uint32_t i = q * R + r;
-			jobs[i] = nmfk_job_create_shared(src, cfg->ks[q]);
+			jobs[i] = nmfk_job_create_in(sw.arena, sw.stream, src->n, m, cfg->ks[q], src);
 			if (!jobs[i]) {
 				e = NMFK_EINVAL;
 				break;
@@ -82,7 +116,7 @@ int nmfk_sweep_run(nmfk_job *src, const nmfk_sweep_config *cfg, nmfk_sweep_out *
 				e = nmfk_job_init_random(jobs[i], nmfk_sweep_seed(cfg->base_seed, cfg->ks[q], r));
 		}
 	if (e)
-		return sweep_fail(jobs, nj, b, dC, e);
+		return sweep_fail(&sw, e);
 
 	nmfk_options opt;
 	opt.nIters = cfg->nIters;
@@ -137,7 +171,7 @@ int nmfk_sweep_run(nmfk_job *src, const nmfk_sweep_config *cfg, nmfk_sweep_out *
 				e = nmfk_job_replan(jobs[i], best_target);
 			tune_s = nmfk_now() - ta;
 		}
-		b = e ? NULL : nmfk_batch_create(cfg->niter_test_conv, nj);
+		b = sw.b = e ? NULL : nmfk_batch_create(cfg->niter_test_conv, nj);
 		if (!e && !b)
 			e = NMFK_EINVAL;
 		for (uint32_t i = 0; i < nj && !e; i++) {
@@ -184,18 +218,15 @@ int nmfk_sweep_run(nmfk_job *src, const nmfk_sweep_config *cfg, nmfk_sweep_out *
 	}
 	const double t1 = nmfk_now();
 	if (e)
-		return sweep_fail(jobs, nj, b, dC, e);
+		return sweep_fail(&sw, e);
 	if (out) {
 		out->seconds = t1 - t0 - tune_s;
 		out->tune_seconds = tune_s;
 	}
 
 	/* Final class vectors (argmax of the final H) and the consensus matrices. */
-	const size_t mm = (size_t)m * m;
-	hipStream_t s = src->stream;
-	e = hipMalloc((void **)&dC, cfg->nk * mm * sizeof(int32_t));
-	if (!e)
-		e = hipMemsetAsync(dC, 0, cfg->nk * mm * sizeof(int32_t), s);
+	hipStream_t s = sw.stream;
+	e = hipMemsetAsync(dC, 0, c_bytes, s);
 	for (uint32_t q = 0; q < cfg->nk && !e; q++)
 		for (uint32_t r = 0; r < R && !e; r++) {
 			nmfk_job *j = jobs[q * R + r];
@@ -209,12 +240,12 @@ int nmfk_sweep_run(nmfk_job *src, const nmfk_sweep_config *cfg, nmfk_sweep_out *
 						   hipMemcpyDeviceToHost, s);
 		}
 	if (!e && out && out->consensus)
-		e = hipMemcpyAsync(out->consensus, dC, cfg->nk * mm * sizeof(int32_t), hipMemcpyDeviceToHost, s);
+		e = hipMemcpyAsync(out->consensus, dC, c_bytes, hipMemcpyDeviceToHost, s);
 	if (!e)
 		e = hipStreamSynchronize(s);
 	if (e) {
 		nmfk_hip_fail(e, "sweep consensus");
-		return sweep_fail(jobs, nj, b, dC, NMFK_EHIP);
+		return sweep_fail(&sw, NMFK_EHIP);
 	}
 	if (out && out->W_H_out) {
 		/* optional per-job factor export, k-major (row-major n x k then m x k) */
@@ -227,11 +258,5 @@ int nmfk_sweep_run(nmfk_job *src, const nmfk_sweep_config *cfg, nmfk_sweep_out *
 			o += (size_t)jobs[i]->m * jobs[i]->k;
 		}
 	}
-	if (b)
-		nmfk_batch_destroy(b);
-	for (uint32_t i = 0; i < nj; i++)
-		nmfk_job_destroy(jobs[i]);
-	free(jobs);
-	hipFree(dC);
-	return e;
+	return sweep_end(&sw, e);
 }
