@@ -192,7 +192,7 @@ int nmfk_launch_batch_partial(const nmfk_bjob *jobs, const nmfk_tile *tiles, uin
 int nmfk_launch_batch_finish(const nmfk_bjob *jobs, const nmfk_tile *tiles, uint32_t ntiles, int half,
 			     int clamp, uint32_t grid, hipStream_t stream);
 /* Test: rows tiles (job, row block of NMFK_TEST_ROWS), then one final workgroup per job. */
-#define NMFK_TEST_ROWS 32
+#define NMFK_TEST_ROWS 8
 int nmfk_launch_batch_test(const nmfk_bjob *jobs, const nmfk_tile *row_tiles, uint32_t nrow_tiles,
 			   uint32_t njobs, uint32_t grid, hipStream_t stream);
 

@@ -249,6 +249,21 @@ __device__ __forceinline__ void load_u(const float *__restrict__ src, int avail,
 		u[r] = (r < avail) ? u[r] : 0.0f;
 }
 
+// Whether the job has converged and a launch is to leave everything as it is: read first, and
+// looked at (stopped) once the first operands are on the way.  A vector load, since those come
+// back in order: a scalar one would be waited for with the kernel's arguments, ahead of the
+// operands' addresses.
+__device__ __forceinline__ uint32_t read_stop(const nmfk_state *st)
+{
+	return st != nullptr ? __hip_atomic_load(&st->converged, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WAVEFRONT) : 0u;
+}
+// The memory clobber keeps the loads before it there; the compiler would move them behind the branch.
+__device__ __forceinline__ bool stopped(uint32_t stop)
+{
+	asm volatile("" : "+v"(stop) : : "memory");
+	return __builtin_amdgcn_readfirstlane(stop) != 0;
+}
+
 // Arguments of one half-step's partial kernel: update A (p x KT) against B (q x KT)
 // through U (q x p, leading dimension ldu).
 struct half_args {
@@ -366,7 +381,7 @@ __global__ __launch_bounds__(NMFK_WG) void k_shadow(const float *__restrict__ A,
 // occupancy to the registers.
 template <int KT, bool PAIR, bool LDS, bool DEEP>
 __device__ __forceinline__ void finish_block(int blk, int tid, const float *__restrict__ part, int S, float *A, int p, int k,
-					     const float *den, float *colA, int clamp, __bf16 *Ab, float *smem)
+					     const float *den, float *colA, int clamp, __bf16 *Ab, float *smem, uint32_t stop = 0)
 {
 	constexpr int TPR = fin_tpr(KT), Q = fin_q(KT);
 	const int a = blk * NMFK_FIN_ROWS + tid / TPR;
@@ -463,15 +478,19 @@ __device__ __forceinline__ void finish_block(int blk, int tid, const float *__re
 			}
 			x[i] = v;
 		}
+	} else {
+#pragma unroll
+		for (int i = 0; i < Q; i++)
+			x[i] = 0.0f;
+	}
+	if (stopped(stop))
+		return;
+	if (a < p) {
 		stq<Q>(A + (size_t)a * KT + c0, x);
 		if constexpr (KT % 32 == 0) {
 			if (Ab != nullptr)
 				store_shadow<KT>(a, c0, x, Ab);
 		}
-	} else {
-#pragma unroll
-		for (int i = 0; i < Q; i++)
-			x[i] = 0.0f;
 	}
 	block_colsum_store<KT, PAIR>(tid, x, blk * NMFK_FIN_ROWS < p ? colA + (size_t)blk * KT : nullptr, smem);
 }
@@ -540,14 +559,14 @@ __device__ __forceinline__ void finish_rows(int bx, int rows, const half_args &h
 // critical path of the streaming ones; the rest of that column return at once.  True for a
 // workgroup with rows (bx, by) to stream.
 template <int KT, bool PAIR, int ROOM>
-__device__ __forceinline__ bool half_tile(const half_args &h, const fin_args &f, float *smem, int &bx, int &by)
+__device__ __forceinline__ bool half_tile(const half_args &h, const fin_args &f, float *smem, uint32_t stop, int &bx, int &by)
 {
 	const int gx = h.part ? h.nab + 1 : h.nab;
 	if (!xcd_tile(gx, gx * h.S, bx, by))
 		return false;
 	if (bx < h.nab)
 		return true;
-	if (by == 0 && f.den != nullptr)
+	if (by == 0 && f.den != nullptr && !stopped(stop))
 		den_reduce<KT, PAIR>(f.colB, f.ncolB, f.den, smem, ROOM - 4 * KT);
 	return false;
 }
@@ -559,7 +578,7 @@ __device__ __forceinline__ bool half_tile(const half_args &h, const fin_args &f,
 // rows (p <= 64 AP / LB) still keeps every lane busy.  The groups' sums are added by a
 // fixed xor tree at the end, then the waves' by a fixed LDS tree.
 template <int KT, int AP, int NW, int LB = 1>
-__device__ __forceinline__ void partial_valu_body(int bx, int by, const half_args &h, float *__restrict__ smem)
+__device__ __forceinline__ void partial_valu_body(int bx, int by, const half_args &h, float *__restrict__ smem, uint32_t stop = 0)
 {
 	static_assert(LB == 1 || LB == 2 || LB == 4 || LB == 8, "lane groups: 1, 2, 4 or 8");
 	constexpr int LA = 64 / LB;
@@ -609,6 +628,8 @@ __device__ __forceinline__ void partial_valu_body(int bx, int by, const half_arg
 #pragma unroll
 	for (int d = 0; d < DR; d++)
 		fetch(b_begin + wave * LB + lg + d * STEP, un[d], bn[d]);
+	if (stopped(stop))
+		return;
 	for (int b = b_begin + wave * LB + lg; b < b_end; b += DR * STEP) {
 #pragma unroll
 		for (int d = 0; d < DR; d++) {
@@ -701,13 +722,12 @@ __global__ __launch_bounds__(64 * NW) void k_partial(half_args h, fin_args f, co
 {
 	constexpr int LDS = max2(smem_valu(KT, AP, NW), smem_finish(KT, 64 / LB * AP));
 	__shared__ __align__(16) float smem[LDS];
-	if (st != nullptr && st->converged)
-		return;
+	const uint32_t stop = read_stop(st);
 	int bx, by;
-	if (!half_tile<KT, false, LDS>(h, f, smem, bx, by))
+	if (!half_tile<KT, false, LDS>(h, f, smem, stop, bx, by))
 		return;
-	partial_valu_body<KT, AP, NW, LB>(bx, by, h, smem);
-	if (h.part == nullptr)
+	partial_valu_body<KT, AP, NW, LB>(bx, by, h, smem, stop);
+	if (h.part == nullptr && !stopped(stop))
 		finish_rows<KT, false, 64 * NW>(bx, 64 / LB * AP, h, f, smem);
 }
 
@@ -869,7 +889,8 @@ __device__ __forceinline__ void mfma_store(floatx4 (&acc)[4][KT / 16], const hal
 // keep the 16-wide GEMM2 at KE 8.
 #define NMFK_G2N_MAX_KE 4
 template <int KT, int NA, int NB, int KE = KT>
-__device__ __forceinline__ void partial_mfma_body(int bx, int by, const half_args &ha, float *__restrict__ smem)
+__device__ __forceinline__ void partial_mfma_body(int bx, int by, const half_args &ha, float *__restrict__ smem,
+						  uint32_t stop = 0)
 {
 	static_assert(KT % 16 == 0, "MFMA path needs KT % 16 == 0");
 	static_assert(KE == KT || (KT == 16 && (KE == 4 || KE == 8)), "GEMM1 width: KT, or 4 / 8 at KT 16");
@@ -1062,6 +1083,8 @@ __device__ __forceinline__ void partial_mfma_body(int bx, int by, const half_arg
 		for (int d = 0; d < D; d++)
 			load_full(blk_row(d), ring[d]);
 	}
+	if (stopped(stop))
+		return;
 	if constexpr (D >= 2) {
 		// Software pipeline across blocks: GEMM1 of the next block is issued next to GEMM2 of
 		// this one (independent MFMA chains), and the next block's ratios fill the gaps, so
@@ -1173,13 +1196,12 @@ __global__ __launch_bounds__(64 * NA * NB, (KT == 32 ? 3 : 1)) void k_partial_mf
 {
 	constexpr int LDS = max2(smem_mfma(KT, NA, NB), smem_finish(KT, 64 * NA));
 	__shared__ __align__(16) float smem[LDS];
-	if (st != nullptr && st->converged)
-		return;
+	const uint32_t stop = read_stop(st);
 	int bx, by;
-	if (!half_tile<KT, false, LDS>(h, f, smem, bx, by))
+	if (!half_tile<KT, false, LDS>(h, f, smem, stop, bx, by))
 		return;
-	partial_mfma_body<KT, NA, NB, KE>(bx, by, h, smem);
-	if (h.part == nullptr)
+	partial_mfma_body<KT, NA, NB, KE>(bx, by, h, smem, stop);
+	if (h.part == nullptr && !stopped(stop))
 		finish_rows<KT, false, 64 * NA * NB>(bx, 64 * NA, h, f, smem);
 }
 
@@ -1221,7 +1243,8 @@ struct bf16_args {
 
 template <int KT, int NA, int NB>
 __device__ __forceinline__ void partial_bf16_body(int bx, int by, const half_args &ha, const bf16_args &bb16,
-						  float *__restrict__ smem)
+						  float *__restrict__ smem,
+						  uint32_t stop)
 {
 	static_assert(KT % 32 == 0, "BF16 path needs KT % 32 == 0");
 	constexpr int H = KT / 16;     // 16-column groups (GEMM2 outputs)
@@ -1389,12 +1412,16 @@ __device__ __forceinline__ void partial_bf16_body(int bx, int by, const half_arg
 		load_u(blk_row(0), ur[0], true);
 		load_u(blk_row(1), ur[1], true);
 		fetch_b(blk_row(0), true);
+		if (stopped(stop))
+			return;
 		for (int i = 0; i < mine; i += 2) {
 			step(ur[0], blk_row(i + 1), blk_row(i + 2));
 			if (i + 1 < mine)
 				step(ur[1], blk_row(i + 2), blk_row(i + 3));
 		}
 	}
+	if (stopped(stop))   // also where a wave has no full block
+		return;
 	if (!idle && (b_end - b_begin) % 32 != 0 && wb == nfull % NB) {
 		const int bb = b_begin + 32 * nfull;
 		float4 u[2][4];
@@ -1419,13 +1446,12 @@ __global__ __launch_bounds__(64 * NA * NB) void k_partial_bf16(half_args h, bf16
 {
 	constexpr int LDS = max2(smem_bf16(KT, NA, NB), smem_finish(KT, 64 * NA));
 	__shared__ __align__(16) float smem[LDS];
-	if (st != nullptr && st->converged)
-		return;
+	const uint32_t stop = read_stop(st);
 	int bx, by;
-	if (!half_tile<KT, false, LDS>(h, f, smem, bx, by))
+	if (!half_tile<KT, false, LDS>(h, f, smem, stop, bx, by))
 		return;
-	partial_bf16_body<KT, NA, NB>(bx, by, h, b, smem);
-	if (h.part == nullptr)
+	partial_bf16_body<KT, NA, NB>(bx, by, h, b, smem, stop);
+	if (h.part == nullptr && !stopped(stop))
 		finish_rows<KT, false, 64 * NA * NB>(bx, 64 * NA, h, f, smem);
 }
 
@@ -1557,7 +1583,8 @@ __host__ __device__ constexpr int smem_split(int kt, int na, int nb)
 }
 
 template <int KT, int NA, int NB>
-__device__ __forceinline__ void partial_split_body(int bx, int by, const half_args &ha, float *__restrict__ smem)
+__device__ __forceinline__ void partial_split_body(int bx, int by, const half_args &ha, float *__restrict__ smem,
+						   uint32_t stop = 0)
 {
 	static_assert(KT == 16 || KT % 32 == 0, "split body: KT 16, or whole 32-column chunks");
 	constexpr int H = KT / 16;
@@ -1610,6 +1637,8 @@ __device__ __forceinline__ void partial_split_body(int bx, int by, const half_ar
 				fetch_b(blk_row(d), br[d]);
 		}
 	}
+	if (stopped(stop))
+		return;
 
 	// GEMM1's A operands.
 	bf16x8 aq[4][CH][NQ];
@@ -1788,13 +1817,12 @@ __global__ __launch_bounds__(64 * NA * NB, (KT <= 32 ? 3 : 2)) void k_partial_sp
 {
 	constexpr int LDS = max2(smem_split(KT, NA, NB), smem_finish(KT, 64 * NA));
 	__shared__ __align__(16) float smem[LDS];
-	if (st != nullptr && st->converged)
-		return;
+	const uint32_t stop = read_stop(st);
 	int bx, by;
-	if (!half_tile<KT, true, LDS>(h, f, smem, bx, by))
+	if (!half_tile<KT, true, LDS>(h, f, smem, stop, bx, by))
 		return;
-	partial_split_body<KT, NA, NB>(bx, by, h, smem);
-	if (h.part == nullptr)
+	partial_split_body<KT, NA, NB>(bx, by, h, smem, stop);
+	if (h.part == nullptr && !stopped(stop))
 		finish_rows<KT, true, 64 * NA * NB>(bx, 64 * NA, h, f, smem);
 }
 
@@ -1806,9 +1834,8 @@ __global__ __launch_bounds__(NMFK_WG) void k_finish(const float *__restrict__ pa
 						    const nmfk_state *__restrict__ st, __bf16 *__restrict__ Ab)
 {
 	__shared__ float smem[smem_fin(KT)];
-	if (st != nullptr && st->converged)
-		return;
-	finish_block<KT, PAIR, false, true>(blockIdx.x, threadIdx.x, part, S, A, p, k, den, colA, clamp, Ab, smem);
+	const uint32_t stop = read_stop(st);
+	finish_block<KT, PAIR, false, true>(blockIdx.x, threadIdx.x, part, S, A, p, k, den, colA, clamp, Ab, smem, stop);
 }
 
 template <int KT, bool PAIR>
@@ -2443,31 +2470,35 @@ __device__ __forceinline__ void test_rows_body(int bx, float *__restrict__ H, in
 	}
 }
 
-// tab: NMFK_KMAX * NMFK_KMAX uint32 of LDS; red: 2 * (NMFK_WG / 64) uint64 of LDS.
-__device__ __forceinline__ void test_final_body(int m, const uint32_t *__restrict__ cls, uint32_t *__restrict__ last,
+#define NMFK_TEST_TAB (NMFK_KMAX * (NMFK_KMAX + 1))
+
+// tab: NMFK_TEST_TAB uint32 of LDS; red: 2 * (NMFK_WG / 64) uint64 of LDS.
+// The table has k rows of k | 1 (one lane per row or column adds without bank conflicts).
+__device__ __forceinline__ void test_final_body(int m, int k, const uint32_t *__restrict__ cls, uint32_t *__restrict__ last,
 						nmfk_state *__restrict__ st, uint32_t *__restrict__ tab,
 						unsigned long long *__restrict__ red)
 {
 	constexpr int NWV = NMFK_WG / 64;
-	for (int e = threadIdx.x; e < NMFK_KMAX * NMFK_KMAX; e += NMFK_WG)
+	const int ks = k | 1, nt = k * ks;
+	for (int e = threadIdx.x; e < nt; e += NMFK_WG)
 		tab[e] = 0;
 	__syncthreads();
 	for (int j = threadIdx.x; j < m; j += NMFK_WG) {
 		const uint32_t c = cls[j], l = last[j];
 		last[j] = c;
-		atomicAdd(&tab[c * NMFK_KMAX + l], 1u);
+		atomicAdd(&tab[c * ks + l], 1u);
 	}
 	__syncthreads();
 	unsigned long long both = 0, t = 0;
-	for (int e = threadIdx.x; e < NMFK_KMAX * NMFK_KMAX; e += NMFK_WG) {
+	for (int e = threadIdx.x; e < nt; e += NMFK_WG) {
 		const unsigned long long v = tab[e];
 		both += v * (v - (v > 0)) / 2;
 	}
-	if (threadIdx.x < NMFK_KMAX) {
+	if (threadIdx.x < (uint32_t)k) {
 		unsigned long long r = 0, c = 0;
-		for (int b = 0; b < NMFK_KMAX; b++) {
-			r += tab[threadIdx.x * NMFK_KMAX + b];
-			c += tab[b * NMFK_KMAX + threadIdx.x];
+		for (int b = 0; b < k; b++) {
+			r += tab[threadIdx.x * ks + b];
+			c += tab[b * ks + threadIdx.x];
 		}
 		t = r * (r - (r > 0)) / 2 + c * (c - (c > 0)) / 2;
 	}
@@ -2511,14 +2542,14 @@ __global__ __launch_bounds__(NMFK_WG) void k_test_rows(float *__restrict__ H, in
 	test_rows_body(blockIdx.x, H, m, k, kt, cls);
 }
 
-__global__ __launch_bounds__(NMFK_WG) void k_test_final(int m, const uint32_t *__restrict__ cls,
+__global__ __launch_bounds__(NMFK_WG) void k_test_final(int m, int k, const uint32_t *__restrict__ cls,
 							uint32_t *__restrict__ last, nmfk_state *__restrict__ st)
 {
-	__shared__ uint32_t tab[NMFK_KMAX * NMFK_KMAX];
+	__shared__ uint32_t tab[NMFK_TEST_TAB];
 	__shared__ unsigned long long red[2 * (NMFK_WG / 64)];
 	if (st->converged)
 		return;
-	test_final_body(m, cls, last, st, tab, red);
+	test_final_body(m, k, cls, last, st, tab, red);
 }
 
 // --------------------------------------------------------------------------------------
@@ -2704,13 +2735,13 @@ __global__ __launch_bounds__(NMFK_WG) void k_batch_test_rows(const nmfk_bjob *__
 
 __global__ __launch_bounds__(NMFK_WG) void k_batch_test_final(const nmfk_bjob *__restrict__ jobs, int njobs)
 {
-	__shared__ uint32_t tab[NMFK_KMAX * NMFK_KMAX];
+	__shared__ uint32_t tab[NMFK_TEST_TAB];
 	__shared__ unsigned long long red[2 * (NMFK_WG / 64)];
 	for (int t = blockIdx.x; t < njobs; t += gridDim.x) {
 		const nmfk_bjob &J = jobs[t];
 		if (!J.live || J.st->converged)
 			continue;
-		test_final_body(J.m, J.cls, J.last, J.st, tab, red);
+		test_final_body(J.m, J.k, J.cls, J.last, J.st, tab, red);
 		__syncthreads();
 	}
 }
@@ -3576,7 +3607,8 @@ extern "C" int nmfk_launch_test(float *H, uint32_t m, uint32_t k, uint32_t kt, u
 	const unsigned g = (m + NMFK_TEST_ROWS - 1) / NMFK_TEST_ROWS;
 	hipLaunchKernelGGL(k_test_rows, dim3(g), dim3(NMFK_WG), 0, stream, H, (int)m, (int)k, (int)kt, cls,
 			   (const nmfk_state *)st);
-	hipLaunchKernelGGL(k_test_final, dim3(1), dim3(NMFK_WG), 0, stream, (int)m, (const uint32_t *)cls, last, st);
+	hipLaunchKernelGGL(k_test_final, dim3(1), dim3(NMFK_WG), 0, stream, (int)m, (int)k,
+			   (const uint32_t *)cls, last, st);
 	return (int)hipGetLastError();
 }
 
