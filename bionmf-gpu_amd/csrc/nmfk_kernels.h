@@ -176,7 +176,8 @@ typedef struct nmfk_bjob {
 } nmfk_bjob;
 
 typedef struct nmfk_tile {
-	uint32_t job, bx, by, pad_;
+	uint32_t job, bx, by;
+	uint32_t part;        /* which eighth of the job's V the tile reads (see the host's spread_tiles) */
 } nmfk_tile;
 
 /* Largest padded rank a batched launch handles (its LDS is sized for it). */
@@ -189,6 +190,11 @@ typedef struct nmfk_tile {
  * other classes are skipped. */
 int nmfk_launch_batch_partial(const nmfk_bjob *jobs, const nmfk_tile *tiles, uint32_t ntiles, int half,
 			      int cls, uint32_t grid, hipStream_t stream);
+/* Half-steps of one split over at most NMFK_SHORT_Q rows (kt 16, matrix cores in 1 x 4 waves, not
+ * on split products), finishes included; a tile is a row group of the job's own grid, one wave. */
+#define NMFK_SHORT_Q 256
+int nmfk_launch_batch_short(const nmfk_bjob *jobs, const nmfk_tile *tiles, uint32_t ntiles, int half,
+			    int clamp, uint32_t grid, hipStream_t stream);
 int nmfk_launch_batch_finish(const nmfk_bjob *jobs, const nmfk_tile *tiles, uint32_t ntiles, int half,
 			     int clamp, uint32_t grid, hipStream_t stream);
 /* Test: rows tiles (job, row block of NMFK_TEST_ROWS), then one final workgroup per job. */

@@ -185,6 +185,25 @@ __host__ __device__ constexpr int fin_q(int kt)
 }
 static_assert(NMFK_FIN_ROWS * 4 == NMFK_WG, "finish block shape");
 
+// Ascending sum of a column of NMFK_FIN_ROWS values of LDS, <stride> apart.  The reads of half a
+// column go out before its additions: left to itself the compiler keeps three in flight.
+__device__ __forceinline__ float column_sum(const float *col, int stride)
+{
+	float s = 0.0f;
+#pragma unroll
+	for (int r0 = 0; r0 < NMFK_FIN_ROWS; r0 += 32) {
+		float v[32];
+#pragma unroll
+		for (int r = 0; r < 32; r++)
+			v[r] = col[(r0 + r) * stride];
+		__builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+		for (int r = 0; r < 32; r++)
+			s += v[r];
+	}
+	return s;
+}
+
 // tid: the thread's index among the block's NMFK_WG threads; out: null where the block has no
 // rows.  tile: NMFK_FIN_ROWS x (KT + 1) floats of LDS.  PAIR: NMFK_WG / KT groups of threads add
 // consecutive rows each, then one thread per column adds the groups.
@@ -218,10 +237,7 @@ __device__ __forceinline__ void block_colsum_store(int tid, const float (&x)[fin
 		return;
 	}
 	if (tid < KT && out != nullptr) {
-		float s = 0.0f;
-		for (int r = 0; r < NMFK_FIN_ROWS; r++)
-			s += tile[r * (KT + 1) + tid];
-		out[tid] = s;
+		out[tid] = column_sum(tile + tid, KT + 1);
 	}
 }
 
@@ -469,14 +485,11 @@ __device__ __forceinline__ void finish_block(int blk, int tid, const float *__re
 			operands();
 #pragma unroll
 		for (int i = 0; i < Q; i++) {
-			float v = 0.0f;
-			if (c0 + i < k) {
-				v = ar[i] * s[i];
-				v = v / dn[i];
-				if (clamp)
-					v = clamp_rmin(v);
-			}
-			x[i] = v;
+			float v = ar[i] * s[i];
+			v = v / dn[i];   // without a branch, so that a thread's divisions overlap
+			if (clamp)
+				v = clamp_rmin(v);
+			x[i] = c0 + i < k ? v : 0.0f;
 		}
 	} else {
 #pragma unroll
@@ -1817,7 +1830,7 @@ __global__ __launch_bounds__(64 * NA * NB, (KT <= 32 ? 3 : 2)) void k_partial_sp
 {
 	constexpr int LDS = max2(smem_split(KT, NA, NB), smem_finish(KT, 64 * NA));
 	__shared__ __align__(16) float smem[LDS];
-	const uint32_t stop = read_stop(st);
+	const uint32_t stop = st != nullptr ? st->converged : 0u;   // (its registers are all taken: 2% at kt 32)
 	int bx, by;
 	if (!half_tile<KT, true, LDS>(h, f, smem, stop, bx, by))
 		return;
@@ -2593,6 +2606,256 @@ __device__ __forceinline__ fin_args batch_fin(const nmfk_bjob &J, int half, int 
 	f.k = J.k;
 	f.clamp = hh ? 0 : clamp;
 	return f;
+}
+
+// --------------------------------------------------------------------------------------
+// Batched half-steps of one split over a short range of U (q <= NMFK_SHORT_Q rows, kt 16 in 1 x 4
+// waves): the W halves of a rank sweep over a matrix of few columns.  As workgroups these tiles
+// are all beginning and end: each wave of a workgroup has 3 or 4 blocks of 16 rows between the
+// loads of its operands and the LDS step, and the partial sums go through memory to a second
+// launch.  Here a wave takes all blocks of its own 64 rows a and finishes them, without a
+// barrier: no launch, no partial sums, a fourth of the operand loads, and waves that drift
+// apart keep the matrix cores busy.  The blocks are walked in the order that gives the bits of
+// the 1 x 4 workgroup: blocks g, g + 4, ... of each of the four wave groups in turn, each
+// group's sums added to the total in that order.  54 jobs at 5000 x 200,
+// k = 2..10: W sums 51 us and finishes 20 us -> 38.5 us, of which the matrix cores are busy 44%.
+// --------------------------------------------------------------------------------------
+
+#define NMFK_SHORT_LDS (64 * 17 + 16)   // floats per wave: its rows' sums, and the denominators
+
+// What a lane of a wave wrote to LDS before, the others read after.
+__device__ __forceinline__ void wave_lds_fence()
+{
+	__builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+	__builtin_amdgcn_wave_barrier();
+}
+
+template <int KE>
+__device__ __forceinline__ void short_body(int bx, const half_args &ha, const fin_args &f, float *__restrict__ tile)
+{
+	constexpr int KT = 16, QN = KE >= 16 ? 4 : KE / 4, TS = KT + 1;
+	constexpr bool G2N = KE <= NMFK_G2N_MAX_KE;
+	static_assert(!G2N || QN == 1, "one GEMM2 operand per row");
+	const int lane = threadIdx.x & 63, j = lane & 15, g = lane >> 4;
+	const int p = ha.p, q = ha.q, a0 = bx * 64, aj = a0 + 4 * j, avail = p - aj;
+	const int ucol = avail > 0 ? aj : 0, c2 = G2N ? j & 3 : j;
+	const size_t ldu = ha.ldu;
+
+	// Operands as in partial_mfma_body; rows of a block at or past q read as zero.
+	floatx4 aop[4];
+#pragma unroll
+	for (int t = 0; t < 4; t++) {
+		const bool ok = t < avail;
+		const float4 v = loadq<QN>(ha.A + (size_t)(ok ? aj + t : 0) * KT + QN * g);
+		aop[t] = ok ? floatx4{v.x, v.y, v.z, v.w} : floatx4{0.f, 0.f, 0.f, 0.f};
+	}
+	struct blk {
+		float4 u[4], b1;
+		float b2[4];
+	};
+	int uoff[4], b2off[4];
+#pragma unroll
+	for (int r = 0; r < 4; r++) {
+		uoff[r] = ((4 * g + r) * (int)ldu + ucol) * 4;
+		b2off[r] = ((4 * g + r) * KT + c2) * 4;
+	}
+	const int b1off = (j * KT + QN * g) * 4;
+	auto load = [&](int i, blk &x) {
+		const int bb = 16 * i, rows = min(16, q - bb);
+		const __amdgpu_buffer_rsrc_t rU = make_rsrc(ha.U + (size_t)bb * ldu, (size_t)rows * ldu * 4);
+		const __amdgpu_buffer_rsrc_t rB = make_rsrc(ha.B + (size_t)bb * KT, (size_t)rows * KT * 4);
+		x.b1 = bloadq<QN>(rB, b1off);   // the first to be used
+#pragma unroll
+		for (int r = 0; r < 4; r++)
+			x.u[r] = bload4(rU, uoff[r], 0);
+#pragma unroll
+		for (int r = 0; r < 4; r++)
+			x.b2[r] = bload1(rB, b2off[r], 0);
+	};
+	auto gemm1 = [&](const blk &x, floatx4 (&s)[4]) {
+#pragma unroll
+		for (int qq = 0; qq < QN; qq++) {
+			const float bv = qq == 0 ? x.b1.x : qq == 1 ? x.b1.y : qq == 2 ? x.b1.z : x.b1.w;
+#pragma unroll
+			for (int t = 0; t < 4; t++)
+				s[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(
+					bv, aop[t][qq], qq == 0 ? floatx4{0.f, 0.f, 0.f, 0.f} : s[t], 0, 0, 0);
+		}
+	};
+	auto ratio = [&](const blk &x, const floatx4 (&s)[4], float (&rt)[4][4], int i) {
+#pragma unroll
+		for (int r = 0; r < 4; r++) {
+			const float uv[4] = {x.u[r].x, x.u[r].y, x.u[r].z, x.u[r].w};
+#pragma unroll
+			for (int t = 0; t < 4; t++)
+				rt[t][r] = uv[t] * __builtin_amdgcn_rcpf(s[t][r]);
+		}
+		if (16 * i + 16 > q) {
+#pragma unroll
+			for (int r = 0; r < 4; r++)
+#pragma unroll
+				for (int t = 0; t < 4; t++)
+					rt[t][r] = 16 * i + 4 * g + r < q ? rt[t][r] : 0.0f;
+		}
+	};
+
+	floatx4 acc[4];
+	float tot[4] = {0.f, 0.f, 0.f, 0.f};   // G2N: the lane's 4 sums; else they are in tile
+#pragma unroll
+	for (int t = 0; t < 4; t++)
+		acc[t] = floatx4{0.f, 0.f, 0.f, 0.f};
+	auto gemm2 = [&](const blk &x, const float (&rt)[4][4]) {
+#pragma unroll
+		for (int r = 0; r < 4; r++)
+#pragma unroll
+			for (int t = 0; t < 4; t++) {
+				if constexpr (G2N)
+					acc[t] = __builtin_amdgcn_mfma_f32_4x4x1f32(rt[t][r], x.b2[r], acc[t], 0, 0, 0);
+				else
+					acc[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(rt[t][r], x.b2[r], acc[t], 0, 0, 0);
+			}
+	};
+	// The end of wave group <grp>: its sums join the total.
+	auto close = [&](int grp) {
+#pragma unroll
+		for (int t = 0; t < 4; t++) {
+			if constexpr (G2N) {
+				// as partial_mfma_body: the lane groups' sums, component i = g left in lane group g
+				const bool hi = (g & 2) != 0, odd = (g & 1) != 0;
+				const floatx4 v = acc[t];
+				const float k0 = hi ? v[2] : v[0], k1 = hi ? v[3] : v[1];
+				const float s0 = hi ? v[0] : v[2], s1 = hi ? v[1] : v[3];
+				const float e0 = k0 + __shfl_xor(s0, 32), e1 = k1 + __shfl_xor(s1, 32);
+				const float o = (odd ? e1 : e0) + __shfl_xor(odd ? e0 : e1, 16);
+				tot[t] = grp == 0 ? o : tot[t] + o;
+			}
+		}
+		if constexpr (!G2N) {
+			float *d = tile + 16 * g * TS + j;   // row 4 (4 g + r) + t
+			if (grp > 0) {
+				float o[4][4];
+#pragma unroll
+				for (int t = 0; t < 4; t++)
+#pragma unroll
+					for (int r = 0; r < 4; r++)
+						o[t][r] = d[(4 * r + t) * TS];
+#pragma unroll
+				for (int t = 0; t < 4; t++)
+#pragma unroll
+					for (int r = 0; r < 4; r++)
+						acc[t][r] = o[t][r] + acc[t][r];
+			}
+#pragma unroll
+			for (int t = 0; t < 4; t++)
+#pragma unroll
+				for (int r = 0; r < 4; r++)
+					d[(4 * r + t) * TS] = acc[t][r];
+		}
+#pragma unroll
+		for (int t = 0; t < 4; t++)
+			acc[t] = floatx4{0.f, 0.f, 0.f, 0.f};
+	};
+
+	// Blocks in group order; a block past the last is the last again, and its products unused.
+	const int nb = (q + 15) / 16;
+	auto next = [&](int i) { return i + 4 < nb ? i + 4 : (i & 3) + 1 < min(nb, 4) ? (i & 3) + 1 : i; };
+	blk ring[2];
+	int cur = 0, nxt = next(0);
+	load(cur, ring[0]);
+	load(nxt, ring[1]);
+	float rt[4][4];
+	{
+		floatx4 s[4];
+		gemm1(ring[0], s);
+		ratio(ring[0], s, rt, cur);
+	}
+	for (int n = 0; n < nb; n += 2) {
+#pragma unroll
+		for (int d = 0; d < 2; d++) {
+			if (n + d < nb) {
+				floatx4 s[4];
+				const int after = next(nxt);
+				gemm1(ring[d ^ 1], s);
+				gemm2(ring[d], rt);
+				load(after, ring[d]);
+				ratio(ring[d ^ 1], s, rt, nxt);
+				if (cur + 4 >= nb)
+					close(cur & 3);
+				cur = nxt, nxt = after;
+			}
+		}
+	}
+	if constexpr (G2N) {
+#pragma unroll
+		for (int t = 0; t < 4; t++)
+			tile[(16 * (j >> 2) + 4 * g + t) * TS + c2] = tot[t];
+	}
+
+	// The finish (finish_block) by one wave: lane t sums row-interleaved quarter t & 3 of column
+	// t >> 2 of B's column-sum partials, as den_reduce, then a lane takes a row of A.
+	float *dn = tile + 64 * TS;
+	float z = 0.0f;
+	for (int i = lane & 3; i < f.ncolB; i += 4)
+		z += f.colB[(size_t)i * KT + (lane >> 2)];
+	const float z1 = __shfl(z, (lane & ~3) + 1), z2 = __shfl(z, (lane & ~3) + 2), z3 = __shfl(z, (lane & ~3) + 3);
+	if ((lane & 3) == 0)
+		dn[lane >> 2] = ((z + z1) + z2) + z3;
+	wave_lds_fence();
+	const int a = a0 + lane;
+	float x[KT];
+	if (a < p) {
+		float *Ar = f.A + (size_t)a * KT;
+		ldq<KT>(Ar, x);
+#pragma unroll
+		for (int c = 0; c < KT; c++) {
+			float v = 0.0f;
+			if (c < f.k) {
+				v = x[c] * tile[lane * TS + c];
+				v = v / dn[c];
+				if (f.clamp)
+					v = clamp_rmin(v);
+			}
+			x[c] = v;
+		}
+		stq<KT>(Ar, x);
+	} else {
+#pragma unroll
+		for (int c = 0; c < KT; c++)
+			x[c] = 0.0f;
+	}
+#pragma unroll
+	for (int c = 0; c < KT; c++)
+		tile[lane * TS + c] = x[c];
+	wave_lds_fence();
+	if (lane < KT) {
+		f.colA[(size_t)bx * KT + lane] = column_sum(tile + lane, TS);
+	}
+}
+
+// One wave per workgroup and tile.
+__global__ __launch_bounds__(64, 3) void k_batch_short(const nmfk_bjob *__restrict__ jobs,
+							   const nmfk_tile *__restrict__ tiles, int ntiles, int half, int clamp)
+{
+	__shared__ __align__(16) float tile[NMFK_SHORT_LDS];
+	for (int t = blockIdx.x; t < ntiles; t += gridDim.x) {
+		const nmfk_tile tl = tiles[t];
+		const nmfk_bjob &J = jobs[tl.job];
+		const int bx = (int)tl.bx;
+		if (!J.live || J.st->converged)
+			continue;
+		const half_args h = batch_half(J, half);
+		if (J.kt != 16 || bx >= h.nab || h.S != 1 || h.q > NMFK_SHORT_Q)
+			continue;
+		const fin_args f = batch_fin(J, half, clamp);
+		const uint32_t ke = half == 0 ? J.planH.ke : J.planW.ke;
+		if (ke == 4)
+			short_body<4>(bx, h, f, tile);
+		else if (ke == 8)
+			short_body<8>(bx, h, f, tile);
+		else
+			short_body<16>(bx, h, f, tile);
+		wave_lds_fence();   // the next tile reuses the LDS
+	}
 }
 
 // VALU body of a batched half-step with lane groups (2, 4 or 8, from its plan).
@@ -3659,6 +3922,16 @@ extern "C" int nmfk_launch_batch_partial(const nmfk_bjob *jobs, const nmfk_tile 
 	default:
 		return (int)hipErrorInvalidValue;
 	}
+	return (int)hipGetLastError();
+}
+
+extern "C" int nmfk_launch_batch_short(const nmfk_bjob *jobs, const nmfk_tile *tiles, uint32_t ntiles, int half,
+				       int clamp, uint32_t grid, hipStream_t stream)
+{
+	if (ntiles == 0)
+		return 0;
+	hipLaunchKernelGGL(k_batch_short, dim3(batch_grid(ntiles, grid)), dim3(64), 0, stream, jobs, tiles,
+			   (int)ntiles, half, clamp);
 	return (int)hipGetLastError();
 }
 

@@ -259,3 +259,26 @@ def test_jobs_are_not_freed_under_a_batch_or_a_sharer(nmfk, orc):
     other.close()                    # the batch goes first: the job may then be freed
     j.close()
     batch.close()
+
+
+@pytest.mark.parametrize("m", [32, 33, 47, 64, 65, 200, 255, 256, 257])
+def test_short_half_steps_same_bits_as_alone(nmfk, orc, m):
+    # W halves of one split over at most 256 rows run one wave per 64 rows in a batch, finish
+    # included; each must give the bits of the job alone: all three GEMM1 widths, one to sixteen
+    # blocks of 16 rows (the last one partial), partly filled row groups, a test pass with its
+    # clamp, and 257 rows, which stay with the workgroups.
+    specs = [(700 + 37 * k, m, k, 30 + k, 40 + k, 20, 1000) for k in (2, 4, 5, 8, 9, 16)]
+    pairs = [twins(nmfk, orc, s) for s in specs]
+    for a, b in pairs:
+        for j in (a, b):
+            j.replan(1)
+            assert j.plan()["W"]["S"] == 1
+    batch = nmfk.Batch(T, 8)
+    for (a, _), s in zip(pairs, specs):
+        batch.add(a, s[5], s[6])
+    done = dict((id(j), r) for j, r in batch.run())
+    for (a, b), s in zip(pairs, specs):
+        assert_same(a, b, done[id(a)], b.run(s[5], T, s[6]), s)
+    batch.close()
+    for a, b in pairs:
+        a.close(), b.close()
