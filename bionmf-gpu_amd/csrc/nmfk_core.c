@@ -329,7 +329,9 @@ nmfk_job *nmfk_job_create_shared(nmfk_job *src, uint32_t k)
 }
 
 /* Jobs planned on their own (no workgroup target) may run on split products; a job replanned
- * to a target, as the sweep and the serving loop do, keeps the FP32 instructions. */
+ * to a target, as the sweep and the serving loop do, keeps the FP32 instructions: on
+ * split products a burst of 33 served jobs ran 10% faster, but came out 0-15% further from 64 bits
+ * over four seeds. */
 static void set_split(nmfk_job *j, uint32_t target_wgs)
 {
 	j->split = target_wgs == 0 && j->planH.path == NMFK_PATH_MFMA32 && j->planW.path == NMFK_PATH_MFMA32 &&
@@ -737,20 +739,28 @@ int nmfk_job_get_H(nmfk_job *j, float *H, size_t ldh)
 
 /* Half-step <half>: 0 = H through V against W, 1 = W through Vt against H.  Finishing it updates
  * the factor, its column-sum partials (the other half's denominators) and its BF16 copy where
- * the other half reads that.  what: the whole half-step, or for timing its sums or its finish. */
-enum { HALF_WHOLE, HALF_SUMS, HALF_FINISH };
+ * the other half reads that.  what: the whole half-step; a lone one, for which nothing is known of
+ * the other factor's column sums; or for timing its sums or its finish. */
+enum { HALF_WHOLE, HALF_LONE, HALF_SUMS, HALF_FINISH };
 
 static int half_step(nmfk_job *j, int half, int what, int clamp, const nmfk_state *st)
 {
 	const nmfk_hplan *pl = half ? &j->planW : &j->planH, *other = half ? &j->planH : &j->planW;
 	const nmfk_half g = {half ? j->Vt : j->V, half ? j->ldvt : j->ldv, half ? j->W : j->H, half ? j->H : j->W,
 			     half ? j->Hb : j->Wb, half ? j->n : j->m, half ? j->m : j->n, j->kt, j->split, j->part};
-	const nmfk_fin f = {half ? j->W : j->H, half ? j->colW : j->colH,
+	int e;
+	nmfk_fin f = {half ? j->W : j->H, half ? j->colW : j->colH,
 			    other->path != NMFK_PATH_MFMA_BF16 ? NULL : half ? j->Wb : j->Hb, half ? j->colH : j->colW,
 			    half ? j->ncolH : j->ncolW, half ? j->denH : j->denW, j->k, clamp};
 	if (what == HALF_FINISH)
 		return nmfk_launch_finish(j->part, pl->S, g.p, j->kt, j->split, &f, st, j->stream);
-	return nmfk_launch_half(&g, pl, what == HALF_WHOLE ? &f : NULL, st, j->stream);
+	if (what == HALF_LONE) {
+		if (!j->split && g.q <= NMFK_DEN_ROWS)
+			f.colB = NULL;
+		else if ((e = nmfk_launch_colsum_parts(g.B, g.q, j->kt, j->split, half ? j->colH : j->colW, j->stream)) != 0)
+			return e;
+	}
+	return nmfk_launch_half(&g, pl, what != HALF_SUMS ? &f : NULL, st, j->stream);
 }
 
 int nmfk_enqueue_half_H(nmfk_job *j, const nmfk_state *st)
@@ -782,11 +792,9 @@ int nmfk_job_update_H(nmfk_job *j)
 {
 	if (j->streamed)
 		return nmfk_stream_update_H(j);
-	int e = nmfk_launch_colsum_parts(j->W, j->n, j->kt, j->split, j->colW, j->stream);
+	int e = nmfk_job_shadow_for_H(j);
 	if (!e)
-		e = nmfk_job_shadow_for_H(j);
-	if (!e)
-		e = nmfk_enqueue_half_H(j, NULL);
+		e = half_step(j, 0, HALF_LONE, 0, NULL);
 	return nmfk_hip_fail(e, "update_H");
 }
 
@@ -797,11 +805,9 @@ int nmfk_job_update_W(nmfk_job *j)
 		return nmfk_stream_update_W(j);
 	if (nmfk_job_refresh_Vt(j))
 		return NMFK_EHIP;
-	int e = nmfk_launch_colsum_parts(j->H, j->m, j->kt, j->split, j->colH, j->stream);
+	int e = nmfk_job_shadow_for_W(j);
 	if (!e)
-		e = nmfk_job_shadow_for_W(j);
-	if (!e)
-		e = nmfk_enqueue_half_W(j, NULL, 0);
+		e = half_step(j, 1, HALF_LONE, 0, NULL);
 	j->colW_valid = 1;
 	return nmfk_hip_fail(e, "update_W");
 }

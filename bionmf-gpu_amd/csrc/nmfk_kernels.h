@@ -105,12 +105,13 @@ typedef struct nmfk_half {
 typedef struct nmfk_fin {
 	float *A, *colA;
 	uint16_t *Ab;         /* BF16 copy of the new A to keep (kt % 32 == 0), or NULL */
-	const float *colB;
+	const float *colB;    /* NULL: the column sums are taken from B (q <= NMFK_DEN_ROWS, no split products) */
 	uint32_t ncolB;
 	float *den;           /* receives the column sums of B */
 	uint32_t k;
 	int clamp;
 } nmfk_fin;
+#define NMFK_DEN_ROWS 1024
 int nmfk_launch_half(const nmfk_half *g, const nmfk_hplan *pl, const nmfk_fin *fin, const nmfk_state *st,
 		     hipStream_t stream);
 

@@ -171,6 +171,44 @@ __device__ __forceinline__ void den_reduce(const float *__restrict__ parts, int 
 			      : ((s4[4 * t] + s4[4 * t + 1]) + s4[4 * t + 2]) + s4[4 * t + 3];
 }
 
+// The same from B itself (q x KT, q <= NMFK_DEN_ROWS), for a half-step called by itself on factors
+// that may have changed since their column sums were taken: sums of blocks of NMFK_FIN_ROWS rows in
+// ascending order, as k_colsum_parts leaves them, then den_reduce's.  A third of the launches of
+// such a half-step: they are what a program that calls small ones waits for, 3.4 us each.
+template <int KT>
+__device__ __forceinline__ void den_direct(const float *__restrict__ B, int q, float *den, float *__restrict__ s4)
+{
+	static_assert(4 * KT <= NMFK_WG, "den_direct: one thread per (column, lane of 4)");
+	const int t = threadIdx.x, c = t >> 2, j = t & 3, nblk = (q + NMFK_FIN_ROWS - 1) / NMFK_FIN_ROWS;
+	float *buf = s4 + 4 * KT;
+	for (int e = t; e < nblk * KT; e += blockDim.x) {
+		const int b0 = e / KT * NMFK_FIN_ROWS;
+		const float *col = B + (size_t)b0 * KT + e % KT;
+		float s = 0.0f;
+#pragma unroll 1
+		for (int r0 = 0; r0 < NMFK_FIN_ROWS; r0 += 16) {
+			float v[16];
+#pragma unroll
+			for (int r = 0; r < 16; r++)
+				v[r] = b0 + r0 + r < q ? col[(size_t)(r0 + r) * KT] : 0.0f;
+#pragma unroll
+			for (int r = 0; r < 16; r++)
+				s += v[r];
+		}
+		buf[e] = s;
+	}
+	__syncthreads();
+	if (t < 4 * KT) {
+		float s = 0.0f;
+		for (int g = j; g < nblk; g += 4)
+			s += buf[g * KT + c];
+		s4[t] = s;
+	}
+	__syncthreads();
+	if (t < KT)
+		den[t] = ((s4[4 * t] + s4[4 * t + 1]) + s4[4 * t + 2]) + s4[4 * t + 3];
+}
+
 // One finish block = NMFK_FIN_ROWS (64) rows of A with 4 threads per row, each thread
 // KT/4 consecutive columns (NMFK_WG threads).  Column sums of the block's rows (ascending
 // rows) are written as one partial row; shared by the finish and column-sum kernels so
@@ -297,7 +335,7 @@ struct fin_args {
 	float *A;             // p x KT
 	float *colA;          // column sums of the new A per NMFK_FIN_ROWS rows
 	__bf16 *Ab;           // BF16 copy of the new A, or null
-	const float *colB;    // column-sum partials of B, ncolB rows, whose sum divides
+	const float *colB;    // column-sum partials of B, ncolB rows, whose sum divides; null: from B (den_direct)
 	float *den;           // that sum
 	int ncolB, k, clamp;
 };
@@ -550,12 +588,21 @@ __host__ __device__ constexpr int smem_finish(int kt, int rows)
 	return (tile_rows(rows) * (kt + 1) + 3) / 4 * 4 + smem_den(kt) + kt;
 }
 
+template <int KT, bool PAIR>
+__device__ __forceinline__ void denominators(const half_args &h, const fin_args &f, float *den, float *s4, int room)
+{
+	if (!PAIR && f.colB == nullptr)
+		den_direct<KT>(h.B, h.q, den, s4);
+	else
+		den_reduce<KT, PAIR>(f.colB, f.ncolB, den, s4, room);
+}
+
 template <int KT, bool PAIR, int NT>
 __device__ __forceinline__ void finish_rows(int bx, int rows, const half_args &h, const fin_args &f, float *smem)
 {
 	constexpr int PP = NT / NMFK_WG;   // blocks at a time
 	float *s4 = smem + (tile_rows(rows) * (KT + 1) + 3) / 4 * 4, *den = s4 + smem_den(KT);
-	den_reduce<KT, PAIR>(f.colB, f.ncolB, den, s4, 32 * KT);
+	denominators<KT, PAIR>(h, f, den, s4, 32 * KT);
 	__syncthreads();
 	if (bx == 0 && threadIdx.x < KT)
 		f.den[threadIdx.x] = den[threadIdx.x];
@@ -580,7 +627,7 @@ __device__ __forceinline__ bool half_tile(const half_args &h, const fin_args &f,
 	if (bx < h.nab)
 		return true;
 	if (by == 0 && f.den != nullptr && !stopped(stop))
-		den_reduce<KT, PAIR>(f.colB, f.ncolB, f.den, smem, ROOM - 4 * KT);
+		denominators<KT, PAIR>(h, f, f.den, smem, ROOM - 4 * KT);
 	return false;
 }
 
@@ -3595,6 +3642,8 @@ static bool kernel_args(const nmfk_half *g, const nmfk_hplan *pl, const nmfk_fin
 	if (fin)
 		*f = fin_args{fin->A, fin->colA, (__bf16 *)fin->Ab, fin->colB, fin->den, (int)fin->ncolB, (int)fin->k, fin->clamp};
 	*grid = dim3(((own ? pl->nab : pl->nab + 1) * pl->S + 7u) & ~7u);
+	if (fin && fin->colB == nullptr && (g->split || g->q > NMFK_DEN_ROWS))
+		return false;
 	return g->part != nullptr && !(own && rows % NMFK_FIN_ROWS != 0 && pl->nab != 1);
 }
 

@@ -200,6 +200,22 @@ def test_one_split_finishes_in_its_launch(nmfk, orc, n, m, k, path, na, nb):
         nmfk.tune_set(nmfk.TUNE_MFMA_NB, old[1])
 
 
+@pytest.mark.parametrize("n,m,k,path", [(64, 33, 3, 2), (65, 1025, 7, 2), (1024, 63, 12, 2), (1025, 1024, 30, 2), (1023, 40, 5, 1),
+                                        (30, 5, 4, 1), (1000, 70, 40, 3), (1024, 1023, 64, 2)])
+def test_lone_half_steps_give_the_bits_of_a_run(nmfk, orc, n, m, k, path):
+    # Half-steps called one by one take their denominators from the factor itself up to 1024 rows,
+    # from its column-sum partials above: in both cases the sums a run's finishes leave behind.
+    jobs = [make_job(nmfk, orc, n, m, k, seed_v=n, seed_init=m)[0] for _ in range(2)]
+    with jobs[0] as a, jobs[1] as b:
+        for j in jobs:
+            j.set_kernel_path(path)
+        a.run(2, 1000, 1000)
+        for _ in range(2):
+            b.update_H()
+            b.update_W()
+        assert np.array_equal(a.get_H(), b.get_H()) and np.array_equal(a.get_W(), b.get_W())
+
+
 def test_golden_tiny_runs(nmfk, orc):
     g = np.load(GOLDEN / "tiny.npz")
     for ci in range(int(g["ncases"])):
