@@ -2488,7 +2488,7 @@ __global__ __launch_bounds__(256) void k_idx_max(const float *__restrict__ A, in
 // Convergence test: adjust(H) + classification + connectivity difference + stop rule
 // (src/NMF_GPU.c:611-708), as two passes.
 //   rows pass: each block clamps NMFK_TEST_ROWS rows of H (written back) and classifies
-//              them (8 rows per wave, loaded together) into cls;
+//              them (2 rows per wave; 8 took 2-4 us longer) into cls;
 //   final pass (one block per job): the contingency table n_ab = #{j : c_j == a, l_j == b}
 //              in LDS, then the difference  #{i<j : [c_i==c_j] != [l_i==l_j]}  as
 //              sum_a C(r_a,2) + sum_b C(s_b,2) - 2 sum_ab C(n_ab,2)  (integer, exact),
