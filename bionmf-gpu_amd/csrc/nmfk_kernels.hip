@@ -328,6 +328,7 @@ struct half_args {
 	float *part;   // null: the one split's sums are left in LDS for finish_rows
 	int S;         // splits of the q rows
 	int lb;        // VALU lane groups (see partial_valu_body)
+	int nt_from;   // BF16: tiles by nab + bx from here on stream U past the last-level cache
 };
 
 // What turns a half-step's partial sums into the new A (see finish_rows).
@@ -1301,7 +1302,7 @@ struct bf16_args {
 	const __bf16 *Bb;    // q x KT, row-major
 };
 
-template <int KT, int NA, int NB>
+template <int KT, int NA, int NB, bool NT>
 __device__ __forceinline__ void partial_bf16_body(int bx, int by, const half_args &ha, const bf16_args &bb16,
 						  float *__restrict__ smem,
 						  uint32_t stop)
@@ -1447,7 +1448,9 @@ __device__ __forceinline__ void partial_bf16_body(int bx, int by, const half_arg
 				int b = bb + 16 * hb + 4 * g + r;
 				if (!full)
 					b = b < b_end ? b : b_begin;
-				u[hb][r] = *reinterpret_cast<const float4 *>(U + (size_t)b * ldu + ucol);
+				const floatx4 *src = reinterpret_cast<const floatx4 *>(U + (size_t)b * ldu + ucol);
+				const floatx4 v = NT ? __builtin_nontemporal_load(src) : *src;
+				u[hb][r] = make_float4(v[0], v[1], v[2], v[3]);
 			}
 	};
 
@@ -1510,7 +1513,10 @@ __global__ __launch_bounds__(64 * NA * NB) void k_partial_bf16(half_args h, bf16
 	int bx, by;
 	if (!half_tile<KT, false, LDS>(h, f, smem, stop, bx, by))
 		return;
-	partial_bf16_body<KT, NA, NB>(bx, by, h, b, smem, stop);
+	if (by * h.nab + bx < h.nt_from)
+		partial_bf16_body<KT, NA, NB, false>(bx, by, h, b, smem, stop);
+	else
+		partial_bf16_body<KT, NA, NB, true>(bx, by, h, b, smem, stop);
 	if (h.part == nullptr && !stopped(stop))
 		finish_rows<KT, false, 64 * NA * NB>(bx, 64 * NA, h, f, smem);
 }
@@ -3629,6 +3635,20 @@ extern "C" void nmfk_plan_half(uint32_t p, uint32_t q, uint32_t kt, nmfk_hplan *
 	nmfk_plan_half_path(p, q, kt, NMFK_PATH_AUTO, pl);
 }
 
+// Tiles of a BF16 half-step that read U through the last-level cache (256 MB): all where V and
+// Vt fit it together, else the first so many that read 112 MB of each.  These stay there from one
+// iteration to the next, since the others, loaded as non-temporal, do not displace them; read in
+// turn without that, V and Vt displace each other and nothing is found again.  Per iteration, all
+// cached / 112 MB: 50000 x 2000, k = 64 183.4 / 172.5 us (64 MB 174, 96 MB 172, 128 MB 175, none
+// 177); 20000 x 3000, k = 40 155.0 / 152.1; 50000 x 1000, k = 64 132.6 / 130.2; 40000 x 1000, k = 48
+// even.  Where both fit, loads past the cache lose: 30000 x 1000, k = 48 85 / 105 us.
+#define NMFK_CACHED_BYTES ((size_t)112 << 20)
+static int cached_tiles(const nmfk_hplan *pl, size_t bytes)
+{
+	const uint32_t tiles = pl->nab * pl->S;
+	return bytes <= ((size_t)128 << 20) ? (int)tiles : (int)((double)tiles * NMFK_CACHED_BYTES / bytes);
+}
+
 // Kernel arguments and grid (padded to a multiple of 8, see xcd_tile) of a half-step; fin may be
 // null (partial sums only).  Workgroups that finish <rows> rows themselves take whole blocks of
 // rows, or all of them.
@@ -3637,7 +3657,7 @@ static bool kernel_args(const nmfk_half *g, const nmfk_hplan *pl, const nmfk_fin
 {
 	const bool own = fin && pl->S == 1;
 	*h = half_args{g->U, g->ldu, g->A, g->B, (int)g->p, (int)g->q, (int)pl->bchunk, (int)pl->nab, own ? nullptr : g->part,
-		       (int)pl->S, (int)pl->lb};
+		       (int)pl->S, (int)pl->lb, cached_tiles(pl, (size_t)g->q * g->ldu * 4)};
 	*f = fin_args{};
 	if (fin)
 		*f = fin_args{fin->A, fin->colA, (__bf16 *)fin->Ab, fin->colB, fin->den, (int)fin->ncolB, (int)fin->k, fin->clamp};
