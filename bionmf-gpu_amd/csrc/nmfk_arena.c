@@ -1,5 +1,5 @@
 /*
- * nmfk_arena.c -- device memory arena of the serving loop.
+ * nmfk_arena.c -- device memory arena of the serving loop and of a rank sweep.
  *
  * The serving loop creates and retires thousands of jobs.  With one hipMalloc per buffer
  * and one hipFree per buffer at retirement, the host thread that keeps the device busy
@@ -9,7 +9,7 @@
  * runtime before nmfk_arena_destroy, except by an explicit nmfk_arena_trim.  Blocks are
  * 256-byte aligned.
  *
- * Not thread-safe: one arena per serving loop, used from its host thread.
+ * Not thread-safe: one arena per serving loop or sweep, used from its host thread.
  */
 #include "nmfk_internal.h"
 
