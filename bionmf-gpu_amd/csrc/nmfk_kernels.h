@@ -223,6 +223,10 @@ int nmfk_launch_gen_planted(float *V, uint32_t n, uint32_t m, uint32_t ldv, uint
 int nmfk_launch_transpose(const float *V, uint32_t n, uint32_t m, size_t ldv, float *Vt, size_t ldvt,
 			  hipStream_t stream);
 
+/* Whether the byte offsets of 16 rows of <ldu> floats fit in the 31 bits of one buffer descriptor,
+ * as the kernels that read 16-row blocks through one address them (up to 33.5 million columns). */
+int nmfk_rows16_fit(size_t ldu);
+
 /* Per-block FP64 partial sums {sum V^2, sum (V-WH)^2, sum V log(V/WH) - V + WH}. */
 uint32_t nmfk_dot_kl_blocks(uint32_t n, uint32_t m);
 int nmfk_launch_dot_kl(const float *V, size_t ldv, const float *W, const float *H, uint32_t n,

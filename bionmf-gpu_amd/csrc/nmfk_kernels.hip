@@ -3248,7 +3248,9 @@ __device__ __forceinline__ double log_ratio(float v, double wh)
 	return fma(ed, 0x1.62e42fefa3800p-1, fma(ed, 0x1.ef35793c76730p-45, a));
 }
 
-template <int KT>
+// WIDE: rows so long that 16 of them pass a buffer's 2 GiB of 32-bit offsets (nmfk_rows16_fit); V is then
+// read through 64-bit addresses, a value at a time.
+template <int KT, bool WIDE>
 __global__ __launch_bounds__(64 * dot_waves(KT)) void k_dot_kl(const float *__restrict__ V, size_t ldv,
 							       const float *__restrict__ W, const float *__restrict__ H,
 							       int n, int m, double *__restrict__ parts)
@@ -3284,12 +3286,24 @@ __global__ __launch_bounds__(64 * dot_waves(KT)) void k_dot_kl(const float *__re
 			float w[KQ];
 		};
 		auto load = [&](int ib, blk &x) {
-			const int rows = min(16, i1 - ib);
-			const size_t row = (size_t)ib * ldv;
-			const __amdgpu_buffer_rsrc_t rv = make_rsrc(V + row, ((size_t)(rows - 1) * ldv + m) * 4);
+			if constexpr (WIDE) {
 #pragma unroll
-			for (int r = 0; r < 4; r++)
-				x.v[r] = bload4(rv, (4 * r + g) * (int)(ldv * 4) + voff, 0);
+				for (int r = 0; r < 4; r++) {
+					const float *row = V + (size_t)min(ib + 4 * r + g, i1 - 1) * ldv;
+					float v[4];
+#pragma unroll
+					for (int t = 0; t < 4; t++)
+						v[t] = row[min(jl + t, m - 1)];
+					x.v[r] = make_float4(v[0], v[1], v[2], v[3]);
+				}
+			} else {
+				const int rows = min(16, i1 - ib);
+				const size_t row = (size_t)ib * ldv;
+				const __amdgpu_buffer_rsrc_t rv = make_rsrc(V + row, ((size_t)(rows - 1) * ldv + m) * 4);
+#pragma unroll
+				for (int r = 0; r < 4; r++)
+					x.v[r] = bload4(rv, (4 * r + g) * (int)(ldv * 4) + voff, 0);
+			}
 			ldq_any<KQ>(W + (size_t)min(ib + l16, n - 1) * KT + KQ * g, x.w);
 		};
 		blk x;
@@ -4094,6 +4108,11 @@ extern "C" uint32_t nmfk_dot_kl_blocks(uint32_t n, uint32_t m)
 	return ((m + 255) / 256) * DOT_ROWSPLIT;
 }
 
+extern "C" int nmfk_rows16_fit(size_t ldu)
+{
+	return ldu <= 0x7fffffffull / 64u;
+}
+
 extern "C" int nmfk_launch_dot_kl(const float *V, size_t ldv, const float *W, const float *H, uint32_t n,
 				  uint32_t m, uint32_t k, uint32_t kt, double *parts, hipStream_t stream)
 {
@@ -4102,8 +4121,12 @@ extern "C" int nmfk_launch_dot_kl(const float *V, size_t ldv, const float *W, co
 	switch (kt) {
 #define X(K)                                                                                      \
 	case K:                                                                                   \
-		hipLaunchKernelGGL((k_dot_kl<K>), grid, dim3(64 * dot_waves(K)), 0, stream, V, ldv, W, H, (int)n, (int)m, \
-				   parts);                                                        \
+		if (nmfk_rows16_fit(ldv))                                                         \
+			hipLaunchKernelGGL((k_dot_kl<K, false>), grid, dim3(64 * dot_waves(K)), 0, stream, V, ldv, W, H, \
+					   (int)n, (int)m, parts);                                \
+		else                                                                              \
+			hipLaunchKernelGGL((k_dot_kl<K, true>), grid, dim3(64 * dot_waves(K)), 0, stream, V, ldv, W, H, \
+					   (int)n, (int)m, parts);                                \
 		return (int)hipGetLastError();
 		NMFK_KT_LIST(X)
 #undef X

@@ -4,6 +4,8 @@ Bars: class vectors, stop iterations and difference counts bit-exact; W, H and t
 divergence within 1e-3 relative of the FP64 oracle (single half-steps: 1e-5)."""
 from __future__ import annotations
 
+import ctypes as C
+
 import numpy as np
 import pytest
 
@@ -577,3 +579,34 @@ def test_config3_full_run_against_fp64(nmfk, path):
         assert np.array_equal(cls, g["cls"])
     else:
         assert err["class_agreement"] >= 0.99
+
+
+@pytest.mark.parametrize("n,m,k,ldv", [(18, 70, 3, 36_000_001), (40, 257, 12, 33_554_433), (5, 9, 2, 150_000_000)])
+def test_dot_kl_of_very_long_rows(nmfk, orc, n, m, k, ldv):
+    # Rows of V so far apart that 16 of them pass 2 GiB: as right as any other pitch.  V is a few
+    # columns of a wider matrix on the device, at the bar of test_dot_and_kl_match_oracle.
+    hip = C.CDLL("libamdhip64.so")
+    hip.hipMalloc.argtypes = [C.POINTER(C.c_void_p), C.c_size_t]
+    hip.hipFree.argtypes = [C.c_void_p]
+    hip.hipMemcpy.argtypes = [C.c_void_p, C.c_void_p, C.c_size_t, C.c_int]
+    V = orc.gen_lognormal(n, m, 7, 0.0, 1.0)
+    W, H = orc.init_WH(n, m, k, 5)
+    dV, out = C.c_void_p(), np.empty(3)
+    lib = nmfk.load()
+    assert hip.hipMalloc(C.byref(dV), 4 * ((n - 1) * ldv + m) + 64) == 0
+    try:
+        d_out = C.c_void_p(dV.value + 4 * m // 64 * 64 + 64)   # between the first two rows
+        for i in range(n):
+            assert hip.hipMemcpy(dV.value + 4 * i * ldv, V[i].ctypes.data, 4 * m, 1) == 0
+        with nmfk.Job(n, m, k) as job:
+            job.set_WH(W, H)
+            inf = job.info()
+            job.sync()
+            assert lib.nmfk_dot_kl_noalloc(dV, ldv, inf.dW, inf.dH, n, m, k, d_out, inf.stream) == 0, nmfk.last_error()
+            job.sync()
+        assert hip.hipMemcpy(out.ctypes.data, d_out, 24, 2) == 0
+    finally:
+        hip.hipFree(dV)
+    dv, dvwh = orc.dot_VWH(V.astype(np.float64), W.astype(np.float64), H.astype(np.float64))
+    kl = orc.kl_div(V, W, H, fp64=True)
+    assert abs(out[0] - dv) / dv < 1e-12 and abs(out[1] - dvwh) / dvwh < 1e-9 and abs(out[2] - kl) / kl < 1e-9
