@@ -225,6 +225,12 @@ int nmfk_batch_add(nmfk_batch *b, nmfk_job *j, const nmfk_options *opt)
 			       "(batched: k <= %d on the default kernel paths)", j->k, NMFK_BATCH_KTMAX);
 		return -1;
 	}
+	/* as nmfk_launch_half refuses for a lone job: the matrix-core bodies address 16 rows of U at once */
+	if (j->kt >= 16 && !(nmfk_rows16_fit(j->ldv) && nmfk_rows16_fit(j->ldvt))) {
+		nmfk_set_error("nmfk_batch_add: rows of V (%zu floats) or of its transposed copy (%zu) are too long for the "
+			       "matrix-core half-steps", j->ldv, j->ldvt);
+		return -1;
+	}
 	uint32_t s = 0;
 	while (s < b->cap && b->job[s])
 		s++;

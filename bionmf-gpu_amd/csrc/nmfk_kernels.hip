@@ -3714,8 +3714,7 @@ static int launch_half_mfma(const nmfk_half *g, const nmfk_hplan *pl, const nmfk
 	half_args h;
 	fin_args f;
 	dim3 grid;
-	// byte offsets within one 16-row block of U are 32-bit
-	if (pl->bchunk % 16 != 0 || !mfma_shape_ok(na, nb) || (size_t)16 * g->ldu * 4 > 0x7fffffffull ||
+	if (pl->bchunk % 16 != 0 || !mfma_shape_ok(na, nb) || !nmfk_rows16_fit(g->ldu) ||
 	    !kernel_args(g, pl, fin, 64u * na, &h, &f, &grid))
 		return (int)hipErrorInvalidValue;
 	if (g->split) {

@@ -282,3 +282,18 @@ def test_short_half_steps_same_bits_as_alone(nmfk, orc, m):
     batch.close()
     for a, b in pairs:
         a.close(), b.close()
+
+
+def test_rows_too_long_for_the_matrix_cores_are_refused(nmfk):
+    # 16 rows of V's transposed copy pass 2 GiB: a lone W half-step refuses such a job, and so does
+    # a batch.
+    n, m, k = 33_554_500, 32, 2
+    with nmfk.Job(n, m, k) as job:
+        with pytest.raises(nmfk.NmfkError):
+            job.update_W()
+        batch = nmfk.Batch(5, 4)
+        try:
+            with pytest.raises(nmfk.NmfkError, match="too long"):
+                batch.add(job, 20, 1000)
+        finally:
+            batch.close()
