@@ -190,6 +190,8 @@ def load(path: os.PathLike | str | None = None):
     _sig(lib, "nmfk_job_info_get", i32, [vp, C.POINTER(JobInfo)])
     _sig(lib, "nmfk_job_time_iterations", i32, [vp, u32, C.POINTER(Timing)])
     _sig(lib, "nmfk_job_set_kernel_path", i32, [vp, i32])
+    _sig(lib, "nmfk_job_set_split", i32, [vp, i32])
+    _sig(lib, "nmfk_job_split", i32, [vp])
     _sig(lib, "nmfk_job_set_schedule", i32, [vp, i32])
     _sig(lib, "nmfk_job_schedule", i32, [vp])
     _sig(lib, "nmfk_job_time_one_pass", i32, [vp, u32, C.POINTER(TimingOnePass)])
@@ -490,6 +492,15 @@ class Job:
 
     def kernel_path(self) -> int:
         return self.lib.nmfk_job_kernel_path(self.h)
+
+    SPLIT_AUTO, SPLIT_OFF, SPLIT_ON = 0, 1, 2
+
+    def set_split(self, mode: int):
+        """Whether FP32 matrix-core half-steps run on split products (nmfk_job_set_split)."""
+        _check(self.lib.nmfk_job_set_split(self.h, mode), "set_split")
+
+    def split(self) -> bool:
+        return bool(self.lib.nmfk_job_split(self.h))
 
     SCHED_AUTO, SCHED_TWO_PASS, SCHED_ONE_PASS = 0, 1, 2
 

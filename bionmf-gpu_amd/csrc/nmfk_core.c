@@ -328,14 +328,12 @@ nmfk_job *nmfk_job_create_shared(nmfk_job *src, uint32_t k)
 	return job_create(src->n, src->m, k, src, NULL, NULL);
 }
 
-/* Jobs planned on their own (no workgroup target) may run on split products; a job replanned
- * to a target, as the sweep and the serving loop do, keeps the FP32 instructions: on
- * split products a burst of 33 served jobs ran 10% faster, but came out 0-15% further from 64 bits
- * over four seeds. */
-static void set_split(nmfk_job *j, uint32_t target_wgs)
+/* Whether the job, as planned now, runs on split products (see nmfk_job_set_split). */
+static void set_split(nmfk_job *j)
 {
-	j->split = target_wgs == 0 && j->planH.path == NMFK_PATH_MFMA32 && j->planW.path == NMFK_PATH_MFMA32 &&
-		   nmfk_split_rule(j->n, j->m, j->kt, j->k);
+	const int rule = j->target_wgs == 0 && nmfk_split_rule(j->n, j->m, j->kt, j->k);
+	j->split = j->planH.path == NMFK_PATH_MFMA32 && j->planW.path == NMFK_PATH_MFMA32 &&
+		   (j->split_mode == NMFK_SPLIT_ON || (j->split_mode == NMFK_SPLIT_AUTO && rule));
 }
 
 static nmfk_job *job_create(uint32_t n, uint32_t m, uint32_t k, nmfk_job *src, nmfk_arena *arena,
@@ -362,7 +360,7 @@ static nmfk_job *job_create(uint32_t n, uint32_t m, uint32_t k, nmfk_job *src, n
 	j->ldv = L.ldv, j->ldvt = L.ldvt;
 	j->planH = L.planH, j->planW = L.planW;
 	j->part_cap = L.n_part;
-	set_split(j, 0);
+	set_split(j);
 	j->ncolW = (n + NMFK_FIN_ROWS - 1) / NMFK_FIN_ROWS;
 	j->ncolH = (m + NMFK_FIN_ROWS - 1) / NMFK_FIN_ROWS;
 	j->ndot = nmfk_dot_kl_blocks(n, m);
@@ -459,6 +457,16 @@ int nmfk_job_info_get(const nmfk_job *j, nmfk_job_info *info)
 	return 0;
 }
 
+/* After a change of what the job's half-steps launch: the captured interval holds the old. */
+static void plan_changed(nmfk_job *j)
+{
+	set_split(j);
+	if (j->chunk_exec) {
+		hipGraphExecDestroy(j->chunk_exec);
+		j->chunk_exec = NULL;
+	}
+}
+
 int nmfk_job_set_kernel_path(nmfk_job *j, int path)
 {
 	if (needs_device_V(j, "nmfk_job_set_kernel_path"))
@@ -479,12 +487,27 @@ int nmfk_job_set_kernel_path(nmfk_job *j, int path)
 	}
 	j->planH = h;
 	j->planW = w;
-	set_split(j, 0);
-	if (j->chunk_exec) {
-		hipGraphExecDestroy(j->chunk_exec);
-		j->chunk_exec = NULL;
-	}
+	j->target_wgs = 0;
+	plan_changed(j);
 	return 0;
+}
+
+int nmfk_job_set_split(nmfk_job *j, int mode)
+{
+	if (needs_device_V(j, "nmfk_job_set_split"))
+		return NMFK_EINVAL;
+	if (mode < NMFK_SPLIT_AUTO || mode > NMFK_SPLIT_ON) {
+		nmfk_set_error("nmfk_job_set_split: unknown mode %d", mode);
+		return NMFK_EINVAL;
+	}
+	j->split_mode = mode;
+	plan_changed(j);
+	return 0;
+}
+
+int nmfk_job_split(const nmfk_job *j)
+{
+	return j->split;
 }
 
 int nmfk_job_replan(nmfk_job *j, uint32_t target_wgs)
@@ -502,11 +525,8 @@ int nmfk_job_replan(nmfk_job *j, uint32_t target_wgs)
 	}
 	j->planH = h;
 	j->planW = w;
-	set_split(j, target_wgs);
-	if (j->chunk_exec) {
-		hipGraphExecDestroy(j->chunk_exec);
-		j->chunk_exec = NULL;
-	}
+	j->target_wgs = target_wgs;
+	plan_changed(j);
 	return 0;
 }
 

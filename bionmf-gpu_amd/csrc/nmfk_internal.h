@@ -42,7 +42,9 @@ struct nmfk_job {
 	nmfk_state *st;                /* device stop-rule state */
 	nmfk_state *h_st;              /* pinned, 2 slots */
 	nmfk_hplan planH, planW;
-	int split;                     /* FP32 matrix-core half-steps run on split products (nmfk_split_rule) */
+	int split_mode;                /* NMFK_SPLIT_* as asked for */
+	uint32_t target_wgs;           /* workgroup target the job was replanned to (0: planned on its own) */
+	int split;                     /* FP32 matrix-core half-steps run on split products (set_split) */
 	hipStream_t stream;
 	hipEvent_t ev[2];
 	hipGraphExec_t chunk_exec;

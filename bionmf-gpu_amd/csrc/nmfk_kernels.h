@@ -45,7 +45,7 @@ uint32_t nmfk_job_kt(uint32_t n, uint32_t m, uint32_t k);
 /* Kernel paths of the partial kernel. */
 #define NMFK_PATH_AUTO 0     /* VALU for kt <= 8, FP32 MFMA otherwise */
 #define NMFK_PATH_VALU 1     /* FP32 FMA on the vector ALUs */
-#define NMFK_PATH_MFMA32 2   /* FP32 MFMA 16x16x4 (kt % 16 == 0) */
+#define NMFK_PATH_MFMA32 2   /* FP32 on the matrix cores (kt % 16 == 0): MFMA 16x16x4, or split products */
 #define NMFK_PATH_MFMA_BF16 3 /* BF16 MFMA 16x16x32, FP32 accumulation (kt % 32 == 0); automatic for kt 64 */
 
 /* Launch plan of one half-step: grid of the partial kernel. */
@@ -115,7 +115,7 @@ typedef struct nmfk_fin {
 int nmfk_launch_half(const nmfk_half *g, const nmfk_hplan *pl, const nmfk_fin *fin, const nmfk_state *st,
 		     hipStream_t stream);
 
-/* Whether a resident FP32 matrix-core job planned on its own runs on split products. */
+/* Whether a resident FP32 matrix-core job planned on its own runs on split products by itself. */
 int nmfk_split_rule(uint32_t n, uint32_t m, uint32_t kt, uint32_t k);
 
 /* One pass over V per iteration (k_fused_mfma): eligible shapes and their launch plan.

@@ -110,7 +110,9 @@ int nmfk_sweep_run(nmfk_job *src, const nmfk_sweep_config *cfg, nmfk_sweep_out *
 				e = NMFK_EINVAL;
 				break;
 			}
-			if (cfg->plan_target)
+			/* one arithmetic for every plan the search may pick (see nmfk_serve.c) */
+			e = nmfk_job_set_split(jobs[i], NMFK_SPLIT_OFF);
+			if (!e && cfg->plan_target)
 				e = nmfk_job_replan(jobs[i], cfg->plan_target);
 			if (!e)
 				e = nmfk_job_init_random(jobs[i], nmfk_sweep_seed(cfg->base_seed, cfg->ks[q], r));

@@ -120,8 +120,9 @@ int nmfk_job_sync(nmfk_job *job);
 
 /* Kernel path of the half-step contractions: 0 = automatic (vector ALUs for k <= 8 when V
  * has fewer than 32 rows or columns, FP32 matrix cores up to k = 32, BF16 matrix cores
- * above), 1 = vector ALUs, 2 = FP32 matrix cores (k padded to 16), 3 = BF16 matrix cores (k
- * padded to 32; FP32 accumulation).  The job's padded rank (nmfk_job_kt) is fixed when it is
+ * above), 1 = vector ALUs, 2 = FP32 on the matrix cores (k padded to 16; see
+ * nmfk_job_set_split for how its products are formed), 3 = BF16 matrix cores (k padded to 32;
+ * FP32 accumulation).  The job's padded rank (nmfk_job_kt) is fixed when it is
  * created, and a path its padding does not fit falls back to the next simpler one. */
 int nmfk_job_set_kernel_path(nmfk_job *job, int path);
 /* Padded rank of a job of n x m at rank k (the row pitch of W and H): 4 or 8 for k <= 8
@@ -130,6 +131,22 @@ int nmfk_job_set_kernel_path(nmfk_job *job, int path);
  * 1.1-2x faster than the vector ALUs at every width but the narrowest. */
 uint32_t nmfk_job_kt(uint32_t n, uint32_t m, uint32_t k);
 int nmfk_job_kernel_path(const nmfk_job *job);
+
+/* How the FP32 matrix-core path (2, or automatic up to k = 32) forms its products: on the FP32
+ * matrix instructions, or as split products, sums of six products of operands in three BF16 parts
+ * each, accumulated in FP32.  Split products are as near to 64 bits (the sums' order, and so
+ * the last bits, are others) and faster on large jobs.  NMFK_SPLIT_AUTO (default): split
+ * products for k > 8 and n m >= 6 Mi (nmfk_split_rule), unless the job is replanned to a
+ * workgroup target, which is meant for many jobs at once.  NMFK_SPLIT_OFF: always the FP32
+ * instructions, on any path and plan.  NMFK_SPLIT_ON: split products whenever both half-steps are on
+ * the FP32 matrix-core path.  Jobs of a rank sweep and of the serving loop are set to
+ * NMFK_SPLIT_OFF.  Streamed jobs always run the FP32 instructions, and refuse the call. */
+#define NMFK_SPLIT_AUTO 0
+#define NMFK_SPLIT_OFF 1
+#define NMFK_SPLIT_ON 2
+int nmfk_job_set_split(nmfk_job *job, int mode);
+/* 1 if the job's half-steps, as planned now, run on split products, else 0. */
+int nmfk_job_split(const nmfk_job *job);
 
 /* Iteration schedule of nmfk_job_run.  NMFK_SCHED_TWO_PASS: one pass over V per half-step
  * (V for the H half, its transposed copy for the W half), the schedule batches and the
@@ -193,7 +210,8 @@ void nmfk_host_free(void *p);
 
 /* Re-plans both half-steps aiming for <target_wgs> partial-kernel workgroups (0 = the
  * process tunables); the number of splits of the contraction range, and with it the
- * summation order, follows the plan, so jobs compared bit for bit must share plans. */
+ * summation order, follows the plan, so jobs compared bit for bit must share plans.  With a
+ * target, a job left at NMFK_SPLIT_AUTO runs the FP32 instructions. */
 int nmfk_job_replan(nmfk_job *job, uint32_t target_wgs);
 /* {nab, S, bchunk, path} of the H half, then of the W half. */
 int nmfk_job_plan_get(const nmfk_job *job, uint32_t out[8]);
@@ -254,7 +272,8 @@ typedef struct nmfk_sweep_config {
 	uint32_t nIters, niter_test_conv, stop_threshold;
 	uint32_t mode;            /* NMFK_SWEEP_BATCHED or NMFK_SWEEP_ONE_AT_A_TIME */
 	uint32_t plan_target;     /* partial-kernel workgroups each job's plan aims for (0: process tunables,
-	                             or, with autotune, chosen by the plan search) */
+	                             or, with autotune, chosen by the plan search); jobs run the FP32
+	                             instructions with every target (NMFK_SPLIT_OFF) */
 	uint32_t autotune;        /* batched mode: tune the launch shape first (and, when plan_target is 0,
 	                             the per-job plan among 8/16/32/64 workgroups and the tunables) */
 	uint32_t autotune_iters;

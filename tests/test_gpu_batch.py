@@ -297,3 +297,22 @@ def test_rows_too_long_for_the_matrix_cores_are_refused(nmfk):
                 batch.add(job, 20, 1000)
         finally:
             batch.close()
+
+
+@pytest.mark.parametrize("mode,autotune", [(0, False), (0, True), (1, False)])
+def test_sweep_jobs_run_the_fp32_instructions(nmfk, mode, autotune):
+    # A matrix large enough for split products: whatever the mode and whatever plan the search picks,
+    # the jobs give the bits of a lone job on the FP32 instructions at that plan.
+    n, m, ks = 6401, 1087, (12, 20)
+    with nmfk.Job(n, m, 1) as src:
+        src.gen_V_lognormal(3, 0.0, 1.0)
+        r = nmfk.sweep(src, ks, 1, 5, nIters=10, niter_test_conv=5, stop_threshold=1000, mode=mode, autotune=autotune,
+                       want_factors=True)
+        for i, k in enumerate(ks):
+            with nmfk.Job.shared(src, k) as job:
+                job.set_split(job.SPLIT_OFF)
+                job.replan(r["plan_target"])
+                job.init_random(nmfk.sweep_seed(5, k, 0))
+                job.run(10, 5, 1000)
+                W, H = r["factors"][i]
+                assert np.array_equal(job.get_W(), W) and np.array_equal(job.get_H(), H)

@@ -218,6 +218,86 @@ def test_lone_half_steps_give_the_bits_of_a_run(nmfk, orc, n, m, k, path):
         assert np.array_equal(a.get_H(), b.get_H()) and np.array_equal(a.get_W(), b.get_W())
 
 
+def test_split_products_are_a_property_of_the_job(nmfk):
+    # Automatic: by size and rank, for a job planned on its own.  On or off holds for every plan;
+    # neither has an effect off the FP32 matrix cores.
+    with nmfk.Job(6401, 1087, 13) as big, nmfk.Job(700, 150, 48) as small:
+        assert big.split() and not small.split()
+        big.replan(1024)
+        assert not big.split()
+        big.set_split(big.SPLIT_ON)
+        assert big.split()
+        big.set_split(big.SPLIT_OFF)
+        for target in (0, 8, 1024):
+            big.replan(target)
+            assert not big.split()
+        big.set_split(big.SPLIT_AUTO)
+        big.replan(0)
+        assert big.split()
+        big.set_kernel_path(1)
+        assert not big.split()
+        big.set_split(big.SPLIT_ON)
+        assert not big.split()
+        big.set_kernel_path(2)
+        assert big.split()
+        small.set_split(small.SPLIT_ON)
+        assert small.kernel_path() == 3 and not small.split()
+        small.set_kernel_path(2)
+        assert small.split()
+        for mode in (-1, 3):
+            with pytest.raises(nmfk.NmfkError):
+                big.set_split(mode)
+    V = np.ones((64, 40), np.float32)
+    with nmfk.Job.streamed(V, 3) as job:
+        assert not job.split()
+        with pytest.raises(nmfk.NmfkError):
+            job.set_split(job.SPLIT_ON)
+
+
+@pytest.mark.parametrize("n,m,k,path", [(64, 33, 3, 2), (65, 1025, 12, 2), (1024, 63, 16, 2), (1025, 1024, 30, 2), (1000, 70, 20, 0),
+                                        (1024, 1023, 64, 2), (1025, 70, 40, 2), (6401, 1087, 13, 0)])
+def test_lone_split_half_steps_give_the_bits_of_a_run(nmfk, orc, n, m, k, path):
+    # On split products the denominators always come from column-sum partials, added as trees by a
+    # kernel of their own here and by the finishes in a run: the same sums.
+    jobs = [make_job(nmfk, orc, n, m, k, seed_v=n, seed_init=m)[0] for _ in range(2)]
+    with jobs[0] as a, jobs[1] as b:
+        for j in jobs:
+            j.set_kernel_path(path)
+            j.set_split(j.SPLIT_ON)
+            assert j.split()
+        a.run(2, 1000, 1000)
+        for _ in range(2):
+            b.update_H()
+            b.update_W()
+        assert np.array_equal(a.get_H(), b.get_H()) and np.array_equal(a.get_W(), b.get_W())
+
+
+@pytest.mark.parametrize("n,m,k,wide", [(900, 130, 12, 1), (900, 130, 30, 1), (12000, 1100, 14, 2), (12000, 1100, 30, 2)])
+def test_split_products_same_bits_in_every_batch_class(nmfk, orc, n, m, k, wide):
+    # kt 16 and 32, in 1 x 4 and (W halves of 1000-4095 columns and enough rows) 2 x 2 waves; split
+    # products at any size when asked for, beside a job on the FP32 instructions in the same batch.
+    V = orc.gen_lognormal(n, m, 4, 0.0, 1.0)
+    jobs = [nmfk.Job(n, m, k) for _ in range(4)]
+    try:
+        for i, j in enumerate(jobs):
+            j.set_V(V)
+            j.init_random(6)
+            j.set_split(j.SPLIT_ON if i < 2 else j.SPLIT_OFF)
+            assert j.split() == (i < 2) and j.plan()["W"]["nab"] == -(-n // (64 * wide))
+        batch = nmfk.Batch(5, 4)
+        batch.add(jobs[1], 10, 1000)
+        batch.add(jobs[3], 10, 1000)
+        batch.run()
+        batch.close()
+        for a, b in ((jobs[0], jobs[1]), (jobs[2], jobs[3])):
+            a.run(10, 5, 1000)
+            assert np.array_equal(a.get_W(), b.get_W()) and np.array_equal(a.get_H(), b.get_H())
+        assert not np.array_equal(jobs[0].get_W(), jobs[2].get_W())
+    finally:
+        for j in jobs:
+            j.close()
+
+
 def test_golden_tiny_runs(nmfk, orc):
     g = np.load(GOLDEN / "tiny.npz")
     for ci in range(int(g["ncases"])):

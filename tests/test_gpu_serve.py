@@ -4,6 +4,7 @@ one it gets when served alone (bitwise: stop iterations, converged restarts, and
 KL divergence of its best restart)."""
 from __future__ import annotations
 
+import numpy as np
 import pytest
 
 pytestmark = pytest.mark.gpu
@@ -112,3 +113,20 @@ def test_served_requests_same_alone_and_in_mix(nmfk, c4_served):
                 kl0 = j.dot_kl()[2]
             assert b["kl"] < kl0, (i, ri)
         assert out[i]["kl_best"] == min(x["kl"] for x in out[i]["restarts"])
+
+
+@pytest.mark.parametrize("target", [0, 64])
+def test_served_jobs_run_the_fp32_instructions(nmfk, target):
+    # A request large enough for split products gives the bits of a lone job on the FP32 instructions
+    # at the served plan, also where that plan is the lone one.
+    n, m, k, seed = 6401, 1087, 14, 21
+    out, _ = nmfk.serve([(n, m, k, 1, seed, 0.0)], nIters=10, niter_test_conv=5, stop_threshold=1000, plan_target=target,
+                        detail=True, factors_of=[0])
+    got = out[0]["restarts"][0]
+    with nmfk.Job(n, m, k) as job:
+        job.set_split(job.SPLIT_OFF)
+        job.replan(target)
+        job.gen_V_lognormal(seed, 5.0, 1.5)
+        job.init_random(nmfk.sweep_seed(seed, k, 0))
+        job.run(10, 5, 1000)
+        assert np.array_equal(job.get_W(), got["W"]) and np.array_equal(job.get_H(), got["H"])
