@@ -1543,12 +1543,14 @@ __global__ __launch_bounds__(64 * NA * NB) void k_partial_bf16(half_args h, bf16
 //          products: [b1 b1][a2 a1], [b2 b2][a2 a1], [b3 b1][a1 a3] over lane groups 0-1, 2-3;
 //   ratio  FP32, then split: lane (g, j) holds rows 4g + r, r = 0..3;
 //   GEMM2  K = the 16 rows of two products: lane group g's 8 elements are rows 4g..4g+3 in one
-//          part, then in another: [r1 r3][b3 b1], [r2 r1][b2 b2], [r2 r1][b1 b1].
+//          part, then in another: [r1 r3][b3 b1], [r2 r1][b2 b2], [r2 r1][b1 b1], added to the
+//          running sums or to fresh ones (see split_fresh).
 // Measured, partials of the two halves (FP32 instructions -> split): 20000 x 1000, k = 32
 // 30.9 + 31.3 -> 23.0 + 23.2 us; 50000 x 2000, k = 64 213 + 239 -> 138 + 155; 20000 x 1000,
-// k = 16 19.0 + 18.8 -> 17.8 + 18.0; 7013 x 333, k = 24 9.0 + 8.3 -> 7.7 + 7.3.  GEMM1 of the next block issued beside GEMM2 of this one, with and without a
-// fixed interleave of matrix and vector instructions, and 3-6 blocks of U in flight were all
-// even or slower: two or three waves per SIMD overlap the two pipes as well.
+// k = 16 19.0 + 18.8 -> 17.8 + 18.0; 7013 x 333, k = 24 9.0 + 8.3 -> 7.7 + 7.3.  GEMM1 of the next
+// block issued beside GEMM2 of this one, with and without a fixed interleave of matrix and vector
+// instructions, and 3-6 blocks of U in flight were all even or slower: two or three waves per SIMD
+// overlap the two pipes as well.
 // --------------------------------------------------------------------------------------
 
 typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
@@ -1648,9 +1650,9 @@ __host__ __device__ constexpr int smem_split(int kt, int na, int nb)
 	return smem_mfma(kt, na, nb) > na * nb * 3 * 8 * (kt + 8) ? smem_mfma(kt, na, nb) : na * nb * 3 * 8 * (kt + 8);
 }
 
-template <int KT, int NA, int NB>
+template <int KT, int NA, int NB, bool FRESH>
 __device__ __forceinline__ void partial_split_body(int bx, int by, const half_args &ha, float *__restrict__ smem,
-						   uint32_t stop = 0)
+						   uint32_t stop)
 {
 	static_assert(KT == 16 || KT % 32 == 0, "split body: KT 16, or whole 32-column chunks");
 	constexpr int H = KT / 16;
@@ -1687,7 +1689,7 @@ __device__ __forceinline__ void partial_split_body(int bx, int by, const half_ar
 		for (int r = 0; r < 4; r++)
 			u[r] = bload4(rU, uoff[r], 0);
 	};
-	constexpr int DU = KT <= 32 ? 2 : 1, DB = 1;   // blocks of U and of B in flight
+	constexpr int DU = KT == 16 || (KT == 32 && !FRESH) ? 2 : 1, DB = 1;   // blocks of U and of B in flight
 	float4 ur[DU][4], br[DB][H];
 	auto fetch_b = [&](int bb, float4 (&b)[H]) {
 		const __amdgpu_buffer_rsrc_t rB = make_rsrc(B + (size_t)bb * KT, (size_t)16 * KT * 4);
@@ -1810,15 +1812,38 @@ __device__ __forceinline__ void partial_split_body(int bx, int by, const half_ar
 					(lds4)(slot + (i * 16 + 4 * g + (j >> 2)) * BS + 16 * h + 4 * (j & 3)));
 				__builtin_memcpy(&b2[i], &v, 8);
 			}
+			if constexpr (FRESH) {
+				// at KT 32 and 64 a tile at a time, for the registers
+				constexpr int TW = KT > 16 ? 1 : 4;
 #pragma unroll
-			for (int t = 0; t < 4; t++)
-				acc[t][h] = mfma(cat8(pr[t][0], pr[t][2]), cat8(b2[2], b2[0]), acc[t][h]);
+				for (int t0 = 0; t0 < 4; t0 += TW) {
+					floatx4 x[TW];
 #pragma unroll
-			for (int t = 0; t < 4; t++)
-				acc[t][h] = mfma(cat8(pr[t][1], pr[t][0]), cat8(b2[1], b2[1]), acc[t][h]);
+					for (int t = 0; t < TW; t++)
+						x[t] = mfma(cat8(pr[t0 + t][0], pr[t0 + t][2]), cat8(b2[2], b2[0]), floatx4{0.f, 0.f, 0.f, 0.f});
 #pragma unroll
-			for (int t = 0; t < 4; t++)
-				acc[t][h] = mfma(cat8(pr[t][1], pr[t][0]), cat8(b2[0], b2[0]), acc[t][h]);
+					for (int t = 0; t < TW; t++)
+						x[t] = mfma(cat8(pr[t0 + t][1], pr[t0 + t][0]), cat8(b2[1], b2[1]), x[t]);
+#pragma unroll
+					for (int t = 0; t < TW; t++)
+						x[t] = mfma(cat8(pr[t0 + t][1], pr[t0 + t][0]), cat8(b2[0], b2[0]), x[t]);
+#pragma unroll
+					for (int t = 0; t < TW; t++)
+						acc[t0 + t][h] += x[t];
+					if constexpr (TW == 1)
+						__builtin_amdgcn_sched_barrier(0);
+				}
+			} else {
+#pragma unroll
+				for (int t = 0; t < 4; t++)
+					acc[t][h] = mfma(cat8(pr[t][0], pr[t][2]), cat8(b2[2], b2[0]), acc[t][h]);
+#pragma unroll
+				for (int t = 0; t < 4; t++)
+					acc[t][h] = mfma(cat8(pr[t][1], pr[t][0]), cat8(b2[1], b2[1]), acc[t][h]);
+#pragma unroll
+				for (int t = 0; t < 4; t++)
+					acc[t][h] = mfma(cat8(pr[t][1], pr[t][0]), cat8(b2[0], b2[0]), acc[t][h]);
+			}
 		}
 	};
 	if (mine > 0) {
@@ -1878,7 +1903,22 @@ __device__ __forceinline__ void partial_split_body(int bx, int by, const half_ar
 	mfma_store<KT, NA, NB>(acc, ha, by, a0, idle, smem);
 }
 
-template <int KT, int NA, int NB>
+// FRESH: the products of each 16-row block are summed from zero and added to the running sums by
+// the vector ALUs.  The matrix instructions truncate small terms against a large sum, so that a
+// sum kept in them falls behind in proportion to its length, and over many iterations W and H
+// drift apart in scale: H of 200000 x 64, k = 12, 784 rows per wave, came out 2.0 times as far
+// from 64 bits after 100 iterations as on the FP32 instructions, and 0.5 times with fresh sums; W of
+// 1000000 x 64, k = 24, 4.0 and 0.4 times.  At KT 16 fresh sums cost 1% (42.3 -> 42.7 us per iteration at 20000 x 1000) and are
+// always taken.  At KT 32 and 64 the registers that they need cost 3% and 7% (54.1 -> 55.9 us at 20000 x
+// 1000, k = 32; 322 -> 344 at 50000 x 2000, k = 64), and they are taken where a wave's rows are
+// many: errors of the kept sums over those of the FP32 instructions, k = 24, 316 rows 0.7-0.9, 392
+// 1.0-1.3, 784 1.6-1.9; k = 48, 236 0.6-0.9, 392 0.9-1.0, 784 1.4-1.6.
+__host__ __device__ constexpr bool split_fresh(int kt, int bchunk, int nb)
+{
+	return kt == 16 || bchunk > (kt == 32 ? 320 : 400) * nb;
+}
+
+template <int KT, int NA, int NB, bool FRESH>
 __global__ __launch_bounds__(64 * NA * NB, (KT <= 32 ? 3 : 2)) void k_partial_split(half_args h, fin_args f, const nmfk_state *__restrict__ st)
 {
 	constexpr int LDS = max2(smem_split(KT, NA, NB), smem_finish(KT, 64 * NA));
@@ -1887,7 +1927,7 @@ __global__ __launch_bounds__(64 * NA * NB, (KT <= 32 ? 3 : 2)) void k_partial_sp
 	int bx, by;
 	if (!half_tile<KT, true, LDS>(h, f, smem, stop, bx, by))
 		return;
-	partial_split_body<KT, NA, NB>(bx, by, h, smem, stop);
+	partial_split_body<KT, NA, NB, FRESH>(bx, by, h, smem, stop);
 	if (h.part == nullptr && !stopped(stop))
 		finish_rows<KT, true, 64 * NA * NB>(bx, 64 * NA, h, f, smem);
 }
@@ -2998,7 +3038,10 @@ __global__ __launch_bounds__(NMFK_WG, (CLS == 0 || CLS == 2 || CLS == 4 ? 4 : CL
 		} else {
 			constexpr int KT = batch_cls_kt(CLS), NA = batch_cls_na(CLS), NB = 4 / NA;
 			if constexpr (CLS >= 6) {
-				partial_split_body<KT, NA, NB>(tl.bx, tl.by, h, smem);
+				if (split_fresh(KT, h.bchunk, NB))
+					partial_split_body<KT, NA, NB, true>(tl.bx, tl.by, h, smem, 0);
+				else
+					partial_split_body<KT, NA, NB, KT == 16>(tl.bx, tl.by, h, smem, 0);
 			} else if constexpr (KT == 16) {
 				// a rank up to 4 or 8 sums only its columns in GEMM1 (nmfk_plan_set_rank)
 				const uint32_t ke = half == 0 ? J.planH.ke : J.planW.ke;
@@ -3632,13 +3675,13 @@ extern "C" void nmfk_plan_set_rank(nmfk_hplan *pl, uint32_t kt, uint32_t k)
 // 34.1, 20000 x 1000 45.9 / 43.7: at kt 16 the line lies between 5 and 8 million values, below
 // which a block's longer chain costs what the shorter products save.  At kt 32 and 64 they are
 // faster at every size (k = 24 or 32: 3000 x 300 26.4 / 24.5, 1000 x 1000 27.5 / 24.8, 20000 x
-// 1000 74.7 / 58.8; k = 48: 10000 x 1000 95.3 / 71.1), and the line is one of accuracy.  The BF16
-// instructions truncate small terms against large ones, 0.1-0.2 ulp toward zero in sums of
-// heavy-tailed terms, and on smaller lognormal matrices, over 100 iterations, that can show: W and
-// H then came out more than 1.5 times as far from 64 bits as on the FP32 instructions, and over
-// 1e-6, in 7 of 78 shapes of 1 to 6 million values, and in none of 82 larger ones, nor of 80
-// planted ones of all sizes.  In the mean, with the tree sums of pair8, their errors are 0.82
-// times those of the FP32 instructions.
+// 1000 74.7 / 58.8; k = 48: 10000 x 1000 95.3 / 71.1); smaller jobs were left out while all sums were
+// kept in the matrix instructions (see split_fresh), for 7 of 78 shapes of 1 to 6 million values
+// whose W and H then came out more than 1.5 times as far from 64 bits.  Errors now, over 120
+// drawn jobs of 6 to 60 million values, k = 9..64, planted and lognormal, 10-100 iterations: 0.76
+// times those of the FP32 instructions in the mean, 1.2 times at most.  Other seeds of lognormal ones
+// scatter more, as the FP32 instructions do between two plans: 6 of 82 over 1.5 times, 20 under 1/1.5.
+// Jobs planned to 96 workgroups: 0.64 times in the mean (1.1 with all sums kept).
 extern "C" int nmfk_split_rule(uint32_t n, uint32_t m, uint32_t kt, uint32_t k)
 {
 	return kt % 16u == 0 && k > 8u && (size_t)n * m >= (6u << 20);
@@ -3720,7 +3763,10 @@ static int launch_half_mfma(const nmfk_half *g, const nmfk_hplan *pl, const nmfk
 	if (g->split) {
 #define X(NA_, NB_)                                                                                    \
 	if (na == NA_ && nb == NB_) {                                                                  \
-		hipLaunchKernelGGL((k_partial_split<KT, NA_, NB_>), grid, dim3(64 * NA_ * NB_), 0, stream, h, f, st); \
+		if (split_fresh(KT, h.bchunk, NB_))                                                    \
+			hipLaunchKernelGGL((k_partial_split<KT, NA_, NB_, true>), grid, dim3(64 * NA_ * NB_), 0, stream, h, f, st); \
+		else                                                                                   \
+			hipLaunchKernelGGL((k_partial_split<KT, NA_, NB_, KT == 16>), grid, dim3(64 * NA_ * NB_), 0, stream, h, f, st); \
 		return (int)hipGetLastError();                                                         \
 	}
 		NMFK_SHAPE_LIST(X)

@@ -123,7 +123,8 @@ static int admit(const nmfk_serve_config *cfg, const nmfk_request *q, req_state 
 		return e;   /* nothing was added to the batch yet */
 	for (uint32_t i = 0; i < q->restarts && !e; i++) {
 		/* FP32 instructions with any target: on split products a burst of 33 served jobs ran 10%
-		 * faster, but came out 0-15% further from 64 bits over four seeds */
+		 * faster, but came out 0-15% further from 64 bits over four seeds (with all sums kept in the
+		 * matrix instructions, see split_fresh) */
 		e = nmfk_job_set_split(r->jobs[i], NMFK_SPLIT_OFF);
 		if (!e && cfg->plan_target)
 			e = nmfk_job_replan(r->jobs[i], cfg->plan_target);

@@ -272,6 +272,23 @@ def test_lone_split_half_steps_give_the_bits_of_a_run(nmfk, orc, n, m, k, path):
         assert np.array_equal(a.get_H(), b.get_H()) and np.array_equal(a.get_W(), b.get_W())
 
 
+@pytest.mark.parametrize("n,m,k", [(500000, 32, 16), (500000, 32, 24), (400000, 40, 40)])
+def test_split_products_do_not_lose_long_sums(nmfk, orc, n, m, k):
+    # Sums of thousands of rows per wave keep no bias: the mean relative error of an H half-step
+    # stays below 2^-25.  Rounding to nearest leaves m k entries within 2^-23 and k denominators within
+    # 2^-24 of their values, whose means are below 2^-25 by far; sums that lose a part of every
+    # term reach 8e-8 here.
+    with nmfk.Job(n, m, k) as job:
+        job.set_kernel_path(2)
+        assert job.split()
+        job.gen_V_planted(3, 6, 0.3)
+        job.init_random(4)
+        W, H = job.get_W(), job.get_H()
+        want = orc.update_H(job.get_V(), W, H).astype(np.float64)
+        job.update_H()
+        assert abs(np.mean(job.get_H() / want) - 1.0) < 2.0 ** -25
+
+
 @pytest.mark.parametrize("n,m,k,wide", [(900, 130, 12, 1), (900, 130, 30, 1), (12000, 1100, 14, 2), (12000, 1100, 30, 2)])
 def test_split_products_same_bits_in_every_batch_class(nmfk, orc, n, m, k, wide):
     # kt 16 and 32, in 1 x 4 and (W halves of 1000-4095 columns and enough rows) 2 x 2 waves; split
