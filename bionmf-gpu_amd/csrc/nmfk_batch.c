@@ -24,10 +24,10 @@
 
 /* Partial tables per half and body class: VALU half-steps without and with lane groups
  * (a factor with few rows), matrix-core half-steps of kt 16 and of kt 32 in 1 x 4 waves, the
- * same in 2 x 2 waves (a lone job's plan over a short contraction range), and these four on
- * split products, each launched on its own so that it runs at its own occupancy.  Empty
+ * same in 2 x 2 waves (a lone job's plan over a short contraction range), and kt 32 on split
+ * products in both, each launched on its own so that it runs at its own occupancy.  Empty
  * classes launch nothing. */
-#define NCLS 10
+#define NCLS 8
 enum { TAB_PART_H0, TAB_PART_W0 = TAB_PART_H0 + NCLS, TAB_SHORT_H = TAB_PART_W0 + NCLS, TAB_SHORT_W, TAB_FIN_H, TAB_FIN_W,
        TAB_TEST, NTAB };
 
@@ -36,7 +36,7 @@ enum { TAB_PART_H0, TAB_PART_W0 = TAB_PART_H0 + NCLS, TAB_SHORT_H = TAB_PART_W0 
 static int half_short(const nmfk_job *j, int half)
 {
 	const nmfk_hplan *p = half ? &j->planW : &j->planH;
-	return j->kt == 16 && !j->split && p->ap == 1 && p->S == 1 && (half ? j->m : j->n) <= NMFK_SHORT_Q;
+	return j->kt == 16 && p->ap == 1 && p->S == 1 && (half ? j->m : j->n) <= NMFK_SHORT_Q;
 }
 
 static int half_cls(const nmfk_job *j, int half)
@@ -46,7 +46,9 @@ static int half_cls(const nmfk_job *j, int half)
 		return -1;
 	if (j->kt <= 8)
 		return p->lb > 1 ? 1 : 0;
-	return (j->kt == 16 ? 2 : 3) + (p->ap == 2 ? 2 : 0) + (j->split ? 4 : 0);
+	if (j->split)
+		return p->ap == 2 ? 7 : 6;
+	return (j->kt == 16 ? 2 : 3) + (p->ap == 2 ? 2 : 0);
 }
 
 struct nmfk_batch {

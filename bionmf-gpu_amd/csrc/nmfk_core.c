@@ -332,7 +332,7 @@ nmfk_job *nmfk_job_create_shared(nmfk_job *src, uint32_t k)
 static void set_split(nmfk_job *j)
 {
 	const int rule = j->target_wgs == 0 && nmfk_split_rule(j->n, j->m, j->kt, j->k);
-	j->split = j->planH.path == NMFK_PATH_MFMA32 && j->planW.path == NMFK_PATH_MFMA32 &&
+	j->split = j->planH.path == NMFK_PATH_MFMA32 && j->planW.path == NMFK_PATH_MFMA32 && j->kt >= 32 &&
 		   (j->split_mode == NMFK_SPLIT_ON || (j->split_mode == NMFK_SPLIT_AUTO && rule));
 }
 

@@ -98,8 +98,8 @@ typedef struct nmfk_half {
 	const float *A, *B;
 	const uint16_t *Bb;   /* row-major BF16 copy of B (plan path NMFK_PATH_MFMA_BF16 reads it instead of B) */
 	uint32_t p, q, kt;
-	int split;            /* products of three-part BF16 operands (FP32 accuracy; kt 16, 32, 64 on plan path
-				 NMFK_PATH_MFMA32; sums every column of kt, and splits, rows and column sums as trees) */
+	int split;            /* products of three-part BF16 operands (FP32 accuracy; kt 32, 64 on plan path
+				 NMFK_PATH_MFMA32; splits, rows and column sums are added as trees) */
 	float *part;
 } nmfk_half;
 typedef struct nmfk_fin {
@@ -187,12 +187,12 @@ typedef struct nmfk_tile {
 /* half: 0 = H half (U = V, A = H, B = W), 1 = W half (U = Vt, A = W, B = H).  cls: the body
  * class of every tile's half-step: 0 = vector ALUs (kt 4/8) without lane groups, 1 = vector
  * ALUs with lane groups (plan lb > 1), 2 and 3 = matrix cores at kt 16 and 32 in 1 x 4 waves,
- * 4 and 5 = the same in 2 x 2 waves (plan ap 2), 6-9 = classes 2-5 on split products; tiles of
- * other classes are skipped. */
+ * 4 and 5 = the same in 2 x 2 waves (plan ap 2), 6 and 7 = classes 3 and 5 on split products;
+ * tiles of other classes are skipped. */
 int nmfk_launch_batch_partial(const nmfk_bjob *jobs, const nmfk_tile *tiles, uint32_t ntiles, int half,
 			      int cls, uint32_t grid, hipStream_t stream);
-/* Half-steps of one split over at most NMFK_SHORT_Q rows (kt 16, matrix cores in 1 x 4 waves, not
- * on split products), finishes included; a tile is a row group of the job's own grid, one wave. */
+/* Half-steps of one split over at most NMFK_SHORT_Q rows (kt 16, matrix cores in 1 x 4 waves),
+ * finishes included; a tile is a row group of the job's own grid, one wave. */
 #define NMFK_SHORT_Q 256
 int nmfk_launch_batch_short(const nmfk_bjob *jobs, const nmfk_tile *tiles, uint32_t ntiles, int half,
 			    int clamp, uint32_t grid, hipStream_t stream);

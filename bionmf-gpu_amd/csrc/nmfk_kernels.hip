@@ -114,7 +114,7 @@ typedef float floatx4 __attribute__((ext_vector_type(4)));
 
 // Eight values as a tree: 3 roundings deep instead of 8.  The sums over splits, rows and
 // column-sum partials of a job on split products are formed this way, which takes their
-// rounding errors well below those of the products (H half at 20000 x 1000, k = 16: 1.5e-7 rms
+// rounding errors well below those of the products (a half-step at 20000 x 1000: 1.5e-7 rms
 // from 64 bits in order, 0.5e-7 without these errors).  Every other job keeps its ascending
 // order, and with it its bits.
 __device__ __forceinline__ float pair8(const float (&v)[8])
@@ -1522,8 +1522,8 @@ __global__ __launch_bounds__(64 * NA * NB) void k_partial_bf16(half_args h, bf16
 }
 
 // --------------------------------------------------------------------------------------
-// The half-step in FP32 accuracy on the BF16 matrix cores (KT 16, 32, 64; nmfk_split_rule says
-// which jobs).
+// The half-step in FP32 accuracy on the BF16 matrix cores (KT 32 and 64; nmfk_split_rule says which
+// jobs).
 // Every FP32 operand is the exact sum of three BF16 numbers, x = x1 + x2 + x3: 3 x 8
 // significand bits, each part the rounding of what the parts before it leave.  A product is
 // formed from the six partial products of relative size 2^-16 and more (x1 y1, x1 y2, x2 y1,
@@ -1532,25 +1532,23 @@ __global__ __launch_bounds__(64 * NA * NB) void k_partial_bf16(half_args h, bf16
 // from the 64-bit sums, against 8.8e-8, 1.2e-7 and 2.4e-7 on the FP32 instructions.  Exact for
 // operands of 7.7e-34 and more (bits below 2^-133 are lost); infinities see partial_split_body.
 //
-// What bounds the FP32 instructions is their rate: 16x16x4 takes 32 cycles, 1024 per 16-row
-// block and 64 rows a at KT 16, 2048 at KT 32, 4096 at KT 64.  The split products take 384,
-// 768 and 1536, and 120-180 vector instructions for the ratios and the splitting.  Ownership
-// of rows, blocks and wave groups is that of the body above; per 16-row block a wave
+// What bounds the FP32 instructions is their rate: 16x16x4 takes 32 cycles, 2048 per 16-row
+// block and 64 rows a at KT 32, 4096 at KT 64.  The split products take 768 and 1536, and 150-180
+// vector instructions for the ratios and the splitting.  Ownership of rows, blocks and wave groups
+// is that of the body above; per 16-row block a wave
 //   stages B (fetched as FP32, one block ahead) in its own LDS slot in three parts, row-major,
 //   from where both operand layouts are read: GEMM1's as 16-byte row segments, GEMM2's with
 //   ds_read_b64_tr_b16 (4 rows of one column per lane);
-//   GEMM1  K = 32 columns of one product; at KT 16 the 32 slots hold the 16 columns of two
-//          products: [b1 b1][a2 a1], [b2 b2][a2 a1], [b3 b1][a1 a3] over lane groups 0-1, 2-3;
+//   GEMM1  K = 32 columns of one product;
 //   ratio  FP32, then split: lane (g, j) holds rows 4g + r, r = 0..3;
 //   GEMM2  K = the 16 rows of two products: lane group g's 8 elements are rows 4g..4g+3 in one
 //          part, then in another: [r1 r3][b3 b1], [r2 r1][b2 b2], [r2 r1][b1 b1], added to the
 //          running sums or to fresh ones (see split_fresh).
 // Measured, partials of the two halves (FP32 instructions -> split): 20000 x 1000, k = 32
-// 30.9 + 31.3 -> 23.0 + 23.2 us; 50000 x 2000, k = 64 213 + 239 -> 138 + 155; 20000 x 1000,
-// k = 16 19.0 + 18.8 -> 17.8 + 18.0; 7013 x 333, k = 24 9.0 + 8.3 -> 7.7 + 7.3.  GEMM1 of the next
-// block issued beside GEMM2 of this one, with and without a fixed interleave of matrix and vector
-// instructions, and 3-6 blocks of U in flight were all even or slower: two or three waves per SIMD
-// overlap the two pipes as well.
+// 30.9 + 31.3 -> 23.0 + 23.2 us; 50000 x 2000, k = 64 213 + 239 -> 138 + 155; 7013 x 333, k = 24 9.0 +
+// 8.3 -> 7.7 + 7.3.  GEMM1 of the next block issued beside GEMM2 of this one, with and without a
+// fixed interleave of matrix and vector instructions, and 3-6 blocks of U in flight were all
+// even or slower: two or three waves per SIMD overlap the two pipes as well.
 // --------------------------------------------------------------------------------------
 
 typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
@@ -1654,10 +1652,9 @@ template <int KT, int NA, int NB, bool FRESH>
 __device__ __forceinline__ void partial_split_body(int bx, int by, const half_args &ha, float *__restrict__ smem,
 						   uint32_t stop)
 {
-	static_assert(KT == 16 || KT % 32 == 0, "split body: KT 16, or whole 32-column chunks");
+	static_assert(KT % 32 == 0, "split body: whole 32-column chunks");
 	constexpr int H = KT / 16;
-	constexpr int CH = KT >= 32 ? KT / 32 : 1;   // 32-column chunks of GEMM1
-	constexpr int NQ = KT >= 32 ? 3 : 2;         // GEMM1 operands of A per tile and chunk
+	constexpr int CH = KT / 32;   // 32-column chunks of GEMM1
 	const float *__restrict__ U = ha.U;
 	const size_t ldu = ha.ldu;
 	const float *__restrict__ A = ha.A;
@@ -1689,7 +1686,7 @@ __device__ __forceinline__ void partial_split_body(int bx, int by, const half_ar
 		for (int r = 0; r < 4; r++)
 			u[r] = bload4(rU, uoff[r], 0);
 	};
-	constexpr int DU = KT == 16 || (KT == 32 && !FRESH) ? 2 : 1, DB = 1;   // blocks of U and of B in flight
+	constexpr int DU = KT == 32 && !FRESH ? 2 : 1, DB = 1;   // blocks of U and of B in flight
 	float4 ur[DU][4], br[DB][H];
 	auto fetch_b = [&](int bb, float4 (&b)[H]) {
 		const __amdgpu_buffer_rsrc_t rB = make_rsrc(B + (size_t)bb * KT, (size_t)16 * KT * 4);
@@ -1709,14 +1706,14 @@ __device__ __forceinline__ void partial_split_body(int bx, int by, const half_ar
 		return;
 
 	// GEMM1's A operands.
-	bf16x8 aq[4][CH][NQ];
+	bf16x8 aq[4][CH][3];
 #pragma unroll
 	for (int t = 0; t < 4; t++) {
 		const bool ok = t < avail;
 		const float *Ar = A + (size_t)(ok ? aj + t : 0) * KT;
 #pragma unroll
 		for (int ch = 0; ch < CH; ch++) {
-			const float *Ac = Ar + (KT >= 32 ? 32 * ch + 8 * g : 8 * (g & 1));
+			const float *Ac = Ar + 32 * ch + 8 * g;
 			float4 lo = *reinterpret_cast<const float4 *>(Ac);
 			float4 hi = *reinterpret_cast<const float4 *>(Ac + 4);
 			if (!ok)
@@ -1724,13 +1721,9 @@ __device__ __forceinline__ void partial_split_body(int bx, int by, const half_ar
 			bf16x4 pl[3], ph[3];
 			split3x4(lo.x, lo.y, lo.z, lo.w, pl);
 			split3x4(hi.x, hi.y, hi.z, hi.w, ph);
-			const bf16x8 a1 = cat8(pl[0], ph[0]), a2 = cat8(pl[1], ph[1]), a3 = cat8(pl[2], ph[2]);
-			if constexpr (KT >= 32) {
-				aq[t][ch][0] = a1, aq[t][ch][1] = a2, aq[t][ch][2] = a3;
-			} else {
-				aq[t][ch][0] = g < 2 ? a2 : a1;
-				aq[t][ch][1] = g < 2 ? a1 : a3;
-			}
+#pragma unroll
+			for (int i = 0; i < 3; i++)
+				aq[t][ch][i] = cat8(pl[i], ph[i]);
 		}
 	}
 	floatx4 acc[4][H];
@@ -1758,32 +1751,18 @@ __device__ __forceinline__ void partial_split_body(int bx, int by, const half_ar
 #pragma unroll
 		for (int t = 0; t < 4; t++)
 			s[t] = floatx4{0.f, 0.f, 0.f, 0.f};
-		if constexpr (KT >= 32) {
-			constexpr int ib[6] = {2, 0, 1, 1, 0, 0}, ia[6] = {0, 2, 1, 0, 1, 0};
+		constexpr int ib[6] = {2, 0, 1, 1, 0, 0}, ia[6] = {0, 2, 1, 0, 1, 0};
 #pragma unroll
-			for (int ch = 0; ch < CH; ch++) {
-				bf16x8 bq[3];
-#pragma unroll
-				for (int i = 0; i < 3; i++)
-					bq[i] = *reinterpret_cast<const bf16x8 *>(slot + (i * 16 + j) * BS + 32 * ch + 8 * g);
-#pragma unroll
-				for (int x = 0; x < 6; x++)
-#pragma unroll
-					for (int t = 0; t < 4; t++)
-						s[t] = mfma(bq[ib[x]], aq[t][ch][ia[x]], s[t]);
-			}
-		} else {
+		for (int ch = 0; ch < CH; ch++) {
 			bf16x8 bq[3];
 #pragma unroll
-			for (int i = 0; i < 3; i++) {
-				const int part = i < 2 ? i : (g < 2 ? 2 : 0);
-				bq[i] = *reinterpret_cast<const bf16x8 *>(slot + (part * 16 + j) * BS + 8 * (g & 1));
-			}
+			for (int i = 0; i < 3; i++)
+				bq[i] = *reinterpret_cast<const bf16x8 *>(slot + (i * 16 + j) * BS + 32 * ch + 8 * g);
 #pragma unroll
-			for (int x = 2; x >= 0; x--)
+			for (int x = 0; x < 6; x++)
 #pragma unroll
 				for (int t = 0; t < 4; t++)
-					s[t] = mfma(bq[x], aq[t][0][x == 2 ? 1 : 0], s[t]);
+					s[t] = mfma(bq[ib[x]], aq[t][ch][ia[x]], s[t]);
 		}
 	};
 	bf16x4 pr[4][3];
@@ -1813,25 +1792,12 @@ __device__ __forceinline__ void partial_split_body(int bx, int by, const half_ar
 				__builtin_memcpy(&b2[i], &v, 8);
 			}
 			if constexpr (FRESH) {
-				// at KT 32 and 64 a tile at a time, for the registers
-				constexpr int TW = KT > 16 ? 1 : 4;
 #pragma unroll
-				for (int t0 = 0; t0 < 4; t0 += TW) {
-					floatx4 x[TW];
-#pragma unroll
-					for (int t = 0; t < TW; t++)
-						x[t] = mfma(cat8(pr[t0 + t][0], pr[t0 + t][2]), cat8(b2[2], b2[0]), floatx4{0.f, 0.f, 0.f, 0.f});
-#pragma unroll
-					for (int t = 0; t < TW; t++)
-						x[t] = mfma(cat8(pr[t0 + t][1], pr[t0 + t][0]), cat8(b2[1], b2[1]), x[t]);
-#pragma unroll
-					for (int t = 0; t < TW; t++)
-						x[t] = mfma(cat8(pr[t0 + t][1], pr[t0 + t][0]), cat8(b2[0], b2[0]), x[t]);
-#pragma unroll
-					for (int t = 0; t < TW; t++)
-						acc[t0 + t][h] += x[t];
-					if constexpr (TW == 1)
-						__builtin_amdgcn_sched_barrier(0);
+				for (int t = 0; t < 4; t++) {   // one at a time, for the registers
+					floatx4 x = mfma(cat8(pr[t][0], pr[t][2]), cat8(b2[2], b2[0]), floatx4{0.f, 0.f, 0.f, 0.f});
+					x = mfma(cat8(pr[t][1], pr[t][0]), cat8(b2[1], b2[1]), x);
+					acc[t][h] += mfma(cat8(pr[t][1], pr[t][0]), cat8(b2[0], b2[0]), x);
+					__builtin_amdgcn_sched_barrier(0);
 				}
 			} else {
 #pragma unroll
@@ -1906,20 +1872,20 @@ __device__ __forceinline__ void partial_split_body(int bx, int by, const half_ar
 // FRESH: the products of each 16-row block are summed from zero and added to the running sums by
 // the vector ALUs.  The matrix instructions truncate small terms against a large sum, so that a
 // sum kept in them falls behind in proportion to its length, and over many iterations W and H
-// drift apart in scale: H of 200000 x 64, k = 12, 784 rows per wave, came out 2.0 times as far
-// from 64 bits after 100 iterations as on the FP32 instructions, and 0.5 times with fresh sums; W of
-// 1000000 x 64, k = 24, 4.0 and 0.4 times.  At KT 16 fresh sums cost 1% (42.3 -> 42.7 us per iteration at 20000 x 1000) and are
-// always taken.  At KT 32 and 64 the registers that they need cost 3% and 7% (54.1 -> 55.9 us at 20000 x
-// 1000, k = 32; 322 -> 344 at 50000 x 2000, k = 64), and they are taken where a wave's rows are
-// many: errors of the kept sums over those of the FP32 instructions, k = 24, 316 rows 0.7-0.9, 392
-// 1.0-1.3, 784 1.6-1.9; k = 48, 236 0.6-0.9, 392 0.9-1.0, 784 1.4-1.6.
+// drift apart in scale: W and H of 200000 x 64, k = 24, 784 rows per wave, came out 1.6 times as far
+// from 64 bits after 100 iterations as on the FP32 instructions, and 0.6 times with fresh sums; those of
+// 1000000 x 64 4.0 and 0.4 times.  The registers that fresh sums need cost 3% at KT 32 and 7% at KT 64
+// (54.1 -> 55.9 us per iteration at 20000 x 1000, k = 32; 322 -> 344 at 50000 x 2000, k = 64), so they
+// are taken where a wave's rows are many: errors of the kept sums over those of the FP32
+// instructions, k = 24, 316 rows 0.7-0.9, 392 1.0-1.3, 784 1.6-1.9; k = 48, 236 0.6-0.9, 392 0.9-1.0,
+// 784 1.4-1.6.
 __host__ __device__ constexpr bool split_fresh(int kt, int bchunk, int nb)
 {
-	return kt == 16 || bchunk > (kt == 32 ? 320 : 400) * nb;
+	return bchunk > (kt == 32 ? 320 : 400) * nb;
 }
 
 template <int KT, int NA, int NB, bool FRESH>
-__global__ __launch_bounds__(64 * NA * NB, (KT <= 32 ? 3 : 2)) void k_partial_split(half_args h, fin_args f, const nmfk_state *__restrict__ st)
+__global__ __launch_bounds__(64 * NA * NB, (KT == 32 ? 3 : 2)) void k_partial_split(half_args h, fin_args f, const nmfk_state *__restrict__ st)
 {
 	constexpr int LDS = max2(smem_split(KT, NA, NB), smem_finish(KT, 64 * NA));
 	__shared__ __align__(16) float smem[LDS];
@@ -2968,19 +2934,19 @@ __device__ __forceinline__ void batch_valu_body(int bx, int by, const half_args 
 	}
 }
 
-// Ten batched partial kernels, one per body class, so each runs at its own occupancy: the
+// Eight batched partial kernels, one per body class, so each runs at its own occupancy: the
 // VALU bodies (KT 4/8) of half-steps without lane groups, those with lane groups (few rows
 // of the updated factor: their variants need more registers), the matrix-core bodies of KT 16
 // and of KT 32 in 1 x 4 waves, the same in 2 x 2 waves (the plan of a lone job over a short
-// contraction range), and these four on split products (classes 6-9); a batch launches each
-// over its own tile table.
+// contraction range), and KT 32 on split products in 1 x 4 and 2 x 2 waves (classes 6 and 7); a
+// batch launches each over its own tile table.
 __host__ __device__ constexpr int batch_cls_kt(int cls)
 {
-	return cls % 2 == 0 ? 16 : 32;
+	return cls == 2 || cls == 4 ? 16 : 32;
 }
 __host__ __device__ constexpr int batch_cls_na(int cls)
 {
-	return (cls - 2) % 4 >= 2 ? 2 : 1;
+	return cls == 4 || cls == 5 || cls == 7 ? 2 : 1;
 }
 
 template <int CLS>
@@ -3041,7 +3007,7 @@ __global__ __launch_bounds__(NMFK_WG, (CLS == 0 || CLS == 2 || CLS == 4 ? 4 : CL
 				if (split_fresh(KT, h.bchunk, NB))
 					partial_split_body<KT, NA, NB, true>(tl.bx, tl.by, h, smem, 0);
 				else
-					partial_split_body<KT, NA, NB, KT == 16>(tl.bx, tl.by, h, smem, 0);
+					partial_split_body<KT, NA, NB, false>(tl.bx, tl.by, h, smem, 0);
 			} else if constexpr (KT == 16) {
 				// a rank up to 4 or 8 sums only its columns in GEMM1 (nmfk_plan_set_rank)
 				const uint32_t ke = half == 0 ? J.planH.ke : J.planW.ke;
@@ -3072,8 +3038,11 @@ __global__ __launch_bounds__(NMFK_WG) void k_batch_finish(const nmfk_bjob *__res
 		const fin_args f = batch_fin(J, half, clamp);
 		const int S = half == 0 ? J.planH.S : J.planW.S, p = half == 0 ? J.m : J.n, tid = threadIdx.x;
 		switch (J.kt + J.split) {
-#define X(K, PAIR)                                                                                     	case K + PAIR:                                                                                 		finish_block<K, PAIR, false, false>(tl.bx, tid, J.part, S, f.A, p, f.k, f.den, f.colA, f.clamp, nullptr, smem); 		break;
-			X(4, false) X(8, false) X(16, false) X(16, true) X(32, false) X(32, true)
+#define X(K, PAIR)                                                                                     \
+	case K + PAIR:                                                                                 \
+		finish_block<K, PAIR, false, false>(tl.bx, tid, J.part, S, f.A, p, f.k, f.den, f.colA, f.clamp, nullptr, smem); \
+		break;
+			X(4, false) X(8, false) X(16, false) X(32, false) X(32, true)
 #undef X
 		}
 		__syncthreads();
@@ -3670,21 +3639,21 @@ extern "C" void nmfk_plan_set_rank(nmfk_hplan *pl, uint32_t kt, uint32_t k)
 }
 
 // Resident jobs on the FP32 matrix-core path, planned on their own, that run on split products
-// (partial_split_body).  Per iteration, FP32 instructions against split products: k = 16 (12),
-// 5000 x 500 21.3 / 21.4 us, 10000 x 500 27.3 / 27.6, 8000 x 1000 30.3 / 28.8, 20000 x 500 36.0 /
-// 34.1, 20000 x 1000 45.9 / 43.7: at kt 16 the line lies between 5 and 8 million values, below
-// which a block's longer chain costs what the shorter products save.  At kt 32 and 64 they are
-// faster at every size (k = 24 or 32: 3000 x 300 26.4 / 24.5, 1000 x 1000 27.5 / 24.8, 20000 x
-// 1000 74.7 / 58.8; k = 48: 10000 x 1000 95.3 / 71.1); smaller jobs were left out while all sums were
-// kept in the matrix instructions (see split_fresh), for 7 of 78 shapes of 1 to 6 million values
-// whose W and H then came out more than 1.5 times as far from 64 bits.  Errors now, over 120
-// drawn jobs of 6 to 60 million values, k = 9..64, planted and lognormal, 10-100 iterations: 0.76
-// times those of the FP32 instructions in the mean, 1.2 times at most.  Other seeds of lognormal ones
-// scatter more, as the FP32 instructions do between two plans: 6 of 82 over 1.5 times, 20 under 1/1.5.
-// Jobs planned to 96 workgroups: 0.64 times in the mean (1.1 with all sums kept).
+// (partial_split_body): kt 32 and 64, where they are faster at every size.  Per iteration, FP32
+// instructions against split products: k = 24 or 32, 3000 x 300 26.4 / 24.5 us, 1000 x 1000 27.5 /
+// 24.8, 20000 x 1000 69.9 / 55.4; k = 20, 60000 x 500 97.2 / 70.8; k = 48, 30000 x 1000 185 / 126.
+// Smaller jobs were left out while all sums were kept in the matrix instructions (see split_fresh),
+// for 7 of 78 shapes of 1 to 6 million values whose W and H then came out more than 1.5 times
+// as far from 64 bits.  Errors now, over 86 drawn jobs of 6 to 60 million values, k = 17..64, planted and
+// lognormal, 10-100 iterations: 0.78 times those of the FP32 instructions in the mean, 1.2 times at
+// most.  Other seeds of lognormal ones scatter more, as the FP32 instructions do between two
+// plans: 6 of 82 over 1.5 times, 20 under 1 / 1.5.
+// Not at kt 16, whose block is too short to pay for the splitting: 20000 x 1000, k = 16 44.7 / 42.6, but 40000
+// x 1000 83.6 / 89.3, 60000 x 110 31.9 / 34.4, 60000 x 1000, k = 12 122.3 / 121.6, and 1-4 us more with operands
+// scaled so that their parts hold every number.
 extern "C" int nmfk_split_rule(uint32_t n, uint32_t m, uint32_t kt, uint32_t k)
 {
-	return kt % 16u == 0 && k > 8u && (size_t)n * m >= (6u << 20);
+	return kt % 32u == 0 && k > 16u && (size_t)n * m >= (6u << 20);
 }
 
 extern "C" void nmfk_plan_half(uint32_t p, uint32_t q, uint32_t kt, nmfk_hplan *pl)
@@ -3761,16 +3730,19 @@ static int launch_half_mfma(const nmfk_half *g, const nmfk_hplan *pl, const nmfk
 	    !kernel_args(g, pl, fin, 64u * na, &h, &f, &grid))
 		return (int)hipErrorInvalidValue;
 	if (g->split) {
+		if constexpr (KT >= 32) {
+			const bool fresh = split_fresh(KT, h.bchunk, nb);
 #define X(NA_, NB_)                                                                                    \
 	if (na == NA_ && nb == NB_) {                                                                  \
-		if (split_fresh(KT, h.bchunk, NB_))                                                    \
+		if (fresh)                                                                             \
 			hipLaunchKernelGGL((k_partial_split<KT, NA_, NB_, true>), grid, dim3(64 * NA_ * NB_), 0, stream, h, f, st); \
 		else                                                                                   \
-			hipLaunchKernelGGL((k_partial_split<KT, NA_, NB_, KT == 16>), grid, dim3(64 * NA_ * NB_), 0, stream, h, f, st); \
+			hipLaunchKernelGGL((k_partial_split<KT, NA_, NB_, false>), grid, dim3(64 * NA_ * NB_), 0, stream, h, f, st); \
 		return (int)hipGetLastError();                                                         \
 	}
-		NMFK_SHAPE_LIST(X)
+			NMFK_SHAPE_LIST(X)
 #undef X
+		}
 		return (int)hipErrorInvalidValue;
 	}
 	// A rank up to 4 or 8 at KT 16 sums only its columns in GEMM1 (the default shapes have
@@ -3870,7 +3842,7 @@ extern "C" int nmfk_launch_finish(const float *part, uint32_t S, uint32_t p, uin
 		return (int)hipGetLastError();                                                         \
 	}
 	X(4, false) X(8, false) X(16, false) X(32, false) X(64, false)
-	X(16, true) X(32, true) X(64, true)
+	X(32, true) X(64, true)
 #undef X
 	return (int)hipErrorInvalidValue;
 }
@@ -3958,7 +3930,7 @@ extern "C" int nmfk_launch_colsum_parts(const float *A, uint32_t p, uint32_t kt,
 	case K:                                                                                   \
 		hipLaunchKernelGGL((k_colsum_parts<K, true>), dim3(g), dim3(NMFK_WG), 0, stream, A, (int)p, colA); \
 		return (int)hipGetLastError();
-			NMFK_KT_MFMA_LIST(X)
+			X(32) X(64)
 #undef X
 		default:
 			return (int)hipErrorInvalidValue;
@@ -4040,12 +4012,6 @@ extern "C" int nmfk_launch_batch_partial(const nmfk_bjob *jobs, const nmfk_tile 
 		break;
 	case 7:
 		hipLaunchKernelGGL((k_batch_partial<7>), g, dim3(NMFK_WG), 0, stream, jobs, tiles, (int)ntiles, half);
-		break;
-	case 8:
-		hipLaunchKernelGGL((k_batch_partial<8>), g, dim3(NMFK_WG), 0, stream, jobs, tiles, (int)ntiles, half);
-		break;
-	case 9:
-		hipLaunchKernelGGL((k_batch_partial<9>), g, dim3(NMFK_WG), 0, stream, jobs, tiles, (int)ntiles, half);
 		break;
 	default:
 		return (int)hipErrorInvalidValue;

@@ -135,11 +135,11 @@ int nmfk_job_kernel_path(const nmfk_job *job);
 /* How the FP32 matrix-core path (2, or automatic up to k = 32) forms its products: on the FP32
  * matrix instructions, or as split products, sums of six products of operands in three BF16 parts
  * each, accumulated in FP32.  Split products are as near to 64 bits (the sums' order, and so
- * the last bits, are others) and faster on large jobs.  NMFK_SPLIT_AUTO (default): split
- * products for k > 8 and n m >= 6 Mi (nmfk_split_rule), unless the job is replanned to a
+ * the last bits, are others) and faster for k > 16.  NMFK_SPLIT_AUTO (default): split
+ * products for k > 16 and n m >= 6 Mi (nmfk_split_rule), unless the job is replanned to a
  * workgroup target, which is meant for many jobs at once.  NMFK_SPLIT_OFF: always the FP32
- * instructions, on any path and plan.  NMFK_SPLIT_ON: split products whenever both half-steps are on
- * the FP32 matrix-core path.  Jobs of a rank sweep and of the serving loop are set to
+ * instructions, on any path and plan.  NMFK_SPLIT_ON: split products whenever the job is on the FP32
+ * matrix-core path at a padded rank of 32 or 64.  Jobs of a rank sweep and of the serving loop are set to
  * NMFK_SPLIT_OFF.  Streamed jobs always run the FP32 instructions, and refuse the call. */
 #define NMFK_SPLIT_AUTO 0
 #define NMFK_SPLIT_OFF 1

@@ -303,7 +303,7 @@ def test_rows_too_long_for_the_matrix_cores_are_refused(nmfk):
 def test_sweep_jobs_run_the_fp32_instructions(nmfk, mode, autotune):
     # A matrix large enough for split products: whatever the mode and whatever plan the search picks,
     # the jobs give the bits of a lone job on the FP32 instructions at that plan.
-    n, m, ks = 6401, 1087, (12, 20)
+    n, m, ks = 6401, 1087, (18, 24)
     with nmfk.Job(n, m, 1) as src:
         src.gen_V_lognormal(3, 0.0, 1.0)
         r = nmfk.sweep(src, ks, 1, 5, nIters=10, niter_test_conv=5, stop_threshold=1000, mode=mode, autotune=autotune,

@@ -119,7 +119,7 @@ def test_served_requests_same_alone_and_in_mix(nmfk, c4_served):
 def test_served_jobs_run_the_fp32_instructions(nmfk, target):
     # A request large enough for split products gives the bits of a lone job on the FP32 instructions
     # at the served plan, also where that plan is the lone one.
-    n, m, k, seed = 6401, 1087, 14, 21
+    n, m, k, seed = 6401, 1087, 24, 21
     out, _ = nmfk.serve([(n, m, k, 1, seed, 0.0)], nIters=10, niter_test_conv=5, stop_threshold=1000, plan_target=target,
                         detail=True, factors_of=[0])
     got = out[0]["restarts"][0]
