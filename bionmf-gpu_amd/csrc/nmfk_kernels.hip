@@ -1529,11 +1529,11 @@ __global__ __launch_bounds__(64 * NA * NB) void k_partial_bf16(half_args h, bf16
 // formed from the six partial products of relative size 2^-16 and more (x1 y1, x1 y2, x2 y1,
 // x2 y2, x1 y3, x3 y1), accumulated in FP32 by v_mfma_f32_16x16x32_bf16; the three left out
 // are below 2^-24.  Sums of 32, 64 and 256 products came out 3.4e-8, 7.4e-8 and 1.9e-7 rms
-// from the 64-bit sums, against 8.8e-8, 1.2e-7 and 2.4e-7 on the FP32 instructions.  Exact for
-// operands of 7.7e-34 and more (bits below 2^-133 are lost); infinities see partial_split_body.
+// from the 64-bit sums, against 8.8e-8, 1.2e-7 and 2.4e-7 on the FP32 instructions.  The parts hold
+// every operand (see SPLIT_UP); for very large values and infinities see partial_split_body.
 //
 // What bounds the FP32 instructions is their rate: 16x16x4 takes 32 cycles, 2048 per 16-row
-// block and 64 rows a at KT 32, 4096 at KT 64.  The split products take 768 and 1536, and 150-180
+// block and 64 rows a at KT 32, 4096 at KT 64.  The split products take 768 and 1536, and 180-200
 // vector instructions for the ratios and the splitting.  Ownership of rows, blocks and wave groups
 // is that of the body above; per 16-row block a wave
 //   stages B (fetched as FP32, one block ahead) in its own LDS slot in three parts, row-major,
@@ -1584,6 +1584,19 @@ __device__ __forceinline__ void split3x4(float a, float b, float c, float d, bf1
 #pragma unroll
 	for (int i = 0; i < 3; i++)
 		p[i] = __builtin_shufflevector(lo[i], hi[i], 0, 1, 2, 3);
+}
+
+// Operands of split products are multiplied by 2^16 before they are split, so that the three parts
+// hold every bit of every FP32 number: a BF16 number ends at 2^-133, an FP32 number at 2^-149.  Then the
+// dot products of A and B come out times 2^32, and the ratios are formed from U times 2^48.  Without
+// this the parts of numbers below 7.7e-34 lose bits: half-steps on a V of about 3e-37 and of 1e-35 came
+// out 4.0e-4 and 3.7e-5 off, and 1e-5 is the bar.  It costs 24 of 180 vector instructions per block at KT
+// 32: 20000 x 1000, k = 32 54.3 -> 56.7 us per iteration, 8000 x 1000, k = 24 34.5 -> 35.0, 50000 x 2000,
+// k = 64 320 -> 328.
+#define SPLIT_UP 0x1p16f
+__device__ __forceinline__ float4 scale_up(float4 x)
+{
+	return make_float4(x.x * SPLIT_UP, x.y * SPLIT_UP, x.z * SPLIT_UP, x.w * SPLIT_UP);
 }
 
 __device__ __forceinline__ bf16x8 cat8(bf16x4 lo, bf16x4 hi)
@@ -1707,6 +1720,7 @@ __device__ __forceinline__ void partial_split_body(int bx, int by, const half_ar
 
 	// GEMM1's A operands.
 	bf16x8 aq[4][CH][3];
+	float bigA = 0.0f, bigB = 0.0f;   // the largest scaled values of A and of B that the lane saw
 #pragma unroll
 	for (int t = 0; t < 4; t++) {
 		const bool ok = t < avail;
@@ -1718,6 +1732,12 @@ __device__ __forceinline__ void partial_split_body(int bx, int by, const half_ar
 			float4 hi = *reinterpret_cast<const float4 *>(Ac + 4);
 			if (!ok)
 				lo = hi = make_float4(0.f, 0.f, 0.f, 0.f);
+			lo = scale_up(lo), hi = scale_up(hi);
+			// (the instruction by name: a tree of fmaxf would keep all of A's rows in registers)
+			asm("v_max3_f32 %0, %0, |%1|, |%2|" : "+v"(bigA) : "v"(lo.x), "v"(lo.y));
+			asm("v_max3_f32 %0, %0, |%1|, |%2|" : "+v"(bigA) : "v"(lo.z), "v"(lo.w));
+			asm("v_max3_f32 %0, %0, |%1|, |%2|" : "+v"(bigA) : "v"(hi.x), "v"(hi.y));
+			asm("v_max3_f32 %0, %0, |%1|, |%2|" : "+v"(bigA) : "v"(hi.z), "v"(hi.w));
 			bf16x4 pl[3], ph[3];
 			split3x4(lo.x, lo.y, lo.z, lo.w, pl);
 			split3x4(hi.x, hi.y, hi.z, hi.w, ph);
@@ -1740,7 +1760,9 @@ __device__ __forceinline__ void partial_split_body(int bx, int by, const half_ar
 		for (int h = 0; h < H; h++) {
 			const int e = (h * 64 + lane) * 4, row = e / KT, col = e % KT;
 			bf16x4 pt[3];
-			split3x4(b[h].x, b[h].y, b[h].z, b[h].w, pt);
+			const float4 v = scale_up(b[h]);
+			bigB = fmaxf(fmaxf(bigB, fmaxf(fabsf(v.x), fabsf(v.y))), fmaxf(fabsf(v.z), fabsf(v.w)));
+			split3x4(v.x, v.y, v.z, v.w, pt);
 #pragma unroll
 			for (int i = 0; i < 3; i++)
 				*reinterpret_cast<bf16x4 *>(slot + (i * 16 + row) * BS + col) = pt[i];
@@ -1774,7 +1796,7 @@ __device__ __forceinline__ void partial_split_body(int bx, int by, const half_ar
 #pragma unroll
 			for (int r = 0; r < 4; r++) {
 				const float uv = t == 0 ? u[r].x : t == 1 ? u[r].y : t == 2 ? u[r].z : u[r].w;
-				const float v = uv * __builtin_amdgcn_rcpf(s[t][r]);
+				const float v = uv * (SPLIT_UP * SPLIT_UP * SPLIT_UP) * __builtin_amdgcn_rcpf(s[t][r]);
 				rt[r] = !MASK || bb + 4 * g + r < b_end ? v : 0.0f;
 			}
 			split3x4(rt[0], rt[1], rt[2], rt[3], pr[t]);
@@ -1848,9 +1870,10 @@ __device__ __forceinline__ void partial_split_body(int bx, int by, const half_ar
 		ratio(u, s, bb, std::true_type{});
 		gemm2();
 	}
-	// Splitting an infinity leaves NaN: where a sum is not finite, the wave's whole share is
-	// summed again on the FP32 instructions, so infinities and NaN come out as those give them.
-	// (Rows a past p divide by zero and are never stored: not looked at.)
+	// Splitting an infinity leaves NaN, also one that the scaling made, and a product of A and B has no
+	// reciprocal from 2^126 on: where a sum is not finite, or such a product can be, the wave's whole
+	// share is summed again on the FP32 instructions, so that very large values, infinities and NaN
+	// come out as those give them.  (Rows a past p divide by zero and are never stored: not looked at.)
 	float z = 0.0f;
 #pragma unroll
 	for (int t = 0; t < 4; t++)
@@ -1858,11 +1881,22 @@ __device__ __forceinline__ void partial_split_body(int bx, int by, const half_ar
 		for (int r = 0; r < 4; r++) {
 			float y = 0.0f;
 #pragma unroll
-			for (int h = 0; h < H; h++)
+			for (int h = 0; h < H; h++) {
 				y = fmaf(acc[t][h][r], 0.0f, y);
+				acc[t][h][r] *= 1.0f / (SPLIT_UP * SPLIT_UP);
+			}
 			z += a0 + 4 * (4 * g + r) + t < p ? y : 0.0f;
 		}
-	if (__builtin_expect(!idle && __any(z != 0.0f), 0))
+	bool redo = __any(z != 0.0f);
+	if (__builtin_expect(__any(!(fmaxf(bigA, bigB) < 0x1p60f)), 0)) {   // else KT products stay below 2^126
+#pragma unroll
+		for (int off = 32; off >= 1; off >>= 1) {
+			bigA = fmaxf(bigA, __shfl_xor(bigA, off, 64));
+			bigB = fmaxf(bigB, __shfl_xor(bigB, off, 64));
+		}
+		redo |= !(bigA * bigB < 0x1p126f / KT);
+	}
+	if (__builtin_expect(!idle && redo, 0))
 		sum32<KT, NB>(ha, aj, wb, b_begin, b_end, acc);
 	if constexpr (NB > 1)
 		__syncthreads();   // every wave is done with its slot, which the sums below reuse

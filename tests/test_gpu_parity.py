@@ -291,6 +291,97 @@ def test_split_products_do_not_lose_long_sums(nmfk, orc, n, m, k):
         assert abs(np.mean(job.get_H() / want) - 1.0) < 2.0 ** -25
 
 
+def each_rel_err(got, want):
+    """Largest relative error of any single value."""
+    return float(np.max(np.abs(got.astype(np.float64) - want) / np.maximum(np.abs(want), 1e-300)))
+
+
+def split_half_steps(nmfk, orc, V, W, H):
+    """Both half-steps on split products and in 64 bits, W from the device's own H."""
+    n, m, k = *V.shape, W.shape[1]
+    with nmfk.Job(n, m, k) as job:
+        job.set_V(V)
+        job.set_kernel_path(2)
+        job.set_split(job.SPLIT_ON)
+        assert job.split()
+        job.set_WH(W, H)
+        job.update_H()
+        H1 = job.get_H()
+        job.update_W()
+        return H1, orc.update_H(V, W, H), job.get_W(), orc.update_W(V, W, H1)
+
+
+@pytest.mark.parametrize("scale", [3e-37, 1e-35, 1e-33, 1e18, 1e24, 1e30])
+@pytest.mark.parametrize("n,m,k", [(700, 150, 24), (333, 150, 20), (700, 65, 40)])
+def test_split_products_at_any_scale_of_V(nmfk, orc, n, m, k, scale):
+    # Every value of H and W, not only the large ones, within the FP32 bar of a half-step: ratios near
+    # the lowest and products near the highest numbers.
+    V = (orc.gen_lognormal(n, m, 3, 0.0, 0.5).astype(np.float64) * scale).astype(np.float32)
+    W, H = orc.init_WH(n, m, k, 5)
+    H1, want_H, W1, want_W = split_half_steps(nmfk, orc, V, W + np.float32(0.1), H + np.float32(0.1))
+    assert each_rel_err(H1, want_H) < 1e-5 and each_rel_err(W1, want_W) < 1e-5
+
+
+@pytest.mark.parametrize("n,m,k", [(700, 150, 24), (333, 150, 20), (700, 65, 40)])
+def test_split_products_keep_tiny_factors(nmfk, orc, n, m, k):
+    # Factors with components on their way to zero and at the clamp (1.18e-38): their columns of the
+    # other factor come from sums of such values alone.
+    rng = np.random.default_rng(n)
+    V = orc.gen_lognormal(n, m, 3, 3.0, 0.5)
+    W, H = (x + np.float32(0.1) for x in orc.init_WH(n, m, k, 5))
+    W[:, 1] *= np.float32(1e-35)
+    W[:, 3] = np.float32(1.17549435e-38)
+    W[:, 4] = np.exp(rng.uniform(np.log(1e-36), np.log(1e-33), n)).astype(np.float32)
+    H[rng.random(H.shape) < 0.2] = np.float32(1.17549435e-38)
+    H[:, 5] *= np.float32(1e-34)
+    H1, want_H, W1, want_W = split_half_steps(nmfk, orc, V, W, H)
+    ok = np.abs(want_H) > 1e-36   # below, FP32 itself runs out of digits
+    assert each_rel_err(H1[ok], want_H[ok]) < 1e-5
+    ok = np.abs(want_W) > 1e-36
+    assert each_rel_err(W1[ok], want_W[ok]) < 1e-5
+
+
+@pytest.mark.parametrize("n,m,k", [(700, 150, 24), (333, 150, 20), (700, 65, 40)])
+def test_split_products_of_large_factors(nmfk, orc, n, m, k):
+    # Products of the factors of 1e29 and more against a V of about 1: ratios of 1e-30 that do not vanish.
+    V = orc.gen_lognormal(n, m, 3, 0.0, 0.5)
+    W, H = orc.init_WH(n, m, k, 5)
+    W, H = (W + np.float32(0.1)) * np.float32(1e15), (H + np.float32(0.1)) * np.float32(3e14)
+    H1, want_H, W1, want_W = split_half_steps(nmfk, orc, V, W, H)
+    assert each_rel_err(H1, want_H) < 1e-5 and each_rel_err(W1, want_W) < 1e-5
+
+
+@pytest.mark.parametrize("n,m,k", [(700, 150, 24), (333, 150, 20), (700, 65, 40)])
+def test_split_products_with_an_empty_row_or_column(nmfk, orc, n, m, k):
+    # A row of V without any value: its row of W goes to the clamp, and all others stay right (four
+    # iterations at the bar of one half-step each).  A column without any makes its row of H zero, and
+    # 0 / 0 in the W half-step: NaN where the FP32 instructions have it.
+    V = orc.gen_lognormal(n, m, 3, 5.0, 1.0)
+    V[17] = 0.0
+    W, H = orc.init_WH(n, m, k, 5)
+    ref = orc.nmf(V, W, H, 4, 1, 1000, fp64=True)
+    with nmfk.Job(n, m, k) as job:
+        job.set_V(V)
+        job.set_kernel_path(2)
+        job.set_split(job.SPLIT_ON)
+        job.set_WH(W, H)
+        job.run(4, 1, 1000)
+        W1, H1 = job.get_W(), job.get_H()
+        assert np.all(W1[17] == np.float32(1.17549435e-38))
+        assert rel_err(H1, ref["H"]) < 4e-5 and rel_err(W1, ref["W"]) < 4e-5
+        V[:, 9] = 0.0
+        job.set_V(V)
+        got = []
+        for mode in (job.SPLIT_ON, job.SPLIT_OFF):
+            job.set_split(mode)
+            job.set_WH(W, H)
+            job.update_H()
+            assert np.all(job.get_H()[9] == 0.0)
+            job.update_W()
+            got.append(np.isnan(job.get_W()))
+        assert got[0].any() and np.array_equal(*got)
+
+
 @pytest.mark.parametrize("n,m,k,wide", [(900, 130, 30, 1), (12000, 1100, 30, 2)])
 def test_split_products_same_bits_in_every_batch_class(nmfk, orc, n, m, k, wide):
     # 1 x 4 and (W halves of 1000-4095 columns and enough rows) 2 x 2 waves; split products at any size when asked for, beside a job on the FP32 instructions in the same batch.
