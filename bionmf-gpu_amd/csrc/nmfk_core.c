@@ -1052,8 +1052,14 @@ int nmfk_job_dot_kl(nmfk_job *j, double *dot_V, double *dot_VWH, double *kl)
 
 /* ---------------------------------------------------------------- timing */
 
+/* kind 0: whole iterations; 1 and 3: the sums of the H and of the W half; 2 and 4: their finishes.  A
+ * half-step of one split is one launch, and timed as such by its sums' kind; its finish takes 0. */
 static int time_loop(nmfk_job *j, uint32_t iters, int kind, double *ms)
 {
+	const int half = kind >= 3, one_launch = kind && (half ? j->planW : j->planH).S == 1;
+	*ms = 0.0;
+	if (one_launch && kind % 2 == 0)
+		return 0;
 	hipEvent_t a, b;
 	int e = hipEventCreate(&a);
 	if (!e)
@@ -1068,24 +1074,12 @@ static int time_loop(nmfk_job *j, uint32_t iters, int kind, double *ms)
 	if (!e)
 		e = hipEventRecord(a, j->stream);
 	for (uint32_t i = 0; i < iters && !e; i++) {
-		switch (kind) {
-		case 0:
+		if (kind == 0) {
 			e = nmfk_enqueue_half_H(j, NULL);
 			if (!e)
 				e = nmfk_enqueue_half_W(j, NULL, 0);
-			break;
-		case 1:
-			e = half_step(j, 0, HALF_SUMS, 0, NULL);
-			break;
-		case 2:
-			e = half_step(j, 0, HALF_FINISH, 0, NULL);
-			break;
-		case 3:
-			e = half_step(j, 1, HALF_SUMS, 0, NULL);
-			break;
-		case 4:
-			e = half_step(j, 1, HALF_FINISH, 0, NULL);
-			break;
+		} else {
+			e = half_step(j, half, one_launch ? HALF_WHOLE : kind % 2 ? HALF_SUMS : HALF_FINISH, 0, NULL);
 		}
 	}
 	if (!e)

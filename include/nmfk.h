@@ -377,7 +377,8 @@ typedef struct nmfk_job_info {
 int nmfk_job_info_get(const nmfk_job *job, nmfk_job_info *info);
 
 /* Times <iters> full iterations (both half-steps, no tests) with HIP events on the job's
- * stream; returns the average ms per iteration and per kernel kind. */
+ * stream; returns the average ms per iteration and per kernel kind.  A half-step planned with
+ * one split is one launch: ms_partial_* is that launch, its finish included, and ms_finish_* 0. */
 typedef struct nmfk_timing {
 	double ms_per_iter;
 	double ms_partial_H, ms_finish_H, ms_partial_W, ms_finish_W;

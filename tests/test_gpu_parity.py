@@ -799,3 +799,16 @@ def test_dot_kl_of_very_long_rows(nmfk, orc, n, m, k, ldv):
     dv, dvwh = orc.dot_VWH(V.astype(np.float64), W.astype(np.float64), H.astype(np.float64))
     kl = orc.kl_div(V, W, H, fp64=True)
     assert abs(out[0] - dv) / dv < 1e-12 and abs(out[1] - dvwh) / dvwh < 1e-9 and abs(out[2] - kl) / kl < 1e-9
+
+
+@pytest.mark.parametrize("n,m,k,path", [(2111, 63, 16, 2), (60, 5000, 9, 2), (2111, 63, 48, 3), (5000, 20, 4, 1), (4000, 1500, 12, 2)])
+def test_timing_describes_the_launches_of_a_run(nmfk, n, m, k, path):
+    # A half-step of one split is one launch, whose finish has no time of its own.
+    with nmfk.Job(n, m, k) as job:
+        job.set_kernel_path(path)
+        job.gen_V_lognormal(3, 0.0, 1.0)
+        job.init_random(4)
+        t, pl = job.time_iterations(3), job.plan()
+        assert t["ms_per_iter"] > 0
+        for half in "HW":
+            assert t[f"ms_partial_{half}"] > 0 and (t[f"ms_finish_{half}"] == 0) == (pl[half]["S"] == 1)
