@@ -214,6 +214,28 @@ def load_fixture(name):
     return np.load(f) if f.exists() else None
 
 
+def partial_kernels(job) -> str:
+    """The kernels of a job's two half-steps, from its plan (kt <= 32, default workgroup shapes)."""
+    inf, names = job.info(), []
+    for half, p in (("H", inf.m), ("W", inf.n)):
+        pl = job.plan()[half]
+        if pl["path"] == KERNEL_PATHS["valu"]:
+            names.append(f"k_partial<{inf.kt},...> ({half} half)")
+            continue
+        na = next(a for a in (1, 2, 4) if -(-p // (64 * a)) == pl["nab"])
+        names.append(f"{'k_partial_split' if job.split() else 'k_partial_mfma'}<{inf.kt},{na},{4 // na}> ({half} half)")
+    return ", ".join(names)
+
+
+def measured_traffic(kernels: str):
+    """HBM bytes per launch from the profile of these kernels on the headline workload, if there is one."""
+    for f in sorted((ROOT / "profiles").glob("traffic_*.json")):
+        t = json.loads(f.read_text())
+        if t.get("kernel") == kernels and t.get("workload", "").startswith(f"V {N}x{M}, k={K} "):
+            return t.get("bytes_per_launch")
+    return None
+
+
 def bench_dense_rank(pkg) -> dict:
     """Dense rank: V 50000 x 2000 planted rank 48, k = 64, 300 iterations: BF16 contractions
     (FP32 accumulation) against the FP32 matrix-core path on the same start, and both
@@ -474,10 +496,8 @@ def main():
     achieved = bytes_partial / (ms * 1e-3) / 1e9
     iter_bytes = 4.0 * (2 * N * M + 3 * N * K + 3 * M * K)
     read_gbs, copy_gbs = pkg.measure_stream(1 << 30, 10, 4096)
-    traffic = None
-    tfile = ROOT / "profiles" / "traffic_partial_mfma_20000x1000_k16.json"
-    if tfile.exists() and args.kernel_path == "auto":
-        traffic = json.loads(tfile.read_text()).get("bytes_per_launch")
+    kernels = partial_kernels(job)
+    traffic = measured_traffic(kernels)
 
     # The one-pass schedule (one pass over V per iteration: k_fused_mfma + k_fused_finish) on
     # the same job, timed the same way; reported beside the default two-pass schedule.
@@ -542,9 +562,7 @@ def main():
         "vs_fp64": accuracy,
         "roofline": {"bound": "hbm", "achieved": achieved, "peak": HBM_PEAK_GBS,
                      "unit": "GB/s", "frac": achieved / HBM_PEAK_GBS, "traffic": traffic,
-                     "kernel": ("k_partial_split<16,1,4> (H half) and k_partial_split<16,2,2> (W half)"
-                                if args.kernel_path in ("auto", "mfma32")
-                                else "k_partial<16,...> (vector ALUs, both half-steps)"),
+                     "kernel": kernels,
                      "bytes_per_launch": bytes_partial, "ms_per_launch": ms,
                      "measured_read_GBps": read_gbs, "measured_copy_GBps": copy_gbs,
                      "frac_of_measured_read": achieved / read_gbs},
