@@ -775,7 +775,7 @@ static int half_step(nmfk_job *j, int half, int what, int clamp, const nmfk_stat
 	if (what == HALF_FINISH)
 		return nmfk_launch_finish(j->part, pl->S, g.p, j->kt, j->split, &f, st, j->stream);
 	if (what == HALF_LONE) {
-		if (!j->split && g.q <= NMFK_DEN_ROWS)
+		if (!j->split && g.q <= (pl->S == 1 ? NMFK_DEN_ROWS_ONE : NMFK_DEN_ROWS))
 			f.colB = NULL;
 		else if ((e = nmfk_launch_colsum_parts(g.B, g.q, j->kt, j->split, half ? j->colH : j->colW, j->stream)) != 0)
 			return e;

@@ -111,7 +111,13 @@ typedef struct nmfk_fin {
 	uint32_t k;
 	int clamp;
 } nmfk_fin;
-#define NMFK_DEN_ROWS 1024
+#define NMFK_DEN_ROWS 1024     /* as many as the kernels have LDS for */
+/* Up to which a lone half-step of one split takes them from B: every one of its workgroups then
+ * reads all of B (with more splits one workgroup does, beside the others).  Against a launch of
+ * their own for the column sums: 16000 x 256, k = 10 9.1 / 10.0 us, 60000 x 256, k = 48 28.5 / 30.0, but
+ * 30000 x 300, k = 48 24.4 / 23.8, 60000 x 1000, k = 64 60.9 / 57.6.  With more splits, 1000 rows: 20000 x
+ * 1000, k = 64 32.1 / 35.6, 1000 x 1000, k = 30 13.3 / 15.8. */
+#define NMFK_DEN_ROWS_ONE 256
 int nmfk_launch_half(const nmfk_half *g, const nmfk_hplan *pl, const nmfk_fin *fin, const nmfk_state *st,
 		     hipStream_t stream);
 

@@ -218,6 +218,20 @@ def test_lone_half_steps_give_the_bits_of_a_run(nmfk, orc, n, m, k, path):
         assert np.array_equal(a.get_H(), b.get_H()) and np.array_equal(a.get_W(), b.get_W())
 
 
+@pytest.mark.parametrize("n,m", [(16000, 256), (16000, 257)])
+def test_lone_half_steps_of_one_split_give_the_bits_of_a_run(nmfk, orc, n, m):
+    # W half-steps of one split on both sides of the line between denominators from H itself and from
+    # its column sums.
+    jobs = [make_job(nmfk, orc, n, m, 48, seed_v=n, seed_init=m)[0] for _ in range(2)]
+    with jobs[0] as a, jobs[1] as b:
+        assert a.kernel_path() == 3 and a.plan()["W"]["S"] == 1
+        a.run(2, 1000, 1000)
+        for _ in range(2):
+            b.update_H()
+            b.update_W()
+        assert np.array_equal(a.get_H(), b.get_H()) and np.array_equal(a.get_W(), b.get_W())
+
+
 def test_split_products_are_a_property_of_the_job(nmfk):
     # Automatic: by size and rank, for a job planned on its own.  On or off holds for every plan;
     # neither has an effect off the FP32 matrix cores, or at padded ranks below 32.
