@@ -31,27 +31,14 @@
 enum { TAB_PART_H0, TAB_PART_W0 = TAB_PART_H0 + NCLS, TAB_SHORT_H = TAB_PART_W0 + NCLS, TAB_SHORT_W, TAB_FIN_H, TAB_FIN_W,
        TAB_TEST, NTAB };
 
-/* Half-steps that one wave per row group sums and finishes (nmfk_launch_batch_short); they have
- * tables of their own, and no finish or denominator tiles. */
-static int half_short(const nmfk_job *j, int half)
+/* Half-steps that one wave per row group can sum and finish (nmfk_launch_batch_short). */
+static int short_fits(const nmfk_job *j, int half)
 {
 	const nmfk_hplan *p = half ? &j->planW : &j->planH;
 	return j->kt == 16 && p->ap == 1 && p->S == 1 && (half ? j->m : j->n) <= NMFK_SHORT_Q;
 }
-
-static int half_cls(const nmfk_job *j, int half)
-{
-	const nmfk_hplan *p = half ? &j->planW : &j->planH;
-	if (half_short(j, half))
-		return -1;
-	if (j->kt <= 8)
-		return p->lb > 1 ? 1 : 0;
-	if (j->split)
-		return p->ap == 2 ? 7 : 6;
-	return (j->kt == 16 ? 2 : 3) + (p->ap == 2 ? 2 : 0);
-}
-
 struct nmfk_batch {
+	uint32_t short_waves[2];      /* row groups of all half-steps that fit the short form */
 	uint32_t T, cap, nslots;      /* nslots: highest slot in use + 1 */
 	hipStream_t stream;
 	hipEvent_t ev;
@@ -317,8 +304,7 @@ static void push_sums(nmfk_tile *t, uint32_t *n, uint32_t job, uint32_t bx, uint
  * eighth x of their V, in table order: jobs on one V (a rank sweep) then read an eighth of it
  * through each XCD's 4 MB of L2, instead of all of it through every one, and the tiles of
  * one split of a job share the other factor's rows there.  Where the eighths do not hold equally many
- * tiles, the fullest give to the XCDs that run out. 
- * tmp: room for cnt tiles.  A burst of 33 jobs of 8 shapes at kt 16: sums 29.0 + 26.9 -> 24.2 + 24.0 us;
+ * tiles, the fullest give to the XCDs that run out.  tmp: room for cnt tiles.  A burst of 33 jobs of 8 shapes at kt 16: sums 29.0 + 26.9 -> 24.2 + 24.0 us;
  * 54 jobs at 5000 x 200: short W halves 45.3 -> 42.6 us. */
 static void spread_tiles(nmfk_tile *t, uint32_t cnt, nmfk_tile *tmp)
 {
@@ -342,6 +328,32 @@ static void spread_tiles(nmfk_tile *t, uint32_t cnt, nmfk_tile *tmp)
 	}
 }
 
+/* Half-steps that run in the short form: they have tables of their own, and no finish or
+ * denominator tiles.  A wave there walks all blocks of its rows alone, where a workgroup's four share
+ * them, so unless the range is short there have to be waves enough to keep the device busy: at least two
+ * per row of U.  Per iteration, workgroups and finishes / short form, jobs of k = 2..10: 5000 rows x 200,
+ * 4 jobs (316 waves) 35.5 / 35.6 us, 8 jobs 45.0 / 41.9, 54 jobs 133 / 100; x 256, 1 job 26.6 / 28.4, 4 jobs
+ * 35.6 / 37.5, 8 jobs (632) 45.0 / 43.4; 1000 rows x 256, 16 jobs (256) 31.3 / 35.0, 54 jobs (864) 47.1 / 43.6;
+ * x 128, 8 jobs (128) 27.1 / 27.9, 16 jobs (256) 29.1 / 28.6; x 64, 1 job 20.7 / 19.4.  Both give
+ * the same bits. */
+static int half_short(const nmfk_batch *b, const nmfk_job *j, int half)
+{
+	const uint32_t q = half ? j->m : j->n;
+	return short_fits(j, half) && (q <= 64 || b->short_waves[half] >= 2 * q);
+}
+
+static int half_cls(const nmfk_batch *b, const nmfk_job *j, int half)
+{
+	const nmfk_hplan *p = half ? &j->planW : &j->planH;
+	if (half_short(b, j, half))
+		return -1;
+	if (j->kt <= 8)
+		return p->lb > 1 ? 1 : 0;
+	if (j->split)
+		return p->ap == 2 ? 7 : 6;
+	return (j->kt == 16 ? 2 : 3) + (p->ap == 2 ? 2 : 0);
+}
+
 /* Partial tiles of one half for every live job of body class cls.  order 0: job by job;
  * order 1: split by split across jobs (round-robin), so concurrently running workgroups
  * belong to many jobs. */
@@ -349,7 +361,7 @@ static void push_partial(nmfk_batch *b, nmfk_tile *t, uint32_t *n, int half, int
 {
 	uint32_t maxS = 0;
 	for (uint32_t s = 0; s < b->nslots; s++)
-		if (b->job[s] && half_cls(b->job[s], half) == cls) {
+		if (b->job[s] && half_cls(b, b->job[s], half) == cls) {
 			const nmfk_hplan *p = half ? &b->job[s]->planW : &b->job[s]->planH;
 			push(t, n, s, p->nab, 0);   /* denominator tile first: the finish needs it */
 			if (p->S > maxS)
@@ -357,7 +369,7 @@ static void push_partial(nmfk_batch *b, nmfk_tile *t, uint32_t *n, int half, int
 		}
 	if (b->tune.order == 0) {
 		for (uint32_t s = 0; s < b->nslots; s++)
-			if (b->job[s] && half_cls(b->job[s], half) == cls) {
+			if (b->job[s] && half_cls(b, b->job[s], half) == cls) {
 				const nmfk_hplan *p = half ? &b->job[s]->planW : &b->job[s]->planH;
 				for (uint32_t by = 0; by < p->S; by++)
 					for (uint32_t bx = 0; bx < p->nab; bx++)
@@ -366,7 +378,7 @@ static void push_partial(nmfk_batch *b, nmfk_tile *t, uint32_t *n, int half, int
 	} else {
 		for (uint32_t by = 0; by < maxS; by++)
 			for (uint32_t s = 0; s < b->nslots; s++)
-				if (b->job[s] && half_cls(b->job[s], half) == cls) {
+				if (b->job[s] && half_cls(b, b->job[s], half) == cls) {
 					const nmfk_hplan *p = half ? &b->job[s]->planW : &b->job[s]->planH;
 					if (by < p->S)
 						for (uint32_t bx = 0; bx < p->nab; bx++)
@@ -396,6 +408,12 @@ static int build_tables(nmfk_batch *b)
 		b->h_tiles = t;
 		b->tiles_cap = need;
 	}
+	for (int half = 0; half < 2; half++) {
+		b->short_waves[half] = 0;
+		for (uint32_t s = 0; s < b->nslots; s++)
+			if (b->job[s] && short_fits(b->job[s], half))
+				b->short_waves[half] += half ? b->job[s]->planW.nab : b->job[s]->planH.nab;
+	}
 	uint32_t n = 0;
 	for (int half = 0; half < 2; half++)
 		for (int cls = 0; cls < NCLS; cls++) {
@@ -412,7 +430,7 @@ static int build_tables(nmfk_batch *b)
 		for (uint32_t ke = 16; ke >= 4; ke /= 2)
 			for (uint32_t s = 0; s < b->nslots; s++) {
 				const nmfk_job *j = b->job[s];
-				if (!j || !half_short(j, half) || (half ? j->planW : j->planH).ke != ke)
+				if (!j || !half_short(b, j, half) || (half ? j->planW : j->planH).ke != ke)
 					continue;
 				const nmfk_hplan *p = half ? &j->planW : &j->planH;
 				for (uint32_t bx = 0; bx < p->nab; bx++)
@@ -425,7 +443,7 @@ static int build_tables(nmfk_batch *b)
 		const int tab = TAB_FIN_H + half;
 		b->off[tab] = n;
 		for (uint32_t s = 0; s < b->nslots; s++)
-			if (b->job[s] && !half_short(b->job[s], half))
+			if (b->job[s] && !half_short(b, b->job[s], half))
 				for (uint32_t bx = 0; bx < cdiv(half ? b->job[s]->n : b->job[s]->m, NMFK_FIN_ROWS); bx++)
 					push(b->h_tiles, &n, s, bx, 0);
 		b->cnt[tab] = n - b->off[tab];

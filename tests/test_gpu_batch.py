@@ -284,6 +284,29 @@ def test_short_half_steps_same_bits_as_alone(nmfk, orc, m):
         a.close(), b.close()
 
 
+@pytest.mark.parametrize("m,njobs", [(65, 6), (128, 6), (129, 6), (200, 6), (255, 6), (256, 6), (257, 6), (200, 4), (200, 3)])
+def test_short_half_steps_in_a_full_batch(nmfk, orc, m, njobs):
+    # Ranges over 64 rows take the short form where the batch has two waves of them per row: six jobs of
+    # 98 to 110 row groups each do up to 256 rows, four of 104 to 110 do at 200, three do not.
+    specs = [(7000 - 37 * k, m, k, 30 + k, 40 + k, 20, 1000) for k in (2, 4, 9, 5, 8, 16)[:njobs]]
+    pairs = [twins(nmfk, orc, s) for s in specs]
+    for a, b in pairs:
+        for j in (a, b):
+            j.replan(1)
+            assert j.plan()["W"]["S"] == 1
+    waves = sum(a.plan()["W"]["nab"] for a, _ in pairs)
+    assert (waves >= 2 * m) == (njobs > 3 and m <= 300)
+    batch = nmfk.Batch(T, 8)
+    for (a, _), s in zip(pairs, specs):
+        batch.add(a, s[5], s[6])
+    done = dict((id(j), r) for j, r in batch.run())
+    for (a, b), s in zip(pairs, specs):
+        assert_same(a, b, done[id(a)], b.run(s[5], T, s[6]), s)
+    batch.close()
+    for a, b in pairs:
+        a.close(), b.close()
+
+
 def test_rows_too_long_for_the_matrix_cores_are_refused(nmfk):
     # 16 rows of V's transposed copy pass 2 GiB: a lone W half-step refuses such a job, and so does
     # a batch.
