@@ -193,7 +193,8 @@ int nmfk_sweep_run(nmfk_job *src, const nmfk_sweep_config *cfg, nmfk_sweep_out *
 		if (out)
 			out->plan_target = best_target;
 		nmfk_batch_tuning tn;
-		nmfk_batch_get_tuning(b, &tn);
+		if (!e)
+			nmfk_batch_get_tuning(b, &tn);
 		nmfk_job **done = (nmfk_job **)malloc(nj * sizeof(nmfk_job *));
 		nmfk_result *rs = (nmfk_result *)malloc(nj * sizeof(nmfk_result));
 		if (!done || !rs) {

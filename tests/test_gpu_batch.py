@@ -339,3 +339,15 @@ def test_sweep_jobs_run_the_fp32_instructions(nmfk, mode, autotune):
                 job.run(10, 5, 1000)
                 W, H = r["factors"][i]
                 assert np.array_equal(job.get_W(), W) and np.array_equal(job.get_H(), H)
+
+
+def test_a_sweep_that_cannot_run_is_an_error(nmfk):
+    # Ranks the batch has no kernels for: an error, also out of the plan search, which ends before
+    # there is a batch to run.
+    with nmfk.Job(300, 80, 1) as src:
+        src.gen_V_lognormal(3, 0.0, 1.0)
+        for autotune in (False, True):
+            with pytest.raises(nmfk.NmfkError, match="kernel plan"):
+                nmfk.sweep(src, (40,), 1, 5, nIters=10, niter_test_conv=5, autotune=autotune)
+        r = nmfk.sweep(src, (4,), 1, 5, nIters=10, niter_test_conv=5, autotune=True)
+        assert r["plan_target"] in (0, 8, 16, 32, 64)
