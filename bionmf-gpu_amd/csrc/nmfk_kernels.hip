@@ -3311,9 +3311,14 @@ __global__ __launch_bounds__(64 * dot_waves(KT)) void k_dot_kl(const float *__re
 	const int nsp = min((int)gridDim.y, (511 + (int)gridDim.x) / (int)gridDim.x);
 	const int rows_per = ((n + nsp - 1) / nsp + 15) & ~15;
 	const int i0 = blockIdx.y * rows_per, i1 = min(n, i0 + rows_per);
+	if (i0 >= i1) {   // a row range not in use (20 x 60000, 61 of 64: 268 -> 234 us without their reductions)
+		if (threadIdx.x < 3)
+			parts[((size_t)blockIdx.y * gridDim.x + blockIdx.x) * 3 + threadIdx.x] = 0.0;
+		return;
+	}
 	const int j0 = blockIdx.x * 256 + cw * 64, jl = j0 + 4 * l16;   // this lane's 4 columns: jl + t
 	double sv = 0.0, sd = 0.0, sk = 0.0;
-	if (rg < nrg && i0 < i1) {
+	if (rg < nrg) {
 		// GEMM operand of H: lane (g, l16) supplies H[jl + t][KQ g + q] for K step q.
 		double hop[4][KQ];
 #pragma unroll
