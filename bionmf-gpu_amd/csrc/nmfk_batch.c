@@ -304,8 +304,8 @@ static void push_sums(nmfk_tile *t, uint32_t *n, uint32_t job, uint32_t bx, uint
  * eighth x of their V, in table order: jobs on one V (a rank sweep) then read an eighth of it
  * through each XCD's 4 MB of L2, instead of all of it through every one, and the tiles of
  * one split of a job share the other factor's rows there.  Where the eighths do not hold equally many
- * tiles, the fullest give to the XCDs that run out.  tmp: room for cnt tiles.  A burst of 33 jobs of 8 shapes at kt 16: sums 29.0 + 26.9 -> 24.2 + 24.0 us;
- * 54 jobs at 5000 x 200: short W halves 45.3 -> 42.6 us. */
+ * tiles, the fullest give to the XCDs that run out.  tmp: room for cnt tiles.
+ * Per iteration: 32 jobs of 8 shapes at kt 16 172 -> 156 us; 54 jobs at 5000 x 200 95.8 -> 94.2. */
 static void spread_tiles(nmfk_tile *t, uint32_t cnt, nmfk_tile *tmp)
 {
 	uint32_t left[8] = {0}, at[8], o = 0;

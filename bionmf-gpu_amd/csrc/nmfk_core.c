@@ -2,8 +2,8 @@
  * nmfk_core.c -- host side (C99) of one KL-NMF factorization on one MI355X.
  *
  * Replaces the buffer set-up of src/GPU_setup.c:1289-1610 and the loop of
- * src/NMF_GPU.c:312-924 with a job handle.  One iteration is four launches on the job's
- * stream (H half: partial + finish, W half: partial + finish); every niter_test_conv
+ * src/NMF_GPU.c:312-924 with a job handle.  One iteration is two to four launches on the job's
+ * stream (each half: partial + finish, or both in one launch where there is one split); every niter_test_conv
  * iterations the test kernel clamps, classifies, counts the connectivity difference and
  * applies the stop rule on the device.  A whole test interval is captured once as a
  * hipGraph and replayed; the host reads the 32-byte state of interval c while interval

@@ -1545,10 +1545,10 @@ __global__ __launch_bounds__(64 * NA * NB) void k_partial_bf16(half_args h, bf16
 //          part, then in another: [r1 r3][b3 b1], [r2 r1][b2 b2], [r2 r1][b1 b1], added to the
 //          running sums or to fresh ones (see split_fresh).
 // Measured, partials of the two halves (FP32 instructions -> split): 20000 x 1000, k = 32
-// 30.9 + 31.3 -> 23.0 + 23.2 us; 50000 x 2000, k = 64 213 + 239 -> 138 + 155; 7013 x 333, k = 24 9.0 +
-// 8.3 -> 7.7 + 7.3.  GEMM1 of the next block issued beside GEMM2 of this one, with and without a
-// fixed interleave of matrix and vector instructions, and 3-6 blocks of U in flight were all
-// even or slower: two or three waves per SIMD overlap the two pipes as well.
+// 30.9 + 31.3 -> 23.4 + 23.4 us; 50000 x 2000, k = 64 213 + 239 -> 147 + 160.  GEMM1 of the next
+// block issued beside GEMM2 of this one, with and without a fixed interleave of matrix and vector
+// instructions, and 3-6 blocks of U in flight were all even or slower: two or three waves per SIMD
+// overlap the two pipes as well.
 // --------------------------------------------------------------------------------------
 
 typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
@@ -2711,7 +2711,7 @@ __device__ __forceinline__ fin_args batch_fin(const nmfk_bjob &J, int half, int 
 // apart keep the matrix cores busy.  The blocks are walked in the order that gives the bits of
 // the 1 x 4 workgroup: blocks g, g + 4, ... of each of the four wave groups in turn, each
 // group's sums added to the total in that order.  54 jobs at 5000 x 200,
-// k = 2..10: W sums 51 us and finishes 20 us -> 38.5 us, of which the matrix cores are busy 44%.
+// k = 2..10: 133 -> 100 us per iteration.
 // --------------------------------------------------------------------------------------
 
 #define NMFK_SHORT_LDS (64 * 17 + 16)   // floats per wave: its rows' sums, and the denominators
@@ -3679,8 +3679,8 @@ extern "C" void nmfk_plan_set_rank(nmfk_hplan *pl, uint32_t kt, uint32_t k)
 
 // Resident jobs on the FP32 matrix-core path, planned on their own, that run on split products
 // (partial_split_body): kt 32 and 64, where they are faster at every size.  Per iteration, FP32
-// instructions against split products: k = 24 or 32, 3000 x 300 26.4 / 24.5 us, 1000 x 1000 27.5 /
-// 24.8, 20000 x 1000 69.9 / 55.4; k = 20, 60000 x 500 97.2 / 70.8; k = 48, 30000 x 1000 185 / 126.
+// instructions against split products: k = 24 or 32, 3000 x 300 25.4 / 22.9 us, 1000 x 1000 26.1 /
+// 23.1, 20000 x 1000 70.1 / 56.5; k = 20, 60000 x 500 97.4 / 73.7; k = 48, 30000 x 1000 186 / 131.
 // Smaller jobs were left out while all sums were kept in the matrix instructions (see split_fresh),
 // for 7 of 78 shapes of 1 to 6 million values whose W and H then came out more than 1.5 times
 // as far from 64 bits.  Errors now, over 86 drawn jobs of 6 to 60 million values, k = 17..64, planted and
