@@ -250,3 +250,12 @@ def test_split_rule(lib):
         assert lib.nmfk_split_rule(n, m, lib.nmfk_job_kt(n, m, k), k) == 0, (n, m, k)
     assert lib.nmfk_split_rule(6144, 1024, 32, 17) == 1 and lib.nmfk_split_rule(6143, 1024, 32, 17) == 0
     assert lib.nmfk_split_rule(70000, 70000, 64, 64) == 1   # n m past 32 bits
+
+
+def test_rows_of_one_descriptor(lib):
+    # 16 rows of <ldu> floats within 2 GiB: the last byte offset the 16-row kernels form stays below
+    # 2^31; longer rows are refused, or read through 64-bit addresses.
+    lib.nmfk_rows16_fit.argtypes = [C.c_size_t]
+    for ldu, fits in ((4, 1), (33_554_431, 1), (33_554_432, 0), (36_000_001, 0), (1 << 40, 0)):
+        assert lib.nmfk_rows16_fit(ldu) == fits, ldu
+        assert not fits or 64 * ldu - 1 < 2 ** 31
