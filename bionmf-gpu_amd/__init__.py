@@ -496,7 +496,7 @@ class Job:
     SPLIT_AUTO, SPLIT_OFF, SPLIT_ON = 0, 1, 2
 
     def set_split(self, mode: int):
-        """Whether FP32 matrix-core half-steps run on split products (nmfk_job_set_split)."""
+        """Whether FP32 matrix-core half-steps run on split products, and how sums are added (nmfk_job_set_split)."""
         _check(self.lib.nmfk_job_set_split(self.h, mode), "set_split")
 
     def split(self) -> bool:

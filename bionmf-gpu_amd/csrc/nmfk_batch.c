@@ -35,7 +35,7 @@ enum { TAB_PART_H0, TAB_PART_W0 = TAB_PART_H0 + NCLS, TAB_SHORT_H = TAB_PART_W0 
 static int short_fits(const nmfk_job *j, int half)
 {
 	const nmfk_hplan *p = half ? &j->planW : &j->planH;
-	return j->kt == 16 && p->ap == 1 && p->S == 1 && (half ? j->m : j->n) <= NMFK_SHORT_Q;
+	return j->kt == 16 && !j->tree && p->ap == 1 && p->S == 1 && (half ? j->m : j->n) <= NMFK_SHORT_Q;
 }
 struct nmfk_batch {
 	uint32_t short_waves[2];      /* row groups of all half-steps that fit the short form */
@@ -195,7 +195,7 @@ static void fill_desc(nmfk_bjob *d, const nmfk_job *j)
 	d->ncolW = j->ncolW, d->ncolH = j->ncolH;
 	d->planH = j->planH, d->planW = j->planW;
 	d->live = 1;
-	d->split = (uint32_t)j->split;
+	d->tree = (uint32_t)j->tree;
 }
 
 int nmfk_batch_add(nmfk_batch *b, nmfk_job *j, const nmfk_options *opt)
@@ -232,7 +232,7 @@ int nmfk_batch_add(nmfk_batch *b, nmfk_job *j, const nmfk_options *opt)
 		return -1;
 	int e = nmfk_launch_state_reset(j->st, opt->stop_threshold, opt->nIters / b->T, j->last, j->m, b->stream);
 	if (!e)
-		e = nmfk_launch_colsum_parts(j->W, j->n, j->kt, j->split, j->colW, b->stream);
+		e = nmfk_launch_colsum_parts(j->W, j->n, j->kt, j->tree, j->colW, b->stream);
 	if (e) {
 		hipck(e, "nmfk_batch_add");
 		return -1;
@@ -728,7 +728,7 @@ int nmfk_batch_autotune(nmfk_batch *b, uint32_t iters, nmfk_batch_tuning *best_o
 			e2 = hipMemcpyAsync(j->H, save + o, 4 * (size_t)j->m * j->kt, hipMemcpyDeviceToDevice, b->stream);
 		o += (size_t)j->m * j->kt;
 		if (!e2)
-			e2 = nmfk_launch_colsum_parts(j->W, j->n, j->kt, j->split, j->colW, b->stream);
+			e2 = nmfk_launch_colsum_parts(j->W, j->n, j->kt, j->tree, j->colW, b->stream);
 		if (!e && e2)
 			e = e2;
 	}

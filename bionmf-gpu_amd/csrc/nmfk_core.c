@@ -328,12 +328,15 @@ nmfk_job *nmfk_job_create_shared(nmfk_job *src, uint32_t k)
 	return job_create(src->n, src->m, k, src, NULL, NULL);
 }
 
-/* Whether the job, as planned now, runs on split products (see nmfk_job_set_split). */
+/* Whether the job, as planned now, runs on split products, and whether it adds as trees (see
+ * nmfk_job_set_split). */
 static void set_split(nmfk_job *j)
 {
-	const int rule = j->target_wgs == 0 && nmfk_split_rule(j->n, j->m, j->kt, j->k);
-	j->split = j->planH.path == NMFK_PATH_MFMA32 && j->planW.path == NMFK_PATH_MFMA32 && j->kt >= 32 &&
-		   (j->split_mode == NMFK_SPLIT_ON || (j->split_mode == NMFK_SPLIT_AUTO && rule));
+	const int paths = j->planH.path == NMFK_PATH_MFMA32 && j->planW.path == NMFK_PATH_MFMA32;
+	const int own = paths && j->target_wgs == 0 && j->split_mode != NMFK_SPLIT_OFF;
+	j->split = (own && nmfk_split_rule(j->n, j->m, j->kt, j->k)) ||
+		   (paths && j->kt >= 32 && j->split_mode == NMFK_SPLIT_ON);
+	j->tree = j->split || (own && nmfk_tree_rule(j->n, j->m, j->kt, j->k));
 }
 
 static nmfk_job *job_create(uint32_t n, uint32_t m, uint32_t k, nmfk_job *src, nmfk_arena *arena,
@@ -767,17 +770,17 @@ static int half_step(nmfk_job *j, int half, int what, int clamp, const nmfk_stat
 {
 	const nmfk_hplan *pl = half ? &j->planW : &j->planH, *other = half ? &j->planH : &j->planW;
 	const nmfk_half g = {half ? j->Vt : j->V, half ? j->ldvt : j->ldv, half ? j->W : j->H, half ? j->H : j->W,
-			     half ? j->Hb : j->Wb, half ? j->n : j->m, half ? j->m : j->n, j->kt, j->split, j->part};
+			     half ? j->Hb : j->Wb, half ? j->n : j->m, half ? j->m : j->n, j->kt, j->split, j->tree, j->part};
 	int e;
 	nmfk_fin f = {half ? j->W : j->H, half ? j->colW : j->colH,
 			    other->path != NMFK_PATH_MFMA_BF16 ? NULL : half ? j->Wb : j->Hb, half ? j->colH : j->colW,
 			    half ? j->ncolH : j->ncolW, half ? j->denH : j->denW, j->k, clamp};
 	if (what == HALF_FINISH)
-		return nmfk_launch_finish(j->part, pl->S, g.p, j->kt, j->split, &f, st, j->stream);
+		return nmfk_launch_finish(j->part, pl->S, g.p, j->kt, j->tree, &f, st, j->stream);
 	if (what == HALF_LONE) {
-		if (!j->split && g.q <= (pl->S == 1 ? NMFK_DEN_ROWS_ONE : NMFK_DEN_ROWS))
+		if (!j->tree && g.q <= (pl->S == 1 ? NMFK_DEN_ROWS_ONE : NMFK_DEN_ROWS))
 			f.colB = NULL;
-		else if ((e = nmfk_launch_colsum_parts(g.B, g.q, j->kt, j->split, half ? j->colH : j->colW, j->stream)) != 0)
+		else if ((e = nmfk_launch_colsum_parts(g.B, g.q, j->kt, j->tree, half ? j->colH : j->colW, j->stream)) != 0)
 			return e;
 	}
 	return nmfk_launch_half(&g, pl, what != HALF_SUMS ? &f : NULL, st, j->stream);
@@ -928,7 +931,7 @@ int nmfk_job_run(nmfk_job *j, const nmfk_options *opt, nmfk_result *res)
 			e = one_pass(j, 0, 0, j->st);
 	} else {
 		if (!e)
-			e = nmfk_launch_colsum_parts(j->W, j->n, j->kt, j->split, j->colW, j->stream);
+			e = nmfk_launch_colsum_parts(j->W, j->n, j->kt, j->tree, j->colW, j->stream);
 		if (!e)
 			e = nmfk_job_shadow_for_H(j);
 	}
@@ -1202,7 +1205,7 @@ int nmfk_job_time_iterations(nmfk_job *j, uint32_t iters, nmfk_timing *t)
 {
 	if (needs_device_V(j, "nmfk_job_time_iterations"))
 		return NMFK_EINVAL;
-	int e = nmfk_launch_colsum_parts(j->W, j->n, j->kt, j->split, j->colW, j->stream);
+	int e = nmfk_launch_colsum_parts(j->W, j->n, j->kt, j->tree, j->colW, j->stream);
 	if (!e)
 		e = nmfk_job_shadow_for_H(j);
 	if (!e)

@@ -45,6 +45,7 @@ struct nmfk_job {
 	int split_mode;                /* NMFK_SPLIT_* as asked for */
 	uint32_t target_wgs;           /* workgroup target the job was replanned to (0: planned on its own) */
 	int split;                     /* FP32 matrix-core half-steps run on split products (set_split) */
+	int tree;                      /* splits, rows and column sums are added as trees (set_split) */
 	hipStream_t stream;
 	hipEvent_t ev[2];
 	hipGraphExec_t chunk_exec;

@@ -99,13 +99,15 @@ typedef struct nmfk_half {
 	const uint16_t *Bb;   /* row-major BF16 copy of B (plan path NMFK_PATH_MFMA_BF16 reads it instead of B) */
 	uint32_t p, q, kt;
 	int split;            /* products of three-part BF16 operands (FP32 accuracy; kt 32, 64 on plan path
-				 NMFK_PATH_MFMA32; splits, rows and column sums are added as trees) */
+				 NMFK_PATH_MFMA32, with tree) */
+	int tree;             /* splits, rows and column sums are added as trees (plan path NMFK_PATH_MFMA32:
+				 with split, or at kt 16) */
 	float *part;
 } nmfk_half;
 typedef struct nmfk_fin {
 	float *A, *colA;
 	uint16_t *Ab;         /* BF16 copy of the new A to keep (kt % 32 == 0), or NULL */
-	const float *colB;    /* NULL: the column sums are taken from B (q <= NMFK_DEN_ROWS, no split products) */
+	const float *colB;    /* NULL: the column sums are taken from B (q <= NMFK_DEN_ROWS, not tree) */
 	uint32_t ncolB;
 	float *den;           /* receives the column sums of B */
 	uint32_t k;
@@ -123,6 +125,8 @@ int nmfk_launch_half(const nmfk_half *g, const nmfk_hplan *pl, const nmfk_fin *f
 
 /* Whether a resident FP32 matrix-core job planned on its own runs on split products by itself. */
 int nmfk_split_rule(uint32_t n, uint32_t m, uint32_t kt, uint32_t k);
+/* Whether one on the FP32 instructions, planned on its own, adds as trees by itself. */
+int nmfk_tree_rule(uint32_t n, uint32_t m, uint32_t kt, uint32_t k);
 
 /* One pass over V per iteration (k_fused_mfma): eligible shapes and their launch plan.
  * Returns 0 and the workgroups G and waves per workgroup when the pass can run the job
@@ -137,13 +141,13 @@ int nmfk_launch_fused(const float *V, size_t ldv, float *W, const float *H, uint
 int nmfk_launch_fused_finish(const float *part, uint32_t G, const float *colW, float *H, uint32_t m, uint32_t k,
 			     uint32_t kt, const nmfk_state *st, hipStream_t stream);
 /* The finish by itself: S slices of part, with fin->den given (colB is not read). */
-int nmfk_launch_finish(const float *part, uint32_t S, uint32_t p, uint32_t kt, int split, const nmfk_fin *fin,
+int nmfk_launch_finish(const float *part, uint32_t S, uint32_t p, uint32_t kt, int tree, const nmfk_fin *fin,
 		       const nmfk_state *st, hipStream_t stream);
 /* The BF16 copy of A alone (initial factors). */
 int nmfk_launch_shadow(const float *A, uint32_t p, uint32_t kt, uint16_t *Ab, hipStream_t stream);
 /* colA[blk][c] = sum of A[a][c] over the rows of block blk (same order as the finish of a job
- * with or without split products). */
-int nmfk_launch_colsum_parts(const float *A, uint32_t p, uint32_t kt, int split, float *colA, hipStream_t stream);
+ * with or without tree sums). */
+int nmfk_launch_colsum_parts(const float *A, uint32_t p, uint32_t kt, int tree, float *colA, hipStream_t stream);
 
 /* den[c] = sum_g parts[g][c] in the fixed order a half-step uses. */
 int nmfk_launch_den(const float *parts, uint32_t nparts, uint32_t kt, float *den, hipStream_t stream);
@@ -179,7 +183,7 @@ typedef struct nmfk_bjob {
 	uint32_t ncolW, ncolH;
 	nmfk_hplan planH, planW;
 	uint32_t live;        /* 0: empty slot, every tile of it returns without reading the job */
-	uint32_t split;       /* the job runs on split products (its finishes add as trees) */
+	uint32_t tree;        /* the job's finishes add as trees */
 } nmfk_bjob;
 
 typedef struct nmfk_tile {

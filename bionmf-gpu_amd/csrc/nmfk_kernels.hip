@@ -113,17 +113,17 @@ __device__ __forceinline__ double wave_sum_d(double v)
 typedef float floatx4 __attribute__((ext_vector_type(4)));
 
 // Eight values as a tree: 3 roundings deep instead of 8.  The sums over splits, rows and
-// column-sum partials of a job on split products are formed this way, which takes their
-// rounding errors well below those of the products (a half-step at 20000 x 1000: 1.5e-7 rms
-// from 64 bits in order, 0.5e-7 without these errors).  Every other job keeps its ascending
-// order, and with it its bits.
+// column-sum partials of a job on split products, or that nmfk_tree_rule names, are formed this
+// way, which takes their rounding errors well below those of the products (a half-step at 20000 x
+// 1000: 1.5e-7 rms from 64 bits in order, 0.5e-7 without these errors).  Every other job keeps its
+// ascending order, and with it its bits.
 __device__ __forceinline__ float pair8(const float (&v)[8])
 {
 	return ((v[0] + v[1]) + (v[2] + v[3])) + ((v[4] + v[5]) + (v[6] + v[7]));
 }
 
 // den[c] = sum_g parts[g][c]: four interleaved ascending sums per column, added in a fixed order
-// at the end (PAIR, jobs on split products: 8 values at a time are added as a tree before they
+// at the end (PAIR, jobs that add as trees: 8 values at a time are added as a tree before they
 // join the running sum; see pair8).  s4 is 4 KT floats of LDS, and <room> more follow it, through
 // which all threads fetch the rows: read one by one from memory by the 4 KT threads that add
 // them, 938 rows at kt 4 (60000 rows of A) took 13 us, longer than the streaming they run beside.
@@ -1251,7 +1251,7 @@ __device__ __forceinline__ void partial_mfma_body(int bx, int by, const half_arg
 	mfma_store<KT, NA, NB>(acc, ha, by, a0, idle, smem);
 }
 
-template <int KT, int NA, int NB, int KE = KT>
+template <int KT, int NA, int NB, int KE = KT, bool PAIR = false>
 __global__ __launch_bounds__(64 * NA * NB, (KT == 32 ? 3 : 1)) void k_partial_mfma(half_args h, fin_args f,
 										       const nmfk_state *__restrict__ st)
 {
@@ -1259,11 +1259,11 @@ __global__ __launch_bounds__(64 * NA * NB, (KT == 32 ? 3 : 1)) void k_partial_mf
 	__shared__ __align__(16) float smem[LDS];
 	const uint32_t stop = read_stop(st);
 	int bx, by;
-	if (!half_tile<KT, false, LDS>(h, f, smem, stop, bx, by))
+	if (!half_tile<KT, PAIR, LDS>(h, f, smem, stop, bx, by))
 		return;
 	partial_mfma_body<KT, NA, NB, KE>(bx, by, h, smem, stop);
 	if (h.part == nullptr && !stopped(stop))
-		finish_rows<KT, false, 64 * NA * NB>(bx, 64 * NA, h, f, smem);
+		finish_rows<KT, PAIR, 64 * NA * NB>(bx, 64 * NA, h, f, smem);
 }
 
 // --------------------------------------------------------------------------------------
@@ -3016,8 +3016,11 @@ __global__ __launch_bounds__(NMFK_WG, (CLS == 0 || CLS == 2 || CLS == 4 ? 4 : CL
 		if (tl.bx == (uint32_t)h.nab) {   // the denominators
 			const fin_args f = batch_fin(J, half, 0);
 			constexpr int LDS = smem_batch_partial<CLS>();
-			if constexpr (CLS > 1)
-				den_reduce<batch_cls_kt(CLS), (CLS >= 6)>(f.colB, f.ncolB, f.den, smem, LDS - 4 * batch_cls_kt(CLS));
+			constexpr int KT = batch_cls_kt(CLS);
+			if (KT == 16 && J.tree)
+				den_reduce<16, true>(f.colB, f.ncolB, f.den, smem, LDS - 64);
+			else if constexpr (CLS > 1)
+				den_reduce<KT, (CLS >= 6)>(f.colB, f.ncolB, f.den, smem, LDS - 4 * KT);
 			else if (J.kt == 4)
 				den_reduce<4>(f.colB, f.ncolB, f.den, smem, LDS - 16);
 			else
@@ -3071,12 +3074,12 @@ __global__ __launch_bounds__(NMFK_WG) void k_batch_finish(const nmfk_bjob *__res
 			continue;
 		const fin_args f = batch_fin(J, half, clamp);
 		const int S = half == 0 ? J.planH.S : J.planW.S, p = half == 0 ? J.m : J.n, tid = threadIdx.x;
-		switch (J.kt + J.split) {
+		switch (J.kt + J.tree) {
 #define X(K, PAIR)                                                                                     \
 	case K + PAIR:                                                                                 \
 		finish_block<K, PAIR, false, false>(tl.bx, tid, J.part, S, f.A, p, f.k, f.den, f.colA, f.clamp, nullptr, smem); \
 		break;
-			X(4, false) X(8, false) X(16, false) X(32, false) X(32, true)
+			X(4, false) X(8, false) X(16, false) X(16, true) X(32, false) X(32, true)
 #undef X
 		}
 		__syncthreads();
@@ -3695,6 +3698,17 @@ extern "C" int nmfk_split_rule(uint32_t n, uint32_t m, uint32_t kt, uint32_t k)
 	return kt % 32u == 0 && k > 16u && (size_t)n * m >= (6u << 20);
 }
 
+// Jobs of the FP32 instructions, planned on their own, that add as trees as well: the longer the
+// sums, the more it gives, and it costs no time (20000 x 1000, k = 16 46.1 us per iteration, 46.2 in
+// ascending order).  The line is that of nmfk_split_rule.  Errors of W and H over 140 drawn jobs of k = 9..16, 6 to
+// 60 million values, 10-100 iterations, in multiples of those of split products with tree sums:
+// planted 0.94 and 0.92 in the mean, lognormal 1.05 and 1.02, and over 1.5 with 2 jobs, 2.07 at most;
+// in ascending order 1.13 to 1.34 and 2.34.
+extern "C" int nmfk_tree_rule(uint32_t n, uint32_t m, uint32_t kt, uint32_t k)
+{
+	return kt == 16u && k > 8u && (size_t)n * m >= (6u << 20);
+}
+
 extern "C" void nmfk_plan_half(uint32_t p, uint32_t q, uint32_t kt, nmfk_hplan *pl)
 {
 	nmfk_plan_half_path(p, q, kt, NMFK_PATH_AUTO, pl);
@@ -3727,7 +3741,7 @@ static bool kernel_args(const nmfk_half *g, const nmfk_hplan *pl, const nmfk_fin
 	if (fin)
 		*f = fin_args{fin->A, fin->colA, (__bf16 *)fin->Ab, fin->colB, fin->den, (int)fin->ncolB, (int)fin->k, fin->clamp};
 	*grid = dim3(((own ? pl->nab : pl->nab + 1) * pl->S + 7u) & ~7u);
-	if (fin && fin->colB == nullptr && (g->split || g->q > NMFK_DEN_ROWS))
+	if (fin && fin->colB == nullptr && (g->tree || g->q > NMFK_DEN_ROWS))
 		return false;
 	return g->part != nullptr && !(own && rows % NMFK_FIN_ROWS != 0 && pl->nab != 1);
 }
@@ -3798,7 +3812,16 @@ static int launch_half_mfma(const nmfk_half *g, const nmfk_hplan *pl, const nmfk
 		NMFK_MFMA_KE(2, 2, 4)
 		NMFK_MFMA_KE(2, 2, 8)
 #undef NMFK_MFMA_KE
+#define X(NA_, NB_)                                                                                    \
+	if (g->tree && na == NA_ && nb == NB_) {                                                       \
+		hipLaunchKernelGGL((k_partial_mfma<KT, NA_, NB_, KT, true>), grid, dim3(64 * NA_ * NB_), 0, stream, h, f, st); \
+		return (int)hipGetLastError();                                                         \
 	}
+		NMFK_SHAPE_LIST(X)
+#undef X
+	}
+	if (g->tree)
+		return (int)hipErrorInvalidValue;
 #define X(NA_, NB_)                                                                                    \
 	if (na == NA_ && nb == NB_) {                                                                  \
 		hipLaunchKernelGGL((k_partial_mfma<KT, NA_, NB_>), grid, dim3(64 * NA_ * NB_), 0, stream, h, f, st); \
@@ -3833,7 +3856,7 @@ static int launch_half_bf16(const nmfk_half *g, const nmfk_hplan *pl, const nmfk
 static int launch_half_sums(const nmfk_half *g, const nmfk_hplan *pl, const nmfk_fin *fin, const nmfk_state *st,
 			    hipStream_t stream)
 {
-	if (g->ldu % 4 != 0 || (g->split && pl->path != NMFK_PATH_MFMA32))
+	if (g->ldu % 4 != 0 || (g->split && !g->tree) || (g->tree && pl->path != NMFK_PATH_MFMA32))
 		return (int)hipErrorInvalidValue;
 	if (pl->path == NMFK_PATH_MFMA_BF16) {
 		switch (g->kt) {
@@ -3868,20 +3891,20 @@ static int launch_half_sums(const nmfk_half *g, const nmfk_hplan *pl, const nmfk
 	}
 }
 
-extern "C" int nmfk_launch_finish(const float *part, uint32_t S, uint32_t p, uint32_t kt, int split, const nmfk_fin *f,
+extern "C" int nmfk_launch_finish(const float *part, uint32_t S, uint32_t p, uint32_t kt, int tree, const nmfk_fin *f,
 				  const nmfk_state *st, hipStream_t stream)
 {
 	const unsigned g = (p + NMFK_FIN_ROWS - 1) / NMFK_FIN_ROWS;
 	if (f->Ab != nullptr && kt % 32 != 0)
 		return (int)hipErrorInvalidValue;
 #define X(K, PAIR)                                                                                     \
-	if (kt == K && (split != 0) == PAIR) {                                                         \
+	if (kt == K && (tree != 0) == PAIR) {                                                         \
 		hipLaunchKernelGGL((k_finish<K, PAIR>), dim3(g), dim3(NMFK_WG), 0, stream, part, (int)S, f->A, (int)p, \
 				   (int)f->k, f->den, f->colA, f->clamp, st, (__bf16 *)f->Ab);          \
 		return (int)hipGetLastError();                                                         \
 	}
 	X(4, false) X(8, false) X(16, false) X(32, false) X(64, false)
-	X(32, true) X(64, true)
+	X(16, true) X(32, true) X(64, true)
 #undef X
 	return (int)hipErrorInvalidValue;
 }
@@ -3894,7 +3917,7 @@ extern "C" int nmfk_launch_half(const nmfk_half *g, const nmfk_hplan *pl, const 
 	const int e = launch_half_sums(g, pl, fin, st, stream);
 	if (e || !fin || pl->S == 1)
 		return e;
-	return nmfk_launch_finish(g->part, pl->S, g->p, g->kt, g->split, fin, st, stream);
+	return nmfk_launch_finish(g->part, pl->S, g->p, g->kt, g->tree, fin, st, stream);
 }
 
 extern "C" int nmfk_fused_plan(uint32_t n, uint32_t m, uint32_t kt, uint32_t *G, uint32_t *nwv)
@@ -3960,16 +3983,16 @@ extern "C" int nmfk_launch_shadow(const float *A, uint32_t p, uint32_t kt, uint1
 	}
 }
 
-extern "C" int nmfk_launch_colsum_parts(const float *A, uint32_t p, uint32_t kt, int split, float *colA, hipStream_t stream)
+extern "C" int nmfk_launch_colsum_parts(const float *A, uint32_t p, uint32_t kt, int tree, float *colA, hipStream_t stream)
 {
 	const unsigned g = (p + NMFK_FIN_ROWS - 1) / NMFK_FIN_ROWS;
-	if (split) {
+	if (tree) {
 		switch (kt) {
 #define X(K)                                                                                      \
 	case K:                                                                                   \
 		hipLaunchKernelGGL((k_colsum_parts<K, true>), dim3(g), dim3(NMFK_WG), 0, stream, A, (int)p, colA); \
 		return (int)hipGetLastError();
-			X(32) X(64)
+			X(16) X(32) X(64)
 #undef X
 		default:
 			return (int)hipErrorInvalidValue;

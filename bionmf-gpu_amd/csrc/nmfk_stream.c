@@ -356,7 +356,7 @@ static int pass(nmfk_job *j, int kind, const float *Hp, int clamp, double acc[3]
 		float *Wb = j->W + (size_t)i0 * j->kt;
 		if (!e && (kind == PASS_WH || kind == PASS_W)) {
 			e = nmfk_launch_transpose(j->Vb[s], r, j->m, j->ldv, j->Vtb[s], j->ldvtb, j->stream);
-			const nmfk_half g = {j->Vtb[s], j->ldvtb, Wb, j->H, NULL, r, j->m, j->kt, 0, j->part};
+			const nmfk_half g = {j->Vtb[s], j->ldvtb, Wb, j->H, NULL, r, j->m, j->kt, 0, 0, j->part};
 			const nmfk_fin f = {Wb, j->colW + (size_t)(i0 / NMFK_FIN_ROWS) * j->kt, NULL, j->colH, j->ncolH,
 					    j->denH, j->k, clamp};
 			if (!e)
@@ -364,7 +364,7 @@ static int pass(nmfk_job *j, int kind, const float *Hp, int clamp, double acc[3]
 		}
 		if (!e && (kind == PASS_H0 || kind == PASS_WH)) {
 			/* sums only: the other blocks' and colsum(W) are complete after the pass */
-			const nmfk_half g = {j->Vb[s], j->ldv, Hp, Wb, NULL, j->m, r, j->kt, 0,
+			const nmfk_half g = {j->Vb[s], j->ldv, Hp, Wb, NULL, j->m, r, j->kt, 0, 0,
 					     j->partH + (size_t)hoff * j->m * j->kt};
 			e = nmfk_launch_half(&g, ph, NULL, st, j->stream);
 			hoff += ph->S;
@@ -399,7 +399,7 @@ int nmfk_stream_run(nmfk_job *j, const nmfk_options *opt, nmfk_result *res)
 	j->stream_bytes = 0.0;
 	int e = nmfk_launch_state_reset(j->st, opt->stop_threshold, UINT32_MAX, j->last, j->m, j->stream);
 	if (!e)
-		e = nmfk_launch_colsum_parts(j->W, j->n, j->kt, j->split, j->colW, j->stream);
+		e = nmfk_launch_colsum_parts(j->W, j->n, j->kt, j->tree, j->colW, j->stream);
 	if (!e)
 		e = nmfk_launch_den(j->colW, j->ncolW, j->kt, j->denW, j->stream);
 	if (!e)
@@ -494,7 +494,7 @@ int nmfk_stream_dot_kl(nmfk_job *j, double *dot_V, double *dot_VWH, double *kl)
  * over V adding the H partial sums, then the H finish.  Not gated by the stop state. */
 int nmfk_stream_update_H(nmfk_job *j)
 {
-	int e = nmfk_launch_colsum_parts(j->W, j->n, j->kt, j->split, j->colW, j->stream);
+	int e = nmfk_launch_colsum_parts(j->W, j->n, j->kt, j->tree, j->colW, j->stream);
 	if (!e)
 		e = nmfk_launch_den(j->colW, j->ncolW, j->kt, j->denW, j->stream);
 	if (e)
@@ -510,7 +510,7 @@ int nmfk_stream_update_H(nmfk_job *j)
  * block by block. */
 int nmfk_stream_update_W(nmfk_job *j)
 {
-	int e = nmfk_launch_colsum_parts(j->H, j->m, j->kt, j->split, j->colH, j->stream);
+	int e = nmfk_launch_colsum_parts(j->H, j->m, j->kt, j->tree, j->colH, j->stream);
 	if (e)
 		return nmfk_hip_fail(e, "update_W");
 	return pass(j, PASS_W, NULL, 0, NULL, NULL);

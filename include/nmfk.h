@@ -139,7 +139,9 @@ int nmfk_job_kernel_path(const nmfk_job *job);
  * products for k > 16 and n m >= 6 Mi (nmfk_split_rule), unless the job is replanned to a
  * workgroup target, which is meant for many jobs at once.  NMFK_SPLIT_OFF: always the FP32
  * instructions, on any path and plan.  NMFK_SPLIT_ON: split products whenever the job is on the FP32
- * matrix-core path at a padded rank of 32 or 64.  Jobs of a rank sweep and of the serving loop are set to
+ * matrix-core path at a padded rank of 32 or 64.  Such jobs add row splits and column sums as trees,
+ * nearer to 64 bits than the ascending order of all others; without NMFK_SPLIT_OFF and a workgroup
+ * target so do those of 8 < k <= 16 and n m >= 6 Mi on the FP32 instructions.  Jobs of a rank sweep and of the serving loop are set to
  * NMFK_SPLIT_OFF.  Streamed jobs always run the FP32 instructions, and refuse the call. */
 #define NMFK_SPLIT_AUTO 0
 #define NMFK_SPLIT_OFF 1
@@ -211,7 +213,7 @@ void nmfk_host_free(void *p);
 /* Re-plans both half-steps aiming for <target_wgs> partial-kernel workgroups (0 = the
  * process tunables); the number of splits of the contraction range, and with it the
  * summation order, follows the plan, so jobs compared bit for bit must share plans.  With a
- * target, a job left at NMFK_SPLIT_AUTO runs the FP32 instructions. */
+ * target, a job left at NMFK_SPLIT_AUTO runs the FP32 instructions and adds in ascending order. */
 int nmfk_job_replan(nmfk_job *job, uint32_t target_wgs);
 /* {nab, S, bchunk, path} of the H half, then of the W half. */
 int nmfk_job_plan_get(const nmfk_job *job, uint32_t out[8]);

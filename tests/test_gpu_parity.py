@@ -421,6 +421,59 @@ def test_split_products_same_bits_in_every_batch_class(nmfk, orc, n, m, k, wide)
             j.close()
 
 
+@pytest.mark.parametrize("n,m,k", [(6401, 1087, 13), (98400, 65, 9), (25601, 257, 16), (12000, 1100, 12)])
+def test_tree_sums_at_padded_rank_16_give_the_same_bits(nmfk, n, m, k):
+    # Alone, by half-steps and in a batch, beside a job that adds in ascending order.
+    jobs = [nmfk.Job(n, m, k) for _ in range(5)]
+    try:
+        for i, j in enumerate(jobs):
+            j.gen_V_lognormal(n, 0.0, 1.0)
+            j.init_random(m)
+            j.set_split(j.SPLIT_OFF if i >= 3 else j.SPLIT_AUTO)
+            assert not j.split()
+        a, b, c, d, e = jobs
+        batch = nmfk.Batch(5, 4)
+        batch.add(b, 10, 1000)
+        batch.add(e, 10, 1000)
+        batch.run()
+        batch.close()
+        for x, y in ((a, b), (d, e)):
+            x.run(10, 5, 1000)
+            assert np.array_equal(x.get_W(), y.get_W()) and np.array_equal(x.get_H(), y.get_H())
+        assert not np.array_equal(a.get_W(), d.get_W())
+        a.init_random(m)
+        a.run(2, 1000, 1000)
+        for _ in range(2):
+            c.update_H()
+            c.update_W()
+        assert np.array_equal(a.get_W(), c.get_W()) and np.array_equal(a.get_H(), c.get_H())
+        a.set_split(a.SPLIT_OFF)   # the captured interval of the trees is not run again
+        for j in (a, d):
+            j.init_random(m)
+            j.run(10, 5, 1000)
+        assert np.array_equal(a.get_W(), d.get_W()) and np.array_equal(a.get_H(), d.get_H())
+    finally:
+        for j in jobs:
+            j.close()
+
+
+@pytest.mark.parametrize("n,m,k", [(98400, 65, 9), (200000, 40, 14)])
+def test_tree_sums_at_padded_rank_16_are_nearer_to_64_bits(nmfk, n, m, k):
+    # Four ascending chains of n / 256 column-sum partials each err by about sqrt(n / 768) / 2
+    # roundings, trees of 8 by a third of that.
+    errs = []
+    for mode in (0, 1):
+        with nmfk.Job(n, m, k) as job:
+            job.set_split(mode)
+            job.gen_V_planted(3, 6, 0.3)
+            job.init_random(4)
+            V, W, H = (x.astype(np.float64) for x in (job.get_V(), job.get_W(), job.get_H()))
+            job.update_H()
+            want = H * ((V / (W @ H.T)).T @ W) / W.sum(axis=0)
+            errs.append(np.sqrt(np.mean((job.get_H() / want - 1.0) ** 2)))
+    assert errs[0] < errs[1], errs
+
+
 def test_golden_tiny_runs(nmfk, orc):
     g = np.load(GOLDEN / "tiny.npz")
     for ci in range(int(g["ncases"])):

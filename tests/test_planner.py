@@ -252,6 +252,15 @@ def test_split_rule(lib):
     assert lib.nmfk_split_rule(70000, 70000, 64, 64) == 1   # n m past 32 bits
 
 
+def test_tree_rule(lib):
+    # Sums as trees without split products: padded rank 16 from the same size on.
+    for n, m, k, tree in [(6144, 1024, 9, 1), (6143, 1024, 9, 0), (98400, 65, 16, 1), (70000, 70000, 12, 1),
+                          (600000, 20, 8, 0), (600000, 20, 4, 0), (6401, 1087, 17, 0), (6401, 1087, 48, 0)]:
+        kt = lib.nmfk_job_kt(n, m, k)
+        assert lib.nmfk_tree_rule(n, m, kt, k) == tree, (n, m, k)
+        assert not (tree and lib.nmfk_split_rule(n, m, kt, k))
+
+
 def test_rows_of_one_descriptor(lib):
     # 16 rows of <ldu> floats within 2 GiB: the last byte offset the 16-row kernels form stays below
     # 2^31; longer rows are refused, or read through 64-bit addresses.
